@@ -169,81 +169,148 @@ __global__ void __launch_bounds__(256) append_kernel(AppendArgs a) {
     }
 }
 
-/* The training-form prologue (reference model/kernels/qk_prologue.cu:8-32): token p = blockIdx.x of rows/H,
- * rows [0, H) q heads, [H, 2H) k heads; input token stride 3 H 128, output contiguous, position p % T. */
-__global__ void __launch_bounds__(256) qkp_forward_kernel(const uint16_t *q, const uint16_t *k, const float *gq,
-                                                          const float *gk, uint16_t *qo, uint16_t *ko,
-                                                          const float *cos, const float *sin, int H, int T) {
-    const int lane = threadIdx.x & (WAVE - 1);
-    const int row = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (row >= 2 * H) return;
-    const long long p = blockIdx.x;
-    const bool isq = row < H;
-    const int h = isq ? row : row - H;
-    const uint16_t *x = (isq ? q : k) + p * 3 * H * HEAD_DIM + h * HEAD_DIM;
-    const float *g = isq ? gq : gk;
-    const long long tab = (p % T) * HALF + lane;
-    float y1, y2;
-    norm_rope_pair(bf16_to_f32(x[lane]), bf16_to_f32(x[lane + HALF]), g[lane], g[lane + HALF], cos[tab], sin[tab], y1,
-                   y2);
-    uint16_t *y = (isq ? qo : ko) + (p * H + h) * HEAD_DIM;
-    y[lane] = f32_to_bf16(y1);
-    y[lane + HALF] = f32_to_bf16(y2);
+/* The training-form prologue (reference model/kernels/qk_prologue.cu:8-32) of q's and k's [tokens][H] rows: input
+ * token stride 3 H 128, output contiguous, position p % T for token p.
+ *
+ * Both directions are bound by HBM (forward: 2 x 256 bytes a row; backward: 3 x 256). 16 lanes take a row (nc_row.h's
+ * form of eight consecutive dims a lane), a 16-lane group QK_HEADS heads of one token, so every access is 16 bytes a
+ * lane, the rotation is read once for QK_HEADS rows and all of a group's rows are in flight together. Against one row a
+ * wave with 2-byte accesses, 65,536 tokens of 6 heads: forward 179 -> 90 us, backward 242 -> 133 us (4.5 TB/s each; a
+ * large copy reaches 4.8). */
+constexpr int QK_HEADS = 3;
+static int qk_head_chunks(int H) { return (H + QK_HEADS - 1) / QK_HEADS; }
+
+/* The rotation of token p's pairs in lane i (see norm_rope_oct): sin is negated in the lanes of the half that `neg`
+ * names. */
+__device__ __forceinline__ void load_rotation(const float *cos, const float *sin, long long pos, int i, bool neg,
+                                              float (&c)[8], float (&s)[8]) {
+    load8_f32(cos + pos * HALF + 8 * (i & 7), c);
+    load8_f32(sin + pos * HALF + 8 * (i & 7), s);
+#pragma unroll
+    for (int e = 0; e < 8; e++) s[e] = neg ? -s[e] : s[e];
 }
 
-/* The training-form prologue's backward (reference model/kernels/qk_prologue.cu:36-90): per (token, head) row, a
- * wave with lane l on dims l and l + 64, recomputing n = x r; the rotation's transpose gives dm (dm1 = dy1 c - dy2 s,
- * dm2 = dy1 s + dy2 c); dn = dm g; dx = r (dn - n b), b = sum(dn n) / 128 (the butterfly); the gain gradient
- * sum_rows dm n accumulates per lane in row order. Grid: QKB_BLOCKS blocks per tensor (q's, then k's), wave w of
- * block j taking rows j 4 + w, + QKB_BLOCKS 4, ...; each block writes its partial [128] (waves added in order). */
+/* Grid x = 16-token blocks times the head chunks of q then of k (chunk fastest), 256 threads. Indexes fit 32 bits: a row
+ * takes 768 bytes of memory or more. */
+__global__ void __launch_bounds__(256) qkp_forward_kernel(const uint16_t *q, const uint16_t *k, const float *gq,
+                                                          const float *gk, uint16_t *qo, uint16_t *ko,
+                                                          const float *cos, const float *sin, long long tokens, int H,
+                                                          int T) {
+    const int i = threadIdx.x & 15, chunks = (H + QK_HEADS - 1) / QK_HEADS;
+    const int block = blockIdx.x / (2 * chunks), chunk = blockIdx.x - block * 2 * chunks;
+    const long long p = (long long)block * 16 + (threadIdx.x >> 4);
+    if (p >= tokens) return;   /* whole 16-lane groups */
+    const bool isq = chunk < chunks;
+    const int h0 = (chunk - (isq ? 0 : chunks)) * QK_HEADS;
+    const uint16_t *x = (isq ? q : k) + (p * 3 * H + h0) * HEAD_DIM + 8 * i;
+    uint16_t *y = (isq ? qo : ko) + (p * H + h0) * HEAD_DIM + 8 * i;
+    uint4 raw[QK_HEADS];
+    float g[8], c[8], s[8];
+#pragma unroll
+    for (int j = 0; j < QK_HEADS; j++)
+        if (h0 + j < H) raw[j] = load8_raw(x + j * HEAD_DIM);
+    load_rotation(cos, sin, (unsigned)p % (unsigned)T, i, i >= 8, c, s);
+    load8_f32((isq ? gq : gk) + 8 * i, g);
+#pragma unroll
+    for (int j = 0; j < QK_HEADS; j++) {
+        if (h0 + j >= H) break;
+        float xr[8], yr[8];
+        unpack8(raw[j], xr);
+        norm_rope_oct(xr, g, c, s, yr);
+        store8_bf16(y + j * HEAD_DIM, yr);
+    }
+}
+
+/* The prologue's backward (reference model/kernels/qk_prologue.cu:36-90): per (token, head) row, recomputing n = x r;
+ * the rotation's transpose gives dm (dm1 = dy1 c - dy2 s, dm2 = dy1 s + dy2 c); dn = dm g; dx = r (dn - n b),
+ * b = sum(dn n) / 128 (the butterfly); the gain gradient sum_rows dm n accumulates per lane in row order. Grid:
+ * QKB_BLOCKS blocks per tensor (q's, then k's); 16-lane group w of a tensor's QKB_GROUPS takes the (token, head chunk)
+ * units w, w + QKB_GROUPS, ...; each block writes its partial [128] (its groups added in order). */
 constexpr int QKB_BLOCKS = 512;   /* fixed, so the gain gradient's summation order is fixed */
+constexpr int QKB_GROUPS = QKB_BLOCKS * 16;
 
 __global__ void __launch_bounds__(256) qkp_backward_kernel(const uint16_t *q, const uint16_t *k, const float *gq,
                                                            const float *gk, const uint16_t *dqo, const uint16_t *dko,
                                                            uint16_t *dq, uint16_t *dk, const float *cos,
-                                                           const float *sin, float *part, long long rows, int H,
+                                                           const float *sin, float *part, long long tokens, int H,
                                                            int T) {
-    __shared__ float wpart[4][HEAD_DIM];
-    const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x >> 6;
+    __shared__ float gpart[16][HEAD_DIM];
+    const int i = threadIdx.x & 15, grp = threadIdx.x >> 4;
     const bool isq = blockIdx.x < QKB_BLOCKS;
-    const long long first = (isq ? blockIdx.x : blockIdx.x - QKB_BLOCKS) * 4 + wave;
     const uint16_t *xin = isq ? q : k, *dyin = isq ? dqo : dko;
     uint16_t *dxout = isq ? dq : dk;
-    const float *g = isq ? gq : gk;
-    const float g1 = g[lane], g2 = g[lane + HALF];
-    float a1 = 0.0f, a2 = 0.0f;
-    for (long long i = first; i < rows; i += (long long)QKB_BLOCKS * 4) {
-        const long long t = i / H, at = t * 3 * H * HEAD_DIM + (i % H) * HEAD_DIM;
-        const long long tab = (t % T) * HALF + lane;
-        const float x1 = bf16_to_f32(xin[at + lane]), x2 = bf16_to_f32(xin[at + lane + HALF]);
-        const float d1 = bf16_to_f32(dyin[i * HEAD_DIM + lane]), d2 = bf16_to_f32(dyin[i * HEAD_DIM + lane + HALF]);
-        const float c = cos[tab], s = sin[tab];
-        const float ss = wave_sum_butterfly(x1 * x1 + x2 * x2);
-        const float r = 1.0f / __builtin_sqrtf(ss / 128.0f + FLT_EPS);
-        const float n1 = x1 * r, n2 = x2 * r;
-        const float dm1 = d1 * c - d2 * s, dm2 = d1 * s + d2 * c;
-        a1 = a1 + dm1 * n1;
-        a2 = a2 + dm2 * n2;
-        const float dn1 = dm1 * g1, dn2 = dm2 * g2;
-        const float b = wave_sum_butterfly(dn1 * n1 + dn2 * n2) / 128.0f;
-        dxout[at + lane] = f32_to_bf16(r * (dn1 - n1 * b));
-        dxout[at + lane + HALF] = f32_to_bf16(r * (dn2 - n2 * b));
+    const unsigned chunks = (H + QK_HEADS - 1) / QK_HEADS;
+    float g[8], acc[8];
+    load8_f32((isq ? gq : gk) + 8 * i, g);
+#pragma unroll
+    for (int e = 0; e < 8; e++) acc[e] = 0.0f;
+    const unsigned units = (unsigned)(tokens * chunks);
+    for (unsigned u = (isq ? blockIdx.x : blockIdx.x - QKB_BLOCKS) * 16 + grp; u < units; u += QKB_GROUPS) {
+        const unsigned t = u / chunks;
+        const int h0 = (int)(u - t * chunks) * QK_HEADS;
+        const long long at = ((long long)t * 3 * H + h0) * HEAD_DIM + 8 * i, row = ((long long)t * H + h0) * HEAD_DIM + 8 * i;
+        uint4 xraw[QK_HEADS], draw[QK_HEADS];
+        float c[8], s[8];
+#pragma unroll
+        for (int j = 0; j < QK_HEADS; j++)
+            if (h0 + j < H) {
+                xraw[j] = load8_raw(xin + at + j * HEAD_DIM);
+                draw[j] = load8_raw(dyin + row + j * HEAD_DIM);
+            }
+        load_rotation(cos, sin, t % (unsigned)T, i, i < 8, c, s);
+#pragma unroll
+        for (int j = 0; j < QK_HEADS; j++) {
+            if (h0 + j >= H) break;
+            float xr[8], d[8], n[8], dn[8], part8[8];
+            unpack8(xraw[j], xr);
+            unpack8(draw[j], d);
+            const float r = rstd_oct(xr);
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                n[e] = xr[e] * r;
+                const float dm = d[e] * c[e] + lane_xor_dpp<8>(d[e]) * s[e];
+                acc[e] = acc[e] + dm * n[e];
+                dn[e] = dm * g[e];
+                const float w = dn[e] * n[e];
+                part8[e] = w + lane_xor_dpp<8>(w);
+            }
+            const float b = oct_row_sum(part8) / 128.0f;
+            float dx[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) dx[e] = r * (dn[e] - n[e] * b);
+            store8_bf16(dxout + at + j * HEAD_DIM, dx);
+        }
     }
-    wpart[wave][lane] = a1;
-    wpart[wave][lane + HALF] = a2;
+#pragma unroll
+    for (int e = 0; e < 8; e++) gpart[grp][8 * i + e] = acc[e];
     __syncthreads();
-    if (threadIdx.x < HEAD_DIM)
-        part[(long long)blockIdx.x * HEAD_DIM + threadIdx.x] =
-            ((wpart[0][threadIdx.x] + wpart[1][threadIdx.x]) + wpart[2][threadIdx.x]) + wpart[3][threadIdx.x];
+    if (threadIdx.x < HEAD_DIM) {
+        float sum = gpart[0][threadIdx.x];
+#pragma unroll
+        for (int w = 1; w < 16; w++) sum = sum + gpart[w][threadIdx.x];
+        part[(long long)blockIdx.x * HEAD_DIM + threadIdx.x] = sum;
+    }
 }
 
-/* Block 0: q's gain gradient, block 1: k's; thread d adds dim d of the QKB_BLOCKS partials in block order
- * (reference qk_prologue.cu:92-97). */
-__global__ void __launch_bounds__(HEAD_DIM) qkp_gain_sum_kernel(const float *part, float *dgq, float *dgk) {
-    const float *p = part + (long long)blockIdx.x * QKB_BLOCKS * HEAD_DIM + threadIdx.x;
-    float sum = 0.0f;
-    for (int j = 0; j < QKB_BLOCKS; j++) sum = sum + p[(long long)j * HEAD_DIM];
-    (blockIdx.x ? dgk : dgq)[threadIdx.x] = sum;
+/* Grid (2 tensors, HEAD_DIM / 16): the gain gradients of 16 dims from the QKB_BLOCKS partials (reference
+ * qk_prologue.cu:92-97). A serial sum of 512 partials is a chain of loads (11 us); here thread (w, d) adds partials
+ * 32 w .. 32 w + 31 of dim d, all loads issued together, and the 16 sums are added in order (4 us). */
+__global__ void __launch_bounds__(256) qkp_gain_sum_kernel(const float *part, float *dgq, float *dgk) {
+    constexpr int PER = QKB_BLOCKS / 16;
+    __shared__ float sums[16][16];
+    const int d = threadIdx.x & 15, w = threadIdx.x >> 4, dim = blockIdx.y * 16 + d;
+    const float *p = part + ((long long)blockIdx.x * QKB_BLOCKS + w * PER) * HEAD_DIM + dim;
+    float v[PER], sum = 0.0f;
+#pragma unroll
+    for (int j = 0; j < PER; j++) v[j] = p[j * HEAD_DIM];
+#pragma unroll
+    for (int j = 0; j < PER; j++) sum = sum + v[j];
+    sums[w][d] = sum;
+    __syncthreads();
+    if (w) return;
+#pragma unroll
+    for (int j = 1; j < 16; j++) sum = sum + sums[j][d];
+    (blockIdx.x ? dgk : dgq)[dim] = sum;
 }
 
 static thread_local int last_error = NC_OK;
@@ -348,8 +415,8 @@ extern "C" void qkp_backward(const void *q, const void *k, const void *gq, const
     hipLaunchKernelGGL(qkp_backward_kernel, dim3(2 * QKB_BLOCKS), dim3(256), 0, (hipStream_t)stream,
                        (const uint16_t *)q, (const uint16_t *)k, (const float *)gq, (const float *)gk,
                        (const uint16_t *)dqo, (const uint16_t *)dko, (uint16_t *)dq, (uint16_t *)dk,
-                       (const float *)cos, (const float *)sin, (float *)part, rows, H, T);
-    hipLaunchKernelGGL(qkp_gain_sum_kernel, dim3(2), dim3(HEAD_DIM), 0, (hipStream_t)stream, (const float *)part,
+                       (const float *)cos, (const float *)sin, (float *)part, rows / H, H, T);
+    hipLaunchKernelGGL(qkp_gain_sum_kernel, dim3(2, HEAD_DIM / 16), dim3(256), 0, (hipStream_t)stream, (const float *)part,
                        (float *)dgq, (float *)dgk);
     last_error = (int)hipGetLastError();
 }
@@ -364,10 +431,10 @@ extern "C" void qkp_forward(const void *q, const void *k, const void *gq, const 
         last_error = NC_ERR_SHAPE;
         return;
     }
-    const dim3 grid((unsigned)(rows / H), (unsigned)((2 * H + 3) / 4));
+    const dim3 grid((unsigned)((rows / H + 15) / 16 * 2 * qk_head_chunks(H)));
     hipLaunchKernelGGL(qkp_forward_kernel, grid, dim3(256), 0, (hipStream_t)stream, (const uint16_t *)q,
                        (const uint16_t *)k, (const float *)gq, (const float *)gk, (uint16_t *)qo, (uint16_t *)ko,
-                       (const float *)cos, (const float *)sin, H, T);
+                       (const float *)cos, (const float *)sin, rows / H, H, T);
     last_error = (int)hipGetLastError();
 }
 

@@ -142,4 +142,79 @@ __device__ __forceinline__ void ve_mix_quad(const uint16_t *h, const float *w, i
     for (int j = 0; j < 8; j++) v[j] = bf16_to_f32(f32_to_bf16(v[j] + g * bf16_to_f32(e[i + 16 * j])));
 }
 
+/* The row math a third way: 16 lanes a row, lane i of a 16-lane group holding the eight consecutive dims 8 i .. 8 i + 7,
+ * so a row moves by one 16-byte access a lane. Lane i's rotation partners (dim +- 64) are lane i ^ 8's elements of the
+ * same index. The element e of lanes i and i ^ 8 stands for lane l = 8 (i % 8) + e of the one-row-a-wave form: its
+ * butterfly steps 32, 16 and 8 pair lanes i with i ^ 4, i ^ 2 and i ^ 1, and steps 4, 2 and 1 pair elements, so every
+ * sum is formed in the same order and has the same bits. All 16 lanes of a group must call these together. */
+__device__ __forceinline__ float oct_row_sum(float (&p)[8]) {
+#pragma unroll
+    for (int e = 0; e < 8; e++) p[e] = p[e] + lane_xor_dpp<4>(p[e]);
+#pragma unroll
+    for (int e = 0; e < 8; e++) p[e] = p[e] + lane_xor_dpp<2>(p[e]);
+#pragma unroll
+    for (int e = 0; e < 8; e++) p[e] = p[e] + lane_xor_dpp<1>(p[e]);
+    return ((p[0] + p[4]) + (p[2] + p[6])) + ((p[1] + p[5]) + (p[3] + p[7]));
+}
+
+/* 1 / sqrt(mean x^2 + FLT_EPSILON) of the row, as norm_rope_pair's r. */
+__device__ __forceinline__ float rstd_oct(const float (&x)[8]) {
+    float part[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const float sq = x[e] * x[e];
+        part[e] = sq + lane_xor_dpp<8>(sq);
+    }
+    const float v = oct_row_sum(part) / 128.0f + FLT_EPS;
+    return 1.0f / __builtin_sqrtf(v);
+}
+
+/* norm_rope_pair in this form. g: the lane's gains; c, s: cos and sin of the lane's pairs, s negated in the upper half's
+ * lanes (i >= 8: y = n2 c - n1 s). */
+__device__ __forceinline__ void norm_rope_oct(const float (&x)[8], const float (&g)[8], const float (&c)[8],
+                                              const float (&s)[8], float (&y)[8]) {
+    const float r = rstd_oct(x);
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const float n = (x[e] * r) * g[e];
+        y[e] = n * c[e] + lane_xor_dpp<8>(n) * s[e];
+    }
+}
+
+/* Eight consecutive elements by 16-byte accesses at any element alignment (the declared alignment is the element's). */
+typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ uint4 load8_raw(const uint16_t *p) {
+    const u32x4_a2 u = *reinterpret_cast<const u32x4_a2 *>(p);
+    return uint4{u[0], u[1], u[2], u[3]};
+}
+
+__device__ __forceinline__ void unpack8(const uint4 &r, float (&x)[8]) {
+    const uint32_t u[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        x[2 * k] = __uint_as_float(u[k] << 16);
+        x[2 * k + 1] = __uint_as_float(u[k] & 0xFFFF0000u);
+    }
+}
+
+__device__ __forceinline__ void load8_f32(const float *p, float (&x)[8]) {
+    const u32x4_a4 a = reinterpret_cast<const u32x4_a4 *>(p)[0], b = reinterpret_cast<const u32x4_a4 *>(p)[1];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        x[k] = __uint_as_float(a[k]);
+        x[4 + k] = __uint_as_float(b[k]);
+    }
+}
+
+/* Rounded to bf16 (nearest even, v_cvt_pk_bf16_f32) and stored. */
+__device__ __forceinline__ void store8_bf16(uint16_t *p, const float (&x)[8]) {
+    bf16x8 v;
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[e] = (__bf16)x[e];
+    const uint4 u = __builtin_bit_cast(uint4, v);
+    *reinterpret_cast<u32x4_a2 *>(p) = u32x4_a2{u.x, u.y, u.z, u.w};
+}
+
 }  // namespace nc

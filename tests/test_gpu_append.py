@@ -206,6 +206,43 @@ def test_qk_backward_matches_oracle(device, B, T, H):
         assert np.all(np.abs(dg.double().numpy() - want_dg) <= depth * 2.0 ** -24 * mag + 1e-30)
 
 
+@pytest.mark.parametrize("B,T,H,offset", [(1, 1, 1, 0), (3, 17, 2, 1), (1, 40, 4, 3), (2, 35, 7, 5), (1, 16, 13, 8)])
+def test_qk_prologue_head_chunks_and_alignment(device, B, T, H, offset):
+    """Head counts around the kernels' three-head chunks, token counts off the 16-token blocks, and a projection that
+    starts `offset` elements into its storage (rows at any 2-byte alignment): the forward's bits equal the oracle's, and
+    the backward's input gradients are within a bf16 rounding of the float64 backward."""
+    from nanochat_amd.qk_prologue import qk_backward
+    from oracle.rope import qk_norm_rope_backward
+
+    gen = torch.Generator().manual_seed(40 + H)
+    n = B * T * 3 * H * 128
+
+    def placed(x):   # x at `offset` elements into a larger buffer
+        buf = torch.zeros(x.numel() + offset, dtype=x.dtype, device=device)
+        buf[offset:] = x.flatten().to(device)
+        return buf[offset:].view(x.shape)
+
+    qkv = torch.randn(n, generator=gen).to(torch.bfloat16).view(B, T, 3, H, 128)
+    dout = torch.randn(2, B, T, H, 128, generator=gen).to(torch.bfloat16)
+    gains = 1 + 0.1 * torch.randn(2, 128, generator=gen)
+    cos, sin = rotary_tables(T, 1e4, device)
+    qkv_d, dout_d, g_d = placed(qkv), [placed(x) for x in dout], [placed(x) for x in gains]
+    outs = qk_forward(qkv_d[:, :, 0], qkv_d[:, :, 1], g_d[0], g_d[1], cos, sin)
+    dqkv = placed(torch.full_like(qkv, 7.0))
+    qk_backward(qkv_d[:, :, 0], qkv_d[:, :, 1], g_d[0], g_d[1], dout_d[0], dout_d[1], cos, sin, dqkv[:, :, 0],
+                dqkv[:, :, 1])
+    torch.cuda.synchronize()
+    c, s = cos.cpu().numpy()[None, :, None], sin.cpu().numpy()[None, :, None]
+    for j in (0, 1):
+        want = qk_norm_rope(f32(qkv[:, :, j]), gains[j].numpy(), c, s)
+        assert np.array_equal(bf16_bits(want), outs[j].view(torch.int16).cpu().numpy().view(np.uint16))
+        dx, _ = qk_norm_rope_backward(f32(qkv[:, :, j]), gains[j].numpy(), c, s, f32(dout[j]))
+        got = dqkv[:, :, j].double().cpu().numpy()
+        ulp = 2.0 ** (np.floor(np.log2(np.maximum(np.abs(dx), 2.0 ** -126))) - 7)
+        assert np.all(np.abs(got - dx) <= ulp + 1e-5 * np.abs(dx).max(axis=-1, keepdims=True))
+    assert bool((dqkv[:, :, 2] == 7.0).all())
+
+
 def test_partial_pages_keep_the_other_slots(device):
     """Appends that start and end inside pages (misaligned starts, num_new shorter than T, new positions filling part
     of one page, a V block's four slots split between old and new) change exactly the new positions' codes and

@@ -117,6 +117,22 @@ int nc_flash_attn_bwd(const void *q, const void *k, const void *v, const void *d
 int nc_flash_attn_bwd_rows(const void *out, long long o_stride, const void *dout, long long do_stride,
                            long long total, int heads, float *dpsum, void *stream);
 
+/*
+ * The training block's output projection with its residual and row statistic (the reference's residual_rms,
+ * model/ops/linear.py:93-100): s = x w^T + res in fp32, out = bf16(s), rstd = 1 / sqrt(mean(s^2) + FLT_EPSILON). x bf16
+ * [rows][k], w bf16 [n][k], res and out bf16 [rows][n], rstd fp32 [rows]; k a multiple of 128, n of 4; x and w 16-byte,
+ * res and out 8-byte aligned. workspace: fp32 [rows][ceil(n / 32)].
+ */
+int nc_linear_residual_rms(const void *x, const void *w, const void *res, long long rows, int n, int k, void *out,
+                           float *rstd, void *workspace, long long workspace_bytes, void *stream);
+
+/* out[i][j] += sum over rows of a[row][i] b[row][j]: a bf16 [rows][n1], b bf16 [rows][n2], out fp32 [n1][n2] (n1, n2
+ * multiples of 8; everything 16-byte aligned), summed in a fixed order. workspace: nc_weight_grad_workspace_bytes (-1
+ * for sizes it does not take), 16-byte aligned. */
+long long nc_weight_grad_workspace_bytes(long long rows, int n1, int n2);
+int nc_weight_grad(const void *a, const void *b, long long rows, int n1, int n2, float *out, void *workspace,
+                   long long workspace_bytes, void *stream);
+
 /* Status of the last void entry point's launch on this host thread (NC_OK or a hipError_t). */
 int nc_last_error(void);
 

@@ -14,8 +14,10 @@ What one call computes, on the fused (B, T, 3C) projection split into q, k and v
 4. the output projection added to the residual in fp32 and rounded once, h = bf16(residual + out W^T), with
    rstd = 1 / sqrt(mean(h^2) + FLT_EPSILON) of the fp32 sum (the reference's residual_rms, model/ops/linear.py:93-100).
 
-The projection's three products are library GEMMs (bf16 operands, fp32 sums). The attention backward's per-(token,
-head) statistic dout . out comes from the HIP kernel `nc_flash_attn_bwd_rows`.
+The forward's projection with its residual and rstd is one HIP GEMM (`nc_linear_residual_rms`) and the weight's gradient
+another (`nc_weight_grad`, fp32 sums added into o_grad); operands those do not take (strided, of another type, misaligned)
+go through library GEMMs, as the gradient of the projection's input does. The attention backward's per-(token, head)
+statistic dout . out comes from the HIP kernel `nc_flash_attn_bwd_rows`.
 
 Layout of this module: every tensor the ops return is described once by a spec (shape and dtype as functions of the
 inputs); the eager ops allocate their placeholders from it and the fake (meta) implementations return it whole. The
@@ -30,6 +32,7 @@ from torch.autograd.function import FunctionCtx
 
 from .config import HEAD_DIM
 from .flash_attn import fa4_window_left, flash_attn_bwd, flash_attn_bwd_rows, flash_attn_fwd
+from .native import check, hip_library, pointer, stream
 from .qk_prologue import qk_backward, qk_forward
 from .ve_gate import ve_backward, ve_forward
 
@@ -99,6 +102,47 @@ def real_segments(cu_seqlens: Tensor, segments: Tensor) -> Tensor:
     return cu_seqlens.narrow(0, 0, int(segments) + 1)
 
 
+def _plain(t: Tensor, dtype: torch.dtype, alignment: int) -> bool:
+    """Whether a kernel may address t as one dense array of dtype at this alignment."""
+    return t.dtype == dtype and t.is_cuda and t.is_contiguous() and t.data_ptr() % alignment == 0
+
+
+SSQ_COLS = 32   # columns of one of nc_linear_residual_rms's sums of squares
+
+
+def project(x: Tensor, o_weight: Tensor, residual: Tensor) -> tuple[Tensor, Tensor]:
+    """x [tokens, K] bf16 (dense), residual [tokens, C] -> (bf16(x o_weight^T + residual), the fp32 sum's rstd
+    [tokens]). Dense bf16 operands of the kernel's sizes (K of 128, C of 4) take one GEMM whose epilogue does all of it
+    (65,536 tokens, C = 768: 350 -> 146 us); anything else a library GEMM and elementwise passes."""
+    tokens, (C, K) = x.size(0), o_weight.shape
+    if (_plain(x, BF16, 16) and _plain(o_weight, BF16, 16) and _plain(residual, BF16, 8) and K % 128 == 0 and C % 4 == 0
+            and residual.shape == (tokens, C) and max(C, K) <= 32768):
+        h, rstd = torch.empty_like(residual), x.new_empty(tokens, dtype=F32)
+        ssq = x.new_empty(tokens * (-(-C // SSQ_COLS)), dtype=F32)
+        check(hip_library().nc_linear_residual_rms(pointer(x), pointer(o_weight), pointer(residual), tokens, C, K,
+                                                   pointer(h), pointer(rstd), pointer(ssq), ssq.numel() * 4, stream()))
+        return h, rstd
+    total = torch.mm(x, o_weight.t(), out_dtype=F32)
+    total += residual
+    rstd = (total.square().mean(-1) + EPS).sqrt().reciprocal()    # correctly rounded sqrt, then 1/x
+    return total.to(BF16), rstd
+
+
+def add_weight_grad(o_grad: Tensor, dh: Tensor, x: Tensor) -> None:
+    """o_grad += dh^T x over the tokens, fp32 sums: dh [tokens, C], x [tokens, K] bf16. Dense 16-byte aligned operands
+    take the HIP kernel, which cuts the long sum over the tokens across the chip (65,536 tokens, 768 x 768: 302 -> 111 us);
+    others a library GEMM."""
+    tokens, C, K = dh.size(0), dh.size(1), x.size(1)
+    if _plain(dh, BF16, 16) and _plain(x, BF16, 16) and _plain(o_grad, F32, 16) and o_grad.shape == (C, K):
+        need = hip_library().nc_weight_grad_workspace_bytes(tokens, C, K)
+        if need >= 0:
+            ws = x.new_empty(need, dtype=torch.uint8)
+            check(hip_library().nc_weight_grad(pointer(dh), pointer(x), tokens, C, K, pointer(o_grad), pointer(ws), need,
+                                               stream()))
+            return
+    o_grad += torch.mm(dh.t(), x, out_dtype=F32)
+
+
 @torch.library.custom_op("nanochat_amd::attention", mutates_args=(), device_types="cuda")
 def attention(qkv: Tensor, q_norm_weight: Tensor, k_norm_weight: Tensor, cos: Tensor, sin: Tensor, window_left: int,
               cu_seqlens: Tensor, segments: Tensor, o_weight: Tensor, o_grad: Tensor | None, residual: Tensor,
@@ -120,10 +164,8 @@ def attention(qkv: Tensor, q_norm_weight: Tensor, k_norm_weight: Tensor, cos: Te
                                      real_segments(cu_seqlens, segments), s.T,
                                      window_left=fa4_window_left(window_left, s.T))
     res["out"] = out.view(s.B, s.T, s.H, HEAD_DIM)
-    total = torch.mm(out.flatten(1), o_weight.t(), out_dtype=F32)
-    total += residual.flatten(0, 1)
-    res["rstd"] = (total.square().mean(-1) + EPS).sqrt().reciprocal()    # correctly rounded sqrt, then 1/x
-    res["h"] = total.to(BF16).view(residual.shape)
+    h, res["rstd"] = project(out.flatten(1), o_weight, residual.flatten(0, 1))
+    res["h"] = h.view(residual.shape)
     return tuple(res[name] for name in FORWARD_OUTPUTS)
 
 
@@ -150,7 +192,7 @@ def attention_bwd(dh: Tensor, qkv: Tensor, q_norm_weight: Tensor, k_norm_weight:
     # o_proj: out's gradient, and the weight's, from the block result's gradient dh
     tokens_dh = dh.flatten(0, 1)
     out_rows = out.flatten(0, 1)
-    o_grad += torch.mm(tokens_dh.t(), out_rows.flatten(1), out_dtype=F32)
+    add_weight_grad(o_grad, tokens_dh, out_rows.flatten(1))
     dout = torch.mm(tokens_dh, o_weight).view(out_rows.shape)
     # attention: the value gradient lands straight in its block of d qkv
     values = s.v if table is None else vmix

@@ -90,17 +90,25 @@ int slot_gemm_reduce(const SkinnyGemm &g, int epi, const float *part, long long 
 int slot_gemm_partials(const SkinnyGemm &g, float *part, long long part_bytes, int S, hipStream_t stream);
 
 /* prefill_gemm.hip: out[m][n] = epilogue(sum_k a[m][k] w[n][k]) for the rows of a prefill call, every output's sum in
- * one fixed order over K whatever M is. Epilogues SG_STORE, SG_RESID, SG_F32, SG_RELU2. Returns 0, a hipError_t, or -2
- * when the shape (K a multiple of 128, N of 4, every array under 2 GiB) or an operand the epilogue needs does not fit. */
+ * one fixed order over K whatever M is. Epilogues SG_STORE, SG_RESID, SG_F32, SG_RELU2, and SG_RESID2: SG_RESID that
+ * also writes each 32-column block's sum of squares of the fp32 sum s + res to ssq, from which tile_rstd makes the rows'
+ * rstd. Returns 0, a hipError_t, or -2 when the shape (K a multiple of 128, N of 4, every array under 2 GiB) or an operand
+ * the epilogue needs does not fit. */
 struct PfGemm {
     const uint16_t *a;     /* [M][K] bf16 */
     const uint16_t *w;     /* [N][K] bf16 */
     int M, N, K;
-    uint16_t *out;         /* [M][N] bf16 (SG_STORE, SG_RESID, SG_RELU2) */
+    uint16_t *out;         /* [M][N] bf16 (SG_STORE, SG_RESID, SG_RESID2, SG_RELU2) */
     float *out_f32;        /* [M][N] fp32 (SG_F32) */
-    const uint16_t *res;   /* [M][N] bf16 (SG_RESID) */
+    const uint16_t *res;   /* [M][N] bf16 (SG_RESID, SG_RESID2) */
     const float *rstd;     /* [M] fp32 (SG_RELU2) */
+    float *ssq;            /* [M][pf_ssq_cols(N)] fp32 (SG_RESID2) */
 };
 int prefill_gemm(const PfGemm &g, int epi, hipStream_t stream);
+
+constexpr int PF_SSQ = 32;   /* columns of a sum of squares of SG_RESID2, the same for every tile size */
+__host__ __device__ static inline int pf_ssq_cols(int N) { return (N + PF_SSQ - 1) / PF_SSQ; }
+/* rstd[m] = 1 / sqrt((row m's sums of squares in a fixed order) / N + FLT_EPSILON). Returns 0 or a hipError_t. */
+int tile_rstd(const float *ssq, int M, int N, float *rstd, hipStream_t stream);
 
 }  // namespace nc

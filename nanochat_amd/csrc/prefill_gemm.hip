@@ -28,7 +28,9 @@
  * and store nothing; columns past N (a last partial tile of 256) are not stored.
  *
  * Epilogues (the SG_* kinds of nc_internal.h; decode.cu:133-168 for the math): SG_STORE bf16(s); SG_RESID
- * bf16(s + res); SG_F32 s; SG_RELU2 bf16(relu(p) p) with p = s rstd[m].
+ * bf16(s + res); SG_F32 s; SG_RELU2 bf16(relu(p) p) with p = s rstd[m]; SG_RESID2 SG_RESID that also writes the sum of
+ * squares of every 32 columns of s + res, so the row's rstd needs no pass over the fp32 sums (tile_rstd adds a row's few
+ * block sums).
  *
  * Reference: the prefill rows of dec_prefill run through the step's GEMM body, model/kernels/decode.cu:170-230,
  * 295-359, 1041-1051.
@@ -213,7 +215,9 @@ __device__ __forceinline__ void pg_run(const PfGemm &g, int m0, int n0, unsigned
 
     const Rsrc ro = pg_rsrc(EPI == SG_F32 ? (const void *)g.out_f32 : (const void *)g.out,
                             (long long)g.M * g.N * (EPI == SG_F32 ? 4 : 2));
-    const Rsrc rr = pg_rsrc(g.res, EPI == SG_RESID ? (long long)g.M * g.N * 2 : 0);
+    const Rsrc rr = pg_rsrc(g.res, EPI == SG_RESID || EPI == SG_RESID2 ? (long long)g.M * g.N * 2 : 0);
+    const int sq_cols = pf_ssq_cols(g.N);
+    const Rsrc rq = pg_rsrc(g.ssq, EPI == SG_RESID2 ? (long long)g.M * sq_cols * 4 : 0);
     const Rsrc rs = pg_rsrc(g.rstd, EPI == SG_RELU2 ? (long long)g.M * 4 : 0);
 #pragma unroll
     for (int u = 0; u < P::NU; u++) {
@@ -223,6 +227,37 @@ __device__ __forceinline__ void pg_run(const PfGemm &g, int m0, int n0, unsigned
 #pragma unroll
         for (int t = 0; t < P::NT; t++) {
             const int n = n0 + P::WN * wn + 16 * t + 4 * grp;
+            if (EPI == SG_RESID2) {
+                /* two tiles a 32-column block (every P holds an even number): a lane's chain of 2 x 4 squares, then its
+                 * row's four lane groups; the same order whatever tile holds the block */
+                if (t & 1) continue;
+                float sq = 0.0f;
+#pragma unroll
+                for (int t2 = t; t2 < t + 2; t2++) {
+                    const int nn = n + 16 * (t2 - t), at2 = m * g.N + nn;
+                    const bool in = nn < g.N;
+                    u32x2 rv = u32x2{0u, 0u};
+                    if (in) rv = __builtin_amdgcn_raw_buffer_load_b64(rr, at2 * 2, 0, 0);
+                    const float res[4] = {bf16_to_f32((uint16_t)rv[0]), bf16_to_f32((uint16_t)(rv[0] >> 16)),
+                                          bf16_to_f32((uint16_t)rv[1]), bf16_to_f32((uint16_t)(rv[1] >> 16))};
+                    uint16_t o[4];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const float v = acc[t2][u][e] + res[e];
+                        sq = in ? __builtin_fmaf(v, v, sq) : sq;
+                        o[e] = f32_to_bf16(v);
+                    }
+                    if (in)
+                        __builtin_amdgcn_raw_buffer_store_b64(
+                            u32x2{(uint32_t)o[0] | (uint32_t)o[1] << 16, (uint32_t)o[2] | (uint32_t)o[3] << 16}, ro,
+                            at2 * 2, 0, 0);
+                }
+                sq = pair_sum32(pair_sum16(sq));
+                const int blk = (n0 + P::WN * wn + 16 * t) / PF_SSQ;
+                if (grp == 0 && blk < sq_cols)
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(sq), rq, (m * sq_cols + blk) * 4, 0, 0);
+                continue;
+            }
             if (n >= g.N) continue;
             const int at = m * g.N + n;   /* rows past M lie outside the views' ranges: no access */
             float s[4] = {acc[t][u][0], acc[t][u][1], acc[t][u][2], acc[t][u][3]};
@@ -281,8 +316,8 @@ __device__ __forceinline__ int2 pg_band(int id, int T, int nx) {
 enum { PG_WHOLE, PG_SPLIT, PG_THIN };
 
 template <int EPI, int MODE>
-__global__ void __launch_bounds__(PG_WAVES * WAVE, 1) prefill_gemm_kernel(PfGemm g, int full, int pieces) {
-    __shared__ __align__(16) unsigned char b0[PG_STAGE], b1[PG_STAGE], b2[PG_STAGE], b3[PG_STAGE];
+__device__ __forceinline__ void pg_body(const PfGemm &g, int full, int pieces, unsigned char *b0, unsigned char *b1,
+                                        unsigned char *b2, unsigned char *b3) {
     const int nx = (g.N + 255) / 256, T = nx * ((g.M + 255) / 256), L = blockIdx.x;
     if (MODE == PG_THIN) {
         pg_run<PgThin, EPI>(g, 0, pg_order(L, nx) * 256, b0, b1, b2, b3);
@@ -302,6 +337,39 @@ __global__ void __launch_bounds__(PG_WAVES * WAVE, 1) prefill_gemm_kernel(PfGemm
         const int m0 = tile.y * 256 + 128 * (p >> 1), n0 = tile.x * 256 + 128 * (p & 1);
         if (m0 < g.M && n0 < g.N) pg_run<PgQuarter, EPI>(g, m0, n0, b0, b1, b2, b3);
     }
+}
+
+template <int EPI, int MODE>
+__global__ void __launch_bounds__(PG_WAVES * WAVE, 1) prefill_gemm_kernel(PfGemm g, int full, int pieces) {
+    __shared__ __align__(16) unsigned char b0[PG_STAGE], b1[PG_STAGE], b2[PG_STAGE], b3[PG_STAGE];
+    pg_body<EPI, MODE>(g, full, pieces, b0, b1, b2, b3);
+}
+
+/* The same with the SG_RESID2 epilogue (a kernel of its own name: a projection with its residual and row statistic). */
+template <int MODE>
+__global__ void __launch_bounds__(PG_WAVES * WAVE, 1) projection_gemm_kernel(PfGemm g, int full, int pieces) {
+    __shared__ __align__(16) unsigned char b0[PG_STAGE], b1[PG_STAGE], b2[PG_STAGE], b3[PG_STAGE];
+    pg_body<SG_RESID2, MODE>(g, full, pieces, b0, b1, b2, b3);
+}
+
+/* 16 lanes a row: lane l adds blocks l, l + 16, ... in order, then the lanes' sums meet by the fixed DPP butterfly. */
+__global__ void __launch_bounds__(256) tile_rstd_kernel(const float *ssq, int M, int cols, float inv, float *rstd) {
+    const int l = threadIdx.x & 15, m = blockIdx.x * 16 + (threadIdx.x >> 4);
+    if (m >= M) return;   /* whole 16-lane groups */
+    float v = 0.0f;
+    for (int j = l; j < cols; j += 16) v = v + ssq[(long long)m * cols + j];
+    v = v + lane_xor_dpp<8>(v);
+    v = v + lane_xor_dpp<4>(v);
+    v = v + lane_xor_dpp<2>(v);
+    v = v + lane_xor_dpp<1>(v);
+    if (l == 0) rstd[m] = 1.0f / __builtin_sqrtf(v * inv + FLT_EPS);
+}
+
+int tile_rstd(const float *ssq, int M, int N, float *rstd, hipStream_t stream) {
+    if (M <= 0) return 0;
+    hipLaunchKernelGGL(tile_rstd_kernel, dim3((M + 15) / 16), dim3(256), 0, stream, ssq, M, pf_ssq_cols(N),
+                       1.0f / (float)N, rstd);
+    return (int)hipGetLastError();
 }
 
 /* The number of compute units of the current device (256 if it cannot be read), once per device. */
@@ -324,8 +392,9 @@ int prefill_gemm(const PfGemm &g, int epi, hipStream_t stream) {
         (long long)g.M * g.N * 4 >= (1LL << 31))
         return NC_ERR_SHAPE;
     const bool f32 = epi == SG_F32;
-    if ((f32 ? !g.out_f32 : !g.out) || (epi == SG_RESID && !g.res) || (epi == SG_RELU2 && !g.rstd) ||
-        (epi != SG_STORE && epi != SG_RESID && epi != SG_F32 && epi != SG_RELU2))
+    if ((f32 ? !g.out_f32 : !g.out) || ((epi == SG_RESID || epi == SG_RESID2) && !g.res) ||
+        (epi == SG_RESID2 && !g.ssq) || (epi == SG_RELU2 && !g.rstd) ||
+        (epi != SG_STORE && epi != SG_RESID && epi != SG_RESID2 && epi != SG_F32 && epi != SG_RELU2))
         return NC_ERR_SHAPE;
     /* T tiles in rounds of one workgroup a CU: the R = T mod CUs tiles of a last part-filled round are cut into 4
      * (R <= CUs / 4) or 2 (R <= CUs / 2) pieces when there are earlier full rounds; otherwise every tile is whole. */
@@ -335,21 +404,30 @@ int prefill_gemm(const PfGemm &g, int epi, hipStream_t stream) {
     const int full = pieces > 1 ? T - R : T;
     const dim3 grid(full + (T - full) * pieces), block(PG_WAVES * WAVE);
     const int mode = g.M <= 128 ? PG_THIN : pieces > 1 ? PG_SPLIT : PG_WHOLE;
-#define PG_LAUNCH(E)                                                                                             \
-    do {                                                                                                         \
-        if (mode == PG_THIN) hipLaunchKernelGGL((prefill_gemm_kernel<E, PG_THIN>), grid, block, 0, stream, g, full,  \
-                                                pieces);                                                         \
-        else if (mode == PG_SPLIT) hipLaunchKernelGGL((prefill_gemm_kernel<E, PG_SPLIT>), grid, block, 0, stream, g, \
-                                                      full, pieces);                                             \
-        else hipLaunchKernelGGL((prefill_gemm_kernel<E, PG_WHOLE>), grid, block, 0, stream, g, full, pieces);     \
+#define PG_LAUNCH_MODES(KERNEL)                                                                          \
+    do {                                                                                                   \
+        if (mode == PG_THIN) hipLaunchKernelGGL((KERNEL(PG_THIN)), grid, block, 0, stream, g, full, pieces);        \
+        else if (mode == PG_SPLIT) hipLaunchKernelGGL((KERNEL(PG_SPLIT)), grid, block, 0, stream, g, full, pieces); \
+        else hipLaunchKernelGGL((KERNEL(PG_WHOLE)), grid, block, 0, stream, g, full, pieces);                \
     } while (0)
+#define PG_STORE_KERNEL(MODE) prefill_gemm_kernel<SG_STORE, MODE>
+#define PG_RESID_KERNEL(MODE) prefill_gemm_kernel<SG_RESID, MODE>
+#define PG_F32_KERNEL(MODE) prefill_gemm_kernel<SG_F32, MODE>
+#define PG_RELU2_KERNEL(MODE) prefill_gemm_kernel<SG_RELU2, MODE>
+#define PG_RESID2_KERNEL(MODE) projection_gemm_kernel<MODE>
     switch (epi) {
-    case SG_STORE: PG_LAUNCH(SG_STORE); break;
-    case SG_RESID: PG_LAUNCH(SG_RESID); break;
-    case SG_F32: PG_LAUNCH(SG_F32); break;
-    default: PG_LAUNCH(SG_RELU2); break;
+    case SG_STORE: PG_LAUNCH_MODES(PG_STORE_KERNEL); break;
+    case SG_RESID: PG_LAUNCH_MODES(PG_RESID_KERNEL); break;
+    case SG_RESID2: PG_LAUNCH_MODES(PG_RESID2_KERNEL); break;
+    case SG_F32: PG_LAUNCH_MODES(PG_F32_KERNEL); break;
+    default: PG_LAUNCH_MODES(PG_RELU2_KERNEL); break;
     }
-#undef PG_LAUNCH
+#undef PG_LAUNCH_MODES
+#undef PG_STORE_KERNEL
+#undef PG_RESID_KERNEL
+#undef PG_F32_KERNEL
+#undef PG_RELU2_KERNEL
+#undef PG_RESID2_KERNEL
     return (int)hipGetLastError();
 }
 

@@ -26,8 +26,9 @@ INCLUDE = PACKAGE.parent / "include"
 LIB_DIR = PACKAGE / "lib"
 LIBRARY = LIB_DIR / "libnanochat_kv.so"
 DECODE_LIBRARY = LIB_DIR / "libnanochat_decode.so"
-KERNEL_SOURCES = [CSRC / "kv_append.hip", CSRC / "attention.hip", CSRC / "ve_gate.hip", CSRC / "flash_attn.hip"]
-DECODE_SOURCES = [CSRC / "decoder.hip", CSRC / "slot_gemm.hip", CSRC / "prefill_gemm.hip"]
+KERNEL_SOURCES = [CSRC / "kv_append.hip", CSRC / "attention.hip", CSRC / "ve_gate.hip", CSRC / "flash_attn.hip",
+                  CSRC / "prefill_gemm.hip", CSRC / "train_gemm.hip"]
+DECODE_SOURCES = [CSRC / "decoder.hip", CSRC / "slot_gemm.hip"]
 SOURCES = KERNEL_SOURCES + DECODE_SOURCES
 HEADERS = [CSRC / "nc_device.h", CSRC / "nc_internal.h", INCLUDE / "nanochat_amd.h", INCLUDE / "nanochat_decode.h"]
 HEAD_DIM = 128
@@ -106,6 +107,10 @@ SIGNATURES = {
     "nc_flash_attn_bwd": ([c_void_p] * 4 + [c_longlong] * 4 + [c_void_p, c_longlong, c_void_p, c_void_p, c_int, c_int,
                                                                 c_int, c_int, c_float, c_void_p, c_void_p, c_void_p,
                                                                 c_longlong, c_longlong, c_longlong, c_void_p], c_int),
+    "nc_linear_residual_rms": ([c_void_p] * 3 + [c_longlong, c_int, c_int] + [c_void_p] * 3 + [c_longlong, c_void_p],
+                               c_int),
+    "nc_weight_grad_workspace_bytes": ([c_longlong, c_int, c_int], c_longlong),
+    "nc_weight_grad": ([c_void_p, c_void_p, c_longlong, c_int, c_int, c_void_p, c_void_p, c_longlong, c_void_p], c_int),
     "nc_flash_attn_bwd_rows": ([c_void_p, c_longlong, c_void_p, c_longlong, c_longlong, c_int, c_void_p, c_void_p],
                                c_int),
 }

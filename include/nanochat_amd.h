@@ -87,6 +87,13 @@ int nc_ve_backward(const void *dout, long long dout_stride, const int32_t *ids, 
                    const float *table, long long vocab, const float *w, const float *gate, void *dn, float *dtable,
                    void *dz, long long rows, int heads, void *stream);
 
+/* The gate weight's gradient dw [heads][C] = dz^T n in fp32, summed in a fixed order: dz bf16 [rows][heads] (of
+ * nc_ve_backward), n bf16 [rows][C] contiguous, 8-byte aligned; rows >= 1. workspace:
+ * nc_ve_weight_grad_workspace_bytes (0 for no rows, -1 for sizes it does not take). */
+long long nc_ve_weight_grad_workspace_bytes(long long rows, int heads);
+int nc_ve_weight_grad(const void *dz, const void *n, long long rows, int heads, float *dw, void *workspace,
+                      long long workspace_bytes, void *stream);
+
 /*
  * Training attention forward: the varlen causal attention the reference runs through FlashAttention-4
  * (model/ops/flash_attn.py:340-345, _flash_attn_fwd(q, k, v, cu_seqlens, cu_seqlens, T, T, causal=True,

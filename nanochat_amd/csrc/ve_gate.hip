@@ -11,7 +11,7 @@
  *   dz[r][h]     = bf16(2 dg[h] (1 - s) s) with s = gate[r][h] / 2   (dz_fp32, unrounded, feeds dn)
  *   dn[r][c]     = bf16(sum_h dz_fp32[h] w[h][c])
  *   dtable[t][c] += sum over the rows of token t of bf16(gate[r][c / 128] * dout[r][c])   (fp32, added in)
- * dw = dz^T n is a library GEMM on the host side, as in the reference. ids must hold equal tokens adjacently (sorted,
+ * dw = dz^T n (nc_ve_weight_grad; a GEMM on the host side in the reference). ids must hold equal tokens adjacently (sorted,
  * the reference's contract, model/ops/ve_gate.py:23-26): the table gradient of a token split into separate runs is
  * undefined.
  *
@@ -234,9 +234,10 @@ __device__ __forceinline__ void stage_w_rows(float *ws, const float *w) {
 
 /* A run's accumulated table gradient added into dtable row t. With equal tokens adjacent in `ids` (sorted, the
  * reference's contract), a run that neither starts at the wave's first position nor ends at its last one holds every
- * occurrence of its token, so no other wave touches that row: a plain read-add-write. The first and last run of a
- * wave's range may continue in the neighbouring waves' ranges: hardware fp32 atomics (two instructions per head,
- * each 64 dwords at 8-byte stride). */
+ * occurrence of its token, so no other wave touches that row: a plain read-add-write. So does a wave's first or last run
+ * when the id before or after its range is another token; otherwise the run continues in a neighbouring wave's range:
+ * hardware fp32 atomics (two instructions per head, each 64 dwords at 8-byte stride). Few rows a wave make most runs
+ * first or last ones: 4,096 rows (one a wave) VEB_FIGURES */
 template <int H>
 __device__ __forceinline__ void flush_run(float *dtable, int t, const float (&acc)[H][2], int lane, bool shared) {
     float *row = dtable + (long long)t * (H * HEAD_DIM) + 2 * lane;
@@ -272,7 +273,9 @@ __global__ void __launch_bounds__(VE_THREADS) ve_backward_kernel(VeBwd a) {
     float acc[H][2];
     uint32_t eb[H];   /* the run's table columns as bf16x2 */
     int cur = -1;
-    bool cur_ok = false, started = false, first = true;   /* first: the current run is the wave's first */
+    bool cur_ok = false, started = false, shared = false;   /* shared: the current run began in the wave before */
+    const int before = p0 > 0 && p0 < p1 ? __builtin_amdgcn_readfirstlane(a.ids[p0 - 1]) : 0;
+    const int after = p1 < a.rows && p0 < p1 ? __builtin_amdgcn_readfirstlane(a.ids[p1]) : 0;
     for (long long p = p0; p < p1; p++) {
         const long long r = uniform64(a.order[p]);
         if (r < 0 || r >= a.rows) continue;   /* not a row: nothing to read or write */
@@ -286,10 +289,8 @@ __global__ void __launch_bounds__(VE_THREADS) ve_backward_kernel(VeBwd a) {
             g[k] = a.gate[r * H + k];
         }
         if (!started || t != cur) {
-            if (started) {
-                if (cur_ok) flush_run<H>(a.dtable, cur, acc, lane, first);
-                first = false;
-            }
+            if (started && cur_ok) flush_run<H>(a.dtable, cur, acc, lane, shared);
+            shared = !started && p0 > 0 && t == before;
             started = true;
             cur = t;
             cur_ok = t >= 0 && (long long)t < a.vocab;
@@ -329,7 +330,114 @@ __global__ void __launch_bounds__(VE_THREADS) ve_backward_kernel(VeBwd a) {
                                                   (k * HEAD_DIM + 2 * lane) * 2, 0, 0);
         }
     }
-    if (started && cur_ok) flush_run<H>(a.dtable, cur, acc, lane, true);
+    if (started && cur_ok) flush_run<H>(a.dtable, cur, acc, lane, shared || (p1 < a.rows && cur == after));
+}
+
+/* The gate weight's gradient dw[h][c] = sum over rows of dz[row][h] n[row][c] (bf16 operands, fp32 sums): H <= 16
+ * outputs a column, so it is bound by reading n once, not by the products, and a matrix product's tiles (H of 16 rows
+ * used, a few column tiles for the whole sum over the rows) leave the chip idle. A block takes a slab of rows and 256
+ * columns, a lane four columns of all H heads; 64 rows at a time, 16 a wave, dz through LDS. The waves' and then the
+ * slabs' sums are added in a fixed order. 65,536 rows, H = 6: VEW_FIGURES */
+struct VeWeight {
+    const uint16_t *dz;   /* [rows][H] bf16 */
+    const uint16_t *n;    /* [rows][C] bf16 */
+    long long rows, per;  /* rows of a slab: a multiple of VW_ROWS */
+    float *part;          /* [slabs][H][C] */
+};
+
+constexpr int VW_ROWS = 64, VW_COLS = 256, VW_WAVES = 4;
+constexpr int VW_PER = VW_ROWS / VW_WAVES;
+
+template <int H>
+__global__ void __launch_bounds__(VW_WAVES *WAVE) ve_weight_kernel(VeWeight a) {
+    constexpr int C = H * HEAD_DIM;
+    __shared__ float z[VW_ROWS * H];
+    __shared__ __align__(16) float red[VW_WAVES][VW_COLS];
+    const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x >> 6;
+    const int col = blockIdx.y * VW_COLS + lane * 4;
+    const bool in = col < C;
+    const long long r0 = blockIdx.x * a.per, r1 = r0 + a.per < a.rows ? r0 + a.per : a.rows;
+    float acc[H][4];
+#pragma unroll
+    for (int h = 0; h < H; h++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[h][e] = 0.0f;
+    for (long long r = r0; r < r1; r += VW_ROWS) {
+        const int live = (int)(r1 - r < VW_ROWS ? r1 - r : VW_ROWS);
+        uint2 x[VW_PER];
+#pragma unroll
+        for (int k = 0; k < VW_PER; k++) {
+            const int row = wave * VW_PER + k;
+            x[k] = in && row < live ? *reinterpret_cast<const uint2 *>(a.n + (r + row) * C + col) : uint2{0u, 0u};
+        }
+        __syncthreads();   /* the rows before are done with z */
+        for (int i = threadIdx.x; i < VW_ROWS * H; i += VW_WAVES * WAVE) z[i] = i < live * H ? bf16_to_f32(a.dz[r * H + i]) : 0.0f;
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < VW_PER; k++) {
+            const float f[4] = {__uint_as_float(x[k].x << 16), __uint_as_float(x[k].x & 0xFFFF0000u),
+                                __uint_as_float(x[k].y << 16), __uint_as_float(x[k].y & 0xFFFF0000u)};
+#pragma unroll
+            for (int h = 0; h < H; h++) {
+                const float d = z[(wave * VW_PER + k) * H + h];
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[h][e] = __builtin_fmaf(d, f[e], acc[h][e]);
+            }
+        }
+    }
+#pragma unroll 1
+    for (int h = 0; h < H; h++) {
+        float4 v = float4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int k = 0; k < H; k++)   /* acc[h] without indexing registers */
+            if (k == h) v = float4{acc[k][0], acc[k][1], acc[k][2], acc[k][3]};
+        __syncthreads();
+        *reinterpret_cast<float4 *>(&red[wave][lane * 4]) = v;
+        __syncthreads();
+        const int c = blockIdx.y * VW_COLS + threadIdx.x;
+        if (c < C)
+            a.part[((long long)blockIdx.x * H + h) * C + c] =
+                ((red[0][threadIdx.x] + red[1][threadIdx.x]) + red[2][threadIdx.x]) + red[3][threadIdx.x];
+    }
+}
+
+/* dw from the slabs' partials: 64 outputs a block, group g of 16 adds the g-th sixteenth of the slabs, then the groups in
+ * order. */
+__global__ void __launch_bounds__(1024) ve_weight_sum_kernel(const float *part, int slabs, int n, float *dw) {
+    __shared__ float sums[16][64];
+    const int o = threadIdx.x & 63, g = threadIdx.x >> 6, i = blockIdx.x * 64 + o;   /* n is a multiple of 64 */
+    const int s0 = slabs * g / 16, s1 = slabs * (g + 1) / 16;
+    float sum = 0.0f;
+#pragma unroll 8
+    for (int s = s0; s < s1; s++) sum = sum + part[(long long)s * n + i];
+    sums[g][o] = sum;
+    __syncthreads();
+    if (g) return;
+    for (int k = 1; k < 16; k++) sum = sum + sums[k][o];
+    dw[i] = sum;
+}
+
+/* Slabs of `rows` rows for H heads: about four blocks a CU, none of fewer than VW_ROWS rows. */
+void ve_weight_slabs(long long rows, int heads, int &slabs, long long &per) {
+    const int chunks = (heads * HEAD_DIM + VW_COLS - 1) / VW_COLS;
+    const long long tiles = (rows + VW_ROWS - 1) / VW_ROWS, most = 1024 / chunks;
+    const long long want = tiles < most ? tiles : most;
+    per = (tiles + want - 1) / want * VW_ROWS;
+    slabs = (int)((rows + per - 1) / per);
+}
+
+template <int H = 1>
+int launch_weight(int heads, const VeWeight &a, int slabs, float *dw, hipStream_t stream) {
+    if constexpr (H > VE_MAX_HEADS) {
+        return NC_ERR_SHAPE;
+    } else {
+        if (heads != H) return launch_weight<H + 1>(heads, a, slabs, dw, stream);
+        constexpr int C = H * HEAD_DIM;
+        hipLaunchKernelGGL(ve_weight_kernel<H>, dim3(slabs, (C + VW_COLS - 1) / VW_COLS), dim3(VW_WAVES * WAVE), 0,
+                           stream, a);
+        hipLaunchKernelGGL(ve_weight_sum_kernel, dim3(H * C / 64), dim3(1024), 0, stream, a.part, slabs, H * C, dw);
+        return (int)hipGetLastError();
+    }
 }
 
 /* Workgroups for `rows` rows: every row a wave, at most as many workgroups as the device holds at once (the
@@ -463,4 +571,29 @@ extern "C" int nc_ve_backward(const void *dout, long long dout_stride, const int
                               float *dtable, void *dz, long long rows, int heads, void *stream) {
     return ve_backward_run(backward_args(dout, dout_stride, ids, order, table, vocab, w, gate, dn, dtable, dz, rows),
                            heads, (hipStream_t)stream);
+}
+
+extern "C" long long nc_ve_weight_grad_workspace_bytes(long long rows, int heads) {
+    if (rows < 0 || rows > (1LL << 40) || heads < 1 || heads > VE_MAX_HEADS) return -1;
+    if (rows == 0) return 0;
+    int slabs;
+    long long per;
+    ve_weight_slabs(rows, heads, slabs, per);
+    return (long long)slabs * heads * heads * HEAD_DIM * 4;
+}
+
+extern "C" int nc_ve_weight_grad(const void *dz, const void *n, long long rows, int heads, float *dw, void *workspace,
+                                 long long workspace_bytes, void *stream) {
+    const long long need = nc_ve_weight_grad_workspace_bytes(rows, heads);
+    if (need <= 0) return NC_ERR_SHAPE;   /* no rows: the caller's zeros */
+    if (!dz || !n || !dw || !workspace) return NC_ERR_NULL;
+    if (((uintptr_t)n & 7) || ((uintptr_t)dz & 1) || (((uintptr_t)dw | (uintptr_t)workspace) & 3)) return NC_ERR_SHAPE;
+    if (workspace_bytes < need) return NC_ERR_WORKSPACE;
+    VeWeight a;
+    a.dz = (const uint16_t *)dz; a.n = (const uint16_t *)n;
+    a.rows = rows;
+    int slabs;
+    ve_weight_slabs(rows, heads, slabs, a.per);
+    a.part = (float *)workspace;
+    return launch_weight(heads, a, slabs, dw, (hipStream_t)stream);
 }

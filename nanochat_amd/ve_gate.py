@@ -43,4 +43,19 @@ def ve_backward(dv: Tensor, n: Tensor, ids: Tensor, order: Tensor, table: Tensor
     check(hip_library().nc_ve_backward(pointer(dv), ctypes.c_longlong(dv.stride(1)), pointer(ids), pointer(order),
                                        pointer(table), table.size(0), pointer(w), pointer(gate), pointer(dn),
                                        pointer(table.grad), pointer(dz), ids.numel(), w.size(0), stream()))
-    return dn, torch.mm(dz.t().contiguous(), n.view(-1, n.size(-1)), out_dtype=w.dtype)
+    return dn, _weight_grad(dz, n.view(-1, n.size(-1)), w)
+
+
+def _weight_grad(dz: Tensor, n: Tensor, w: Tensor) -> Tensor:
+    """dw = dz^T n over the rows, fp32 sums, like w: the HIP kernel for dense bf16 rows and fp32 w, else a library GEMM."""
+    rows = dz.size(0)
+    if (rows and n.dtype == torch.bfloat16 and n.is_contiguous() and n.data_ptr() % 8 == 0 and w.dtype == torch.float32
+            and tuple(n.shape) == (rows, w.size(1)) and w.size(1) == w.size(0) * 128 and dz.size(1) == w.size(0)):
+        lib = hip_library()
+        need = lib.nc_ve_weight_grad_workspace_bytes(rows, w.size(0))
+        if need > 0:
+            dw = torch.empty_like(w, memory_format=torch.contiguous_format)
+            ws = torch.empty(need, dtype=torch.uint8, device=n.device)
+            check(lib.nc_ve_weight_grad(pointer(dz), pointer(n), rows, w.size(0), pointer(dw), pointer(ws), need, stream()))
+            return dw
+    return torch.mm(dz.t().contiguous(), n, out_dtype=w.dtype)

@@ -213,3 +213,57 @@ def test_torch_surface_matches_oracle(device):
     dw64 = ov.weight_grad(dz_b, n_)
     bound = (np.abs(dz_b).astype(np.float64).T @ np.abs(n_).astype(np.float64))
     assert np.all(np.abs(dw.cpu().numpy() - dw64) <= bound * 2.0 ** -7 + 1e-6)
+
+
+@pytest.mark.parametrize("rows,H", [(1, 1), (63, 2), (65, 3), (1000, 6), (20000, 6), (70001, 13), (513, 16)])
+def test_weight_grad_matches_float64(device, rows, H):
+    """dw = dz^T n at row counts around the kernel's 64-row tiles and its slabs, odd and even head counts (a half-empty
+    last column chunk): within the bound of an fp32 sum of `rows` terms, and the same bits twice; rows that are not
+    8-byte aligned go through the library and agree."""
+    from nanochat_amd.ve_gate import _weight_grad
+
+    gen = torch.Generator().manual_seed(rows + H)
+    dz = torch.randn(rows, H, generator=gen).bfloat16()
+    n = torch.randn(rows, H * HEAD_DIM, generator=gen).bfloat16()
+    w = torch.empty(H, H * HEAD_DIM, device=device)
+    odd = torch.empty(n.numel() + 1, dtype=n.dtype, device=device)[1:].view(n.shape)
+    odd.copy_(n)
+    got = [_weight_grad(dz.to(device), x, w) for x in (n.to(device), n.to(device), odd)]
+    torch.cuda.synchronize()
+    assert torch.equal(got[0], got[1])
+    want, mag = dz.double().t() @ n.double(), dz.double().abs().t() @ n.double().abs()
+    for g in got[::2]:
+        assert bool(((g.double().cpu() - want).abs() <= (rows + 16) * 2.0 ** -23 * mag).all())
+
+
+def test_runs_that_end_at_wave_borders(device):
+    """Fewer rows than waves (a row a wave): every run is a wave's first and last, alone or shared with its neighbours;
+    runs of one, two and many rows, a skipped row (order outside the rows) inside a run. dtable within fp32 rounding of
+    float64."""
+    H, vocab = 2, 40
+    C = H * HEAD_DIM
+    idx = torch.tensor([0] * 9 + [3] + [5, 5] + [7] + [9] * 4 + [11, 12, 13] + [39] * 2, dtype=torch.int32)
+    rows = idx.numel()
+    gen = torch.Generator().manual_seed(2)
+    table = torch.randn(vocab, C, generator=gen)
+    w = torch.randn(H, C, generator=gen) * 0.05
+    gate = torch.rand(rows, H, generator=gen) * 2
+    dout = torch.randn(rows, C, generator=gen).bfloat16()
+    order = torch.arange(rows)
+    order[4] = rows + 5                                     # skipped
+    dtable0 = torch.randn(vocab, C, generator=gen)
+    d = [t.to(device) for t in (dout, idx, order, table, w, gate, dtable0)]
+    dn, dz = torch.empty(rows, C, dtype=torch.bfloat16, device=device), torch.empty(rows, H, dtype=torch.bfloat16,
+                                                                                    device=device)
+    assert hip_library().nc_ve_backward(pointer(d[0]), C, pointer(d[1]), pointer(d[2]), pointer(d[3]), vocab,
+                                        pointer(d[4]), pointer(d[5]), pointer(dn), pointer(d[6]), pointer(dz), rows, H,
+                                        stream()) == 0
+    torch.cuda.synchronize()
+    want, mag = dtable0.double().clone(), dtable0.double().abs()
+    for p in range(rows):
+        if p == 4:
+            continue
+        g = (gate[p].repeat_interleave(HEAD_DIM) * dout[p].float()).bfloat16().double()
+        want[idx[p]] += g
+        mag[idx[p]] += g.abs()
+    assert bool(((d[6].double().cpu() - want).abs() <= 12 * 2.0 ** -24 * mag + 1e-12).all())

@@ -234,12 +234,15 @@ __device__ __forceinline__ void stage_w_rows(float *ws, const float *w) {
 
 /* A run's accumulated table gradient added into dtable row t. With equal tokens adjacent in `ids` (sorted, the
  * reference's contract), a run that neither starts at the wave's first position nor ends at its last one holds every
- * occurrence of its token, so no other wave touches that row: a plain read-add-write. So does a wave's first or last run
- * when the id before or after its range is another token; otherwise the run continues in a neighbouring wave's range:
- * hardware fp32 atomics (two instructions per head, each 64 dwords at 8-byte stride). Few rows a wave make most runs
- * first or last ones: 4,096 rows (one a wave) VEB_FIGURES */
+ * occurrence of its token, so no other wave touches that row: a plain read-add-write, the row read when the run began
+ * (old). So does a wave's first or last run when the id before or after its range is another token; otherwise (shared) the
+ * run continues in a neighbouring wave's range: hardware fp32 atomics (two instructions per head, each 64 dwords at
+ * 8-byte stride). */
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
 template <int H>
-__device__ __forceinline__ void flush_run(float *dtable, int t, const float (&acc)[H][2], int lane, bool shared) {
+__device__ __forceinline__ void flush_run(float *dtable, int t, const float (&acc)[H][2], const u32x2 (&old)[H], int lane,
+                                          bool shared) {
     float *row = dtable + (long long)t * (H * HEAD_DIM) + 2 * lane;
     if (shared) {
 #pragma unroll
@@ -248,96 +251,172 @@ __device__ __forceinline__ void flush_run(float *dtable, int t, const float (&ac
             unsafeAtomicAdd(row + k * HEAD_DIM + 1, acc[k][1]);
         }
     } else {
-        float2 cur[H];
-#pragma unroll
-        for (int k = 0; k < H; k++) cur[k] = *reinterpret_cast<const float2 *>(row + k * HEAD_DIM);
 #pragma unroll
         for (int k = 0; k < H; k++)
-            *reinterpret_cast<float2 *>(row + k * HEAD_DIM) = float2{cur[k].x + acc[k][0], cur[k].y + acc[k][1]};
+            *reinterpret_cast<float2 *>(row + k * HEAD_DIM) =
+                float2{__uint_as_float(old[k][0]) + acc[k][0], __uint_as_float(old[k][1]) + acc[k][1]};
+    }
+}
+
+/* What one position needs, fetched a position ahead: its row and token, the row of dout and, when it begins a run, the
+ * token's table row and (for a run this wave alone holds from here) its row of dtable. */
+template <int H>
+struct VeRow {
+    long long r;
+    int t;
+    bool valid, fresh, ok;   /* a row; the first of a run; a token of the table */
+    bool shared;             /* fresh: the run began in the wave before */
+    uint32_t d[H], g;        /* g: lane h the row's gate of head h */
+    u32x2 e[H], old[H];
+};
+
+/* Up to 64 positions' rows and tokens, lane l position l's. */
+struct VePositions {
+    uint32_t row_lo, row_hi;
+    int id;
+    int n;
+};
+
+/* Position q's row, with `run` the token of the run before it (started: there is one). Loads a position does not need go
+ * through zero-size descriptors: no access, and no branch that would make the compiler wait for those in flight. */
+template <int H>
+__device__ __forceinline__ void ve_fetch(const VeBwd &a, const VePositions &ps, int q, bool has_before, int before,
+                                         bool started, int run, int lane, VeRow<H> &w) {
+    constexpr int C = H * HEAD_DIM;
+    const bool in = q < ps.n;
+    const int l = q & (WAVE - 1);
+    const uint32_t lo = __builtin_amdgcn_readlane(ps.row_lo, l), hi = __builtin_amdgcn_readlane(ps.row_hi, l);
+    w.r = in ? (long long)(((unsigned long long)hi << 32) | lo) : -1;
+    w.t = __builtin_amdgcn_readlane(ps.id, l);
+    w.valid = w.r >= 0 && w.r < a.rows;   /* not a row: nothing to read or write */
+    w.fresh = w.valid && (!started || w.t != run);
+    w.ok = w.t >= 0 && (long long)w.t < a.vocab;
+    w.shared = !started && has_before && w.t == before;
+    const bool row = w.fresh && w.ok;
+    const Rsrc rd = row_rsrc(a.dout + (w.valid ? w.r * a.dout_stride : 0), w.valid ? C * 2 : 0);
+    const Rsrc re = row_rsrc(a.table + (row ? (long long)w.t * C : 0), row ? C * 4 : 0);
+    const Rsrc ro = row_rsrc(a.dtable + (row ? (long long)w.t * C : 0), row && !w.shared ? C * 4 : 0);
+    w.g = __builtin_amdgcn_raw_buffer_load_b32(row_rsrc(a.gate + (w.valid ? w.r * H : 0), w.valid ? H * 4 : 0), lane * 4,
+                                               0, 0);
+#pragma unroll
+    for (int k = 0; k < H; k++) {
+        w.d[k] = __builtin_amdgcn_raw_buffer_load_b32(rd, (k * HEAD_DIM + 2 * lane) * 2, 0, 2);
+        w.e[k] = __builtin_amdgcn_raw_buffer_load_b64(re, (k * HEAD_DIM + 2 * lane) * 4, 0, 0);
+        w.old[k] = __builtin_amdgcn_raw_buffer_load_b64(ro, (k * HEAD_DIM + 2 * lane) * 4, 0, 0);
+    }
+}
+
+/* The run a wave is in. */
+template <int H>
+struct VeRun {
+    bool started, ok, shared;
+    int t;
+    uint32_t eb[H];     /* the token's table columns as bf16x2 */
+    float acc[H][2];
+    u32x2 old[H];       /* the token's row of dtable before the run */
+};
+
+template <int H>
+__device__ __forceinline__ void ve_row(const VeBwd &a, const float *ws, const VeRow<H> &w, VeRun<H> &run, int lane) {
+    constexpr int C = H * HEAD_DIM;
+    if (!w.valid) return;
+    if (w.fresh) {
+        if (run.started && run.ok) flush_run<H>(a.dtable, run.t, run.acc, run.old, lane, run.shared);
+        run.started = true;
+        run.shared = w.shared;
+        run.t = w.t;
+        run.ok = w.ok;
+#pragma unroll
+        for (int k = 0; k < H; k++) {
+            run.eb[k] = (uint32_t)f32_to_bf16(__uint_as_float(w.e[k][0])) |
+                        ((uint32_t)f32_to_bf16(__uint_as_float(w.e[k][1])) << 16);
+            run.old[k] = w.old[k];
+            run.acc[k][0] = 0.0f;
+            run.acc[k][1] = 0.0f;
+        }
+    }
+    float dz[H], mine = 0.0f;
+#pragma unroll
+    for (int k = 0; k < H; k++) {
+        const float g = __uint_as_float(__builtin_amdgcn_readlane(w.g, k));
+        const float d0 = __uint_as_float(w.d[k] << 16), d1 = __uint_as_float(w.d[k] & 0xFFFF0000u);
+        const float e0 = __uint_as_float(run.eb[k] << 16), e1 = __uint_as_float(run.eb[k] & 0xFFFF0000u);
+        run.acc[k][0] = run.acc[k][0] + bf16r(g * d0);
+        run.acc[k][1] = run.acc[k][1] + bf16r(g * d1);
+        const float dg = wave_sum(__builtin_fmaf(d1, e1, d0 * e0)), sg = g * 0.5f;
+        dz[k] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(2.0f * dg * (1.0f - sg) * sg)));
+        if (lane == k) mine = dz[k];
+    }
+    __builtin_amdgcn_raw_buffer_store_b16(f32_to_bf16(mine), row_rsrc(a.dz + w.r * H, H * 2), lane * 2, 0, 0);
+    const Rsrc rn = row_rsrc(a.dn + w.r * C, C * 2);
+    /* dn one head's columns at a time (a loop, so w's LDS reads are not all hoisted into registers) */
+#pragma unroll 1
+    for (int k = 0; k < H; k++) {
+        float x0 = 0.0f, x1 = 0.0f;
+#pragma unroll
+        for (int h = 0; h < H; h++) {
+            const float2 wv = *reinterpret_cast<const float2 *>(ws + h * C + k * HEAD_DIM + 2 * lane);
+            x0 = __builtin_fmaf(dz[h], wv.x, x0);
+            x1 = __builtin_fmaf(dz[h], wv.y, x1);
+        }
+        __builtin_amdgcn_raw_buffer_store_b32((uint32_t)f32_to_bf16(x0) | ((uint32_t)f32_to_bf16(x1) << 16), rn,
+                                              (k * HEAD_DIM + 2 * lane) * 2, 0, 0);
     }
 }
 
 /* Backward mapping (unlike the forward's): lane l holds columns k*128 + 2l and k*128 + 2l + 1 of every head k, so a
  * head's gate is one scalar, dg is a whole-wave sum, and every access of dout, the table, dn and dtable is 4 or 8
- * contiguous bytes per lane, 256 or 512 contiguous bytes per instruction. */
+ * contiguous bytes per lane, 256 or 512 contiguous bytes per instruction. A position is a chain of loads (its row's
+ * number, then the row, then at a run's end the row of dtable: 2.4 us a position). So 64 positions' numbers and tokens
+ * are read at once, one a lane, and a position's rows are loaded before the arithmetic of the one before it, into a
+ * second register set (the loop alternates two by name). H = 6, tokens of a log-uniform
+ * vocabulary: 4,096 rows 34 -> 16 us, 20,000 65 -> 39, 65,536 100 -> 98 (its bytes take 84). */
 template <int H>
 __global__ void __launch_bounds__(VE_THREADS) ve_backward_kernel(VeBwd a) {
     constexpr int C = H * HEAD_DIM;
     __shared__ __attribute__((aligned(16))) float ws[H * C];
-    stage_w_rows<H>(ws, a.w);
-    __syncthreads();
     const int lane = threadIdx.x & (WAVE - 1);
     const long long nw = (long long)gridDim.x * VE_WAVES;
     const long long wid = uniform64((long long)blockIdx.x * VE_WAVES + (threadIdx.x >> 6));
     const long long p0 = a.rows * wid / nw, p1 = a.rows * (wid + 1) / nw;
-    float acc[H][2];
-    uint32_t eb[H];   /* the run's table columns as bf16x2 */
-    int cur = -1;
-    bool cur_ok = false, started = false, shared = false;   /* shared: the current run began in the wave before */
-    const int before = p0 > 0 && p0 < p1 ? __builtin_amdgcn_readfirstlane(a.ids[p0 - 1]) : 0;
-    const int after = p1 < a.rows && p0 < p1 ? __builtin_amdgcn_readfirstlane(a.ids[p1]) : 0;
-    for (long long p = p0; p < p1; p++) {
-        const long long r = uniform64(a.order[p]);
-        if (r < 0 || r >= a.rows) continue;   /* not a row: nothing to read or write */
-        const int t = __builtin_amdgcn_readfirstlane(a.ids[p]);
-        const Rsrc rd = row_rsrc(a.dout + r * a.dout_stride, C * 2);
-        uint32_t d[H];
-        float g[H];
-#pragma unroll
-        for (int k = 0; k < H; k++) {
-            d[k] = __builtin_amdgcn_raw_buffer_load_b32(rd, (k * HEAD_DIM + 2 * lane) * 2, 0, 2);
-            g[k] = a.gate[r * H + k];
+    const bool has_before = p0 > 0 && p0 < p1, has_after = p1 < a.rows && p0 < p1;
+    const int before = has_before ? __builtin_amdgcn_readfirstlane(a.ids[p0 - 1]) : 0;
+    const int after = has_after ? __builtin_amdgcn_readfirstlane(a.ids[p1]) : 0;
+    VeRun<H> run;
+    run.started = run.ok = run.shared = false;
+    run.t = -1;
+    bool staged = false;
+    for (long long base = p0; base < p1 || !staged; base += WAVE) {
+        VePositions ps;
+        ps.n = base < p1 ? (int)(p1 - base < WAVE ? p1 - base : WAVE) : 0;
+        const unsigned long long row = lane < ps.n ? (unsigned long long)a.order[base + lane] : ~0ull;
+        ps.row_lo = (uint32_t)row;
+        ps.row_hi = (uint32_t)(row >> 32);
+        ps.id = lane < ps.n ? a.ids[base + lane] : -1;
+        VeRow<H> x, y;
+        ve_fetch<H>(a, ps, 0, has_before, before, run.started, run.t, lane, x);
+        if (!staged) {   /* w, behind the first row's loads; every wave comes here once */
+            stage_w_rows<H>(ws, a.w);
+            __syncthreads();
+            staged = true;
         }
-        if (!started || t != cur) {
-            if (started && cur_ok) flush_run<H>(a.dtable, cur, acc, lane, shared);
-            shared = !started && p0 > 0 && t == before;
-            started = true;
-            cur = t;
-            cur_ok = t >= 0 && (long long)t < a.vocab;
-            const Rsrc re = row_rsrc(a.table + (cur_ok ? (long long)t * C : 0), cur_ok ? C * 4 : 0);
-#pragma unroll
-            for (int k = 0; k < H; k++) {
-                const auto e = __builtin_amdgcn_raw_buffer_load_b64(re, (k * HEAD_DIM + 2 * lane) * 4, 0, 0);
-                eb[k] = (uint32_t)f32_to_bf16(__uint_as_float(e[0])) | ((uint32_t)f32_to_bf16(__uint_as_float(e[1])) << 16);
-                acc[k][0] = 0.0f;
-                acc[k][1] = 0.0f;
-            }
-        }
-        float dz[H], mine = 0.0f;
-#pragma unroll
-        for (int k = 0; k < H; k++) {
-            const float d0 = __uint_as_float(d[k] << 16), d1 = __uint_as_float(d[k] & 0xFFFF0000u);
-            const float e0 = __uint_as_float(eb[k] << 16), e1 = __uint_as_float(eb[k] & 0xFFFF0000u);
-            acc[k][0] = acc[k][0] + bf16r(g[k] * d0);
-            acc[k][1] = acc[k][1] + bf16r(g[k] * d1);
-            const float dg = wave_sum(__builtin_fmaf(d1, e1, d0 * e0)), sg = g[k] * 0.5f;
-            dz[k] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(2.0f * dg * (1.0f - sg) * sg)));
-            if (lane == k) mine = dz[k];
-        }
-        __builtin_amdgcn_raw_buffer_store_b16(f32_to_bf16(mine), row_rsrc(a.dz + r * H, H * 2), lane * 2, 0, 0);
-        const Rsrc rn = row_rsrc(a.dn + r * C, C * 2);
-        /* dn one head's columns at a time (a loop, so w's LDS reads are not all hoisted into registers) */
-#pragma unroll 1
-        for (int k = 0; k < H; k++) {
-            float x0 = 0.0f, x1 = 0.0f;
-#pragma unroll
-            for (int h = 0; h < H; h++) {
-                const float2 wv = *reinterpret_cast<const float2 *>(ws + h * C + k * HEAD_DIM + 2 * lane);
-                x0 = __builtin_fmaf(dz[h], wv.x, x0);
-                x1 = __builtin_fmaf(dz[h], wv.y, x1);
-            }
-            __builtin_amdgcn_raw_buffer_store_b32((uint32_t)f32_to_bf16(x0) | ((uint32_t)f32_to_bf16(x1) << 16), rn,
-                                                  (k * HEAD_DIM + 2 * lane) * 2, 0, 0);
+        for (int q = 0; q < ps.n; q += 2) {
+            ve_fetch<H>(a, ps, q + 1, has_before, before, run.started || x.valid, x.valid ? x.t : run.t, lane, y);
+            ve_row<H>(a, ws, x, run, lane);
+            if (q + 1 >= ps.n) break;
+            ve_fetch<H>(a, ps, q + 2, has_before, before, run.started || y.valid, y.valid ? y.t : run.t, lane, x);
+            ve_row<H>(a, ws, y, run, lane);
         }
     }
-    if (started && cur_ok) flush_run<H>(a.dtable, cur, acc, lane, shared || (p1 < a.rows && cur == after));
+    if (run.started && run.ok)
+        flush_run<H>(a.dtable, run.t, run.acc, run.old, lane, run.shared || (has_after && run.t == after));
 }
 
 /* The gate weight's gradient dw[h][c] = sum over rows of dz[row][h] n[row][c] (bf16 operands, fp32 sums): H <= 16
  * outputs a column, so it is bound by reading n once, not by the products, and a matrix product's tiles (H of 16 rows
  * used, a few column tiles for the whole sum over the rows) leave the chip idle. A block takes a slab of rows and 256
  * columns, a lane four columns of all H heads; 64 rows at a time, 16 a wave, dz through LDS. The waves' and then the
- * slabs' sums are added in a fixed order. 65,536 rows, H = 6: VEW_FIGURES */
+ * slabs' sums are added in a fixed order. 65,536 rows, H = 6: 143 -> 40 us (2.5 TB/s of n) */
 struct VeWeight {
     const uint16_t *dz;   /* [rows][H] bf16 */
     const uint16_t *n;    /* [rows][C] bf16 */
@@ -440,10 +519,10 @@ int launch_weight(int heads, const VeWeight &a, int slabs, float *dw, hipStream_
     }
 }
 
-/* Workgroups for `rows` rows: every row a wave, at most as many workgroups as the device holds at once (the
+/* Workgroups for `rows` rows: `per` rows a wave, at most as many workgroups as the device holds at once (the
  * kernel's resident workgroups per device, cached per device in `resident`). */
 template <typename K>
-int ve_blocks(K kernel, long long rows, int (&resident)[64]) {
+int ve_blocks(K kernel, long long rows, int per, int (&resident)[64]) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return -1;
     if (!resident[dev]) {
@@ -453,14 +532,14 @@ int ve_blocks(K kernel, long long rows, int (&resident)[64]) {
             return -1;
         resident[dev] = max(1, cus) * max(1, per_cu);
     }
-    const long long need = (rows + VE_WAVES - 1) / VE_WAVES;
+    const long long need = (rows + VE_WAVES * per - 1) / (VE_WAVES * per);
     return (int)max(1LL, min(need, (long long)resident[dev]));
 }
 
 template <int H>
 int launch_forward(const VeFwd &a, hipStream_t stream) {
     static int resident[64] = {0};
-    const int blocks = ve_blocks(ve_forward_kernel<H>, a.rows, resident);
+    const int blocks = ve_blocks(ve_forward_kernel<H>, a.rows, 1, resident);
     if (blocks < 0) return (int)hipErrorInvalidDevice;
     hipLaunchKernelGGL(ve_forward_kernel<H>, dim3(blocks), dim3(VE_THREADS), 0, stream, a);
     return (int)hipGetLastError();
@@ -469,7 +548,11 @@ int launch_forward(const VeFwd &a, hipStream_t stream) {
 template <int H>
 int launch_backward(const VeBwd &a, hipStream_t stream) {
     static int resident[64] = {0};
-    const int blocks = ve_blocks(ve_backward_kernel<H>, a.rows, resident);
+    /* Rows a wave: a frequent token's rows all add into one row of dtable, a wave at a time, so more waves mean more
+     * adds at the same addresses; fewer leave the chip idle (H = 6, one / two / four rows a wave: 1,024 rows 10 / 9 / 13
+     * us, 2,048 16 / 13 / 14, 4,096 19 / 19 / 16; from 8,192 the same). */
+    const int per = (int)max(1LL, min(4LL, a.rows / 1024));
+    const int blocks = ve_blocks(ve_backward_kernel<H>, a.rows, per, resident);
     if (blocks < 0) return (int)hipErrorInvalidDevice;
     hipLaunchKernelGGL(ve_backward_kernel<H>, dim3(blocks), dim3(VE_THREADS), 0, stream, a);
     return (int)hipGetLastError();

@@ -619,20 +619,32 @@ __global__ void __launch_bounds__(FA_THREADS, 2) flash_bwd_dq_kernel(FlashBwd a)
     }
 }
 
-/* D[row][h] = sum_d dO . O in fp32: one wave per (row, head), two dims per lane. */
+/* D[row][h] = sum_d dO . O in fp32, bound by HBM (512 bytes a row): 16 lanes a (row, head), eight consecutive dims a lane by
+ * 16-byte loads (4-byte aligned; the one-wave-a-row form's 4 bytes a lane took 62 us at 65,536 tokens of 6 heads, this 31), the lanes' sums by the
+ * fixed butterfly. */
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+
 __global__ void __launch_bounds__(256) flash_bwd_rows_kernel(const uint16_t *out, long long o_stride,
                                                              const uint16_t *dout, long long do_stride, long long n,
                                                              int H, float *dpsum) {
-    const long long w = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (w >= n) return;
-    const int lane = threadIdx.x & (WAVE - 1), h = (int)(w % H);
-    const long long row = w / H;
-    const uint32_t o = *reinterpret_cast<const uint32_t *>(out + row * o_stride + (long long)h * HEAD_DIM + 2 * lane);
-    const uint32_t d = *reinterpret_cast<const uint32_t *>(dout + row * do_stride + (long long)h * HEAD_DIM + 2 * lane);
-    const float v = __builtin_fmaf(__uint_as_float(o & 0xFFFF0000u), __uint_as_float(d & 0xFFFF0000u),
-                                   __uint_as_float(o << 16) * __uint_as_float(d << 16));
-    const float sum = wave_sum_butterfly(v);
-    if (lane == 0) dpsum[w] = sum;
+    const long long w = (long long)blockIdx.x * 16 + (threadIdx.x >> 4);
+    if (w >= n) return;   /* whole 16-lane groups */
+    const int i = threadIdx.x & 15;
+    const long long row = n < (1LL << 31) ? (long long)((unsigned)w / (unsigned)H) : w / H;
+    const int h = (int)(w - row * H);
+    const u32x4_a4 o = *reinterpret_cast<const u32x4_a4 *>(out + row * o_stride + (long long)h * HEAD_DIM + 8 * i);
+    const u32x4_a4 d = *reinterpret_cast<const u32x4_a4 *>(dout + row * do_stride + (long long)h * HEAD_DIM + 8 * i);
+    float v = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        v = __builtin_fmaf(__uint_as_float(o[k] << 16), __uint_as_float(d[k] << 16), v);
+        v = __builtin_fmaf(__uint_as_float(o[k] & 0xFFFF0000u), __uint_as_float(d[k] & 0xFFFF0000u), v);
+    }
+    v = v + lane_xor_dpp<8>(v);
+    v = v + lane_xor_dpp<4>(v);
+    v = v + lane_xor_dpp<2>(v);
+    v = v + lane_xor_dpp<1>(v);
+    if (i == 0) dpsum[w] = v;
 }
 
 }  // namespace
@@ -675,7 +687,7 @@ extern "C" int nc_flash_attn_bwd_rows(const void *out, long long o_stride, const
     if (!out || !dout || !dpsum) return NC_ERR_NULL;
     if (((uintptr_t)out | (uintptr_t)dout) & 3) return NC_ERR_SHAPE;
     const long long n = total * heads;
-    hipLaunchKernelGGL(flash_bwd_rows_kernel, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, (hipStream_t)stream,
+    hipLaunchKernelGGL(flash_bwd_rows_kernel, dim3((unsigned)((n + 15) / 16)), dim3(256), 0, (hipStream_t)stream,
                        (const uint16_t *)out, o_stride, (const uint16_t *)dout, do_stride, n, heads, dpsum);
     return (int)hipGetLastError();
 }

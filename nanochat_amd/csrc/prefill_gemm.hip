@@ -111,7 +111,8 @@ __device__ __forceinline__ void pg_barrier() {
  * cannot tell a read of one stage buffer from the DMA into the others, and with builtin reads it waited for most DMA
  * in flight before each stage's first read, which left one stage in flight instead of three. A read's result is used
  * only after the s_waitcnt lgkmcnt(0) at the head of the next ring position (pg_wait_stage), and the MFMAs, being
- * volatile too, stay after that wait.
+ * volatile too, stay after that wait. The compiler takes a read's registers as written at once, so they must not be free
+ * before that wait either: every read is used after it, the last stage's by the empty statements behind the K walk.
  *
  * The compiler does not see the MFMAs as matrix instructions, so it inserts none of their wait states; the kernel
  * keeps their hazards by construction. Operands are written only by LDS reads, waited for as above, never by VALU
@@ -204,6 +205,14 @@ __device__ __forceinline__ void pg_run(const PfGemm &g, int m0, int n0, unsigned
         PG_STEP(j + 2, b2, b3, 0, 1);
         PG_STEP(j + 3, b3, b0, 1, 0);
     }
+    /* The last stage's reads of the stage past it (into set 0) are in flight and used by nothing: their registers stay
+     * taken until they have landed, or the compiler would put the epilogue's first values there and the reads would land
+     * on them (tests/test_projection_gemm_isa.py). */
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int t = 0; t < P::NT; t++) asm volatile("" : "+v"(fw[0][t]));
+#pragma unroll
+    for (int u = 0; u < P::NU; u++) asm volatile("" : "+v"(fa[0][u]));
     __builtin_amdgcn_s_waitcnt(0);                 /* no DMA may land in LDS after this */
     /* 32 wait states: every product has written its accumulator before the epilogue reads it (each accumulator is
      * tied to this point, so no read moves above it) */

@@ -17,9 +17,9 @@
  * position.
  *
  * Workgroups take their tiles in an XCD-aware order (pg_order), so the workgroups an XCD runs together share operand
- * tiles in its L2. The tiles that would leave the last round of workgroups part-filled (T mod CUs of T tiles) are cut
- * into halves (256 x 128) or quarters (128 x 128), so that round has a workgroup on every CU and each takes in half or
- * a quarter of the operands; the waves of a smaller tile hold fewer fragments (PgTile).
+ * tiles in its L2. The tiles that would leave the last (or only) round of workgroups part-filled (T mod CUs of T tiles) are
+ * cut into halves (256 x 128) or quarters (128 x 128), so that round has a workgroup on more of the CUs and each takes in
+ * half or a quarter of the operands; the waves of a smaller tile hold fewer fragments (PgTile).
  *
  * Every output's sum runs over K in one fixed order (the stages in order, each stage one MFMA's own order), whatever M
  * is and whatever size of tile holds it, so a row's result depends on its own a row alone: a prompt's rows give the
@@ -61,7 +61,7 @@ struct PgTile {
 typedef PgTile<256, 256> PgFull;
 typedef PgTile<256, 128> PgHalf;
 typedef PgTile<128, 128> PgQuarter;
-typedef PgTile<128, 256> PgThin;   /* calls of M <= 128 rows (a decode step's slots) */
+typedef PgTile<128, 256> PgThin;   /* calls of M <= 128 rows (a decode step's slots) and many columns */
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -321,7 +321,8 @@ __device__ __forceinline__ int2 pg_band(int id, int T, int nx) {
 /* Workgroups [0, full) take whole tiles 0 .. full - 1; the rest take pieces (2: halves by n, 4: quarters) of tiles
  * full .. T - 1, the pieces of a tile on consecutive items of one XCD. A piece past M or N has nothing to compute.
  * Launches with no pieces use the instantiation without them (MODE PG_WHOLE): the same whole-tile loop ran 3-6 %
- * slower in a kernel that also holds the pieces' code. Calls of M <= 128 rows take tiles of 128 rows (PG_THIN). */
+ * slower in a kernel that also holds the pieces' code. Calls of M <= 128 rows and many columns take 128 x 256 tiles
+ * (PG_THIN). */
 enum { PG_WHOLE, PG_SPLIT, PG_THIN };
 
 template <int EPI, int MODE>
@@ -406,13 +407,17 @@ int prefill_gemm(const PfGemm &g, int epi, hipStream_t stream) {
         (epi != SG_STORE && epi != SG_RESID && epi != SG_RESID2 && epi != SG_F32 && epi != SG_RELU2))
         return NC_ERR_SHAPE;
     /* T tiles in rounds of one workgroup a CU: the R = T mod CUs tiles of a last part-filled round are cut into 4
-     * (R <= CUs / 4) or 2 (R <= CUs / 2) pieces when there are earlier full rounds; otherwise every tile is whole. */
-    const int cus = device_cus(), T = ((g.N + 255) / 256) * ((g.M + 255) / 256), R = T % cus;
-    const bool cut = g.M > 128 && T > cus && R > 0;
-    const int pieces = cut && 4 * R <= cus ? 4 : cut && 2 * R <= cus ? 2 : 1;
+     * (R <= CUs / 4) or 2 (R <= CUs / 2) pieces; more would need a second round of pieces, which costs more than it saves
+     * (a stage takes a quarter 0.31 us, a half 0.53, a whole tile 0.73). The round may be the only one: a prompt of a few
+     * thousand tokens makes fewer tiles than CUs, and its GEMM then lasts as long as one tile (M = 1,500, N x K = 768 x
+     * 3,072: 18 whole tiles 71 us, 72 quarters 31 us; M = 6,594, 78 tiles 73 us, 156 halves 51 us). Calls of M <= 128
+     * rows (a decode step's slots) take quarters as long as their (N / 128) column tiles fit the CUs, else 128 x 256. */
+    const int cus = device_cus(), nx = (g.N + 255) / 256, T = nx * ((g.M + 255) / 256), R = T % cus;
+    const bool one = g.M <= 128, thin = one && 2 * nx > cus;
+    const int pieces = thin || R == 0 ? 1 : one || 4 * R <= cus ? 4 : 2 * R <= cus ? 2 : 1;
     const int full = pieces > 1 ? T - R : T;
     const dim3 grid(full + (T - full) * pieces), block(PG_WAVES * WAVE);
-    const int mode = g.M <= 128 ? PG_THIN : pieces > 1 ? PG_SPLIT : PG_WHOLE;
+    const int mode = thin ? PG_THIN : pieces > 1 ? PG_SPLIT : PG_WHOLE;
 #define PG_LAUNCH_MODES(KERNEL)                                                                          \
     do {                                                                                                   \
         if (mode == PG_THIN) hipLaunchKernelGGL((KERNEL(PG_THIN)), grid, block, 0, stream, g, full, pieces);        \

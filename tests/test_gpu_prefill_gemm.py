@@ -91,3 +91,20 @@ def test_split_tiles_match_whole_tiles(device, N, K, M, epi):
         r1 = min(M, r0 + 256)
         part = run(epi, w, a[r0:r1].contiguous(), rstd=rstd[r0:r1].contiguous())
         assert torch.equal(full[r0:r1].view(bits), part.view(bits)), (r0, r1)
+
+
+@pytest.mark.parametrize("N,K,M", [(768, 768, 1), (768, 256, 128), (32772, 128, 100), (33000, 128, 128), (2304, 256, 129),
+                                   (768, 1024, 1500), (4992, 128, 1000), (4992, 256, 1290), (768, 128, 16500)])
+def test_part_filled_single_round_matches_whole_rows(device, N, K, M):
+    """Calls with fewer tiles than CUs: quarters, halves and (M <= 128) quarters or 128 x 256 tiles by their column
+    count. fp32 sums within fp32 accumulation error of float64, and each row's bits those it has alone."""
+    gen = torch.Generator().manual_seed(N + M)
+    w = torch.randn(N, K, generator=gen).bfloat16().to(device)
+    a = torch.randn(M, K, generator=gen).bfloat16().to(device)
+    got = run(F32, w, a)
+    rows = sorted({0, M // 2, M - 1})
+    want = a[rows].double().cpu() @ w.double().cpu().t()
+    mag = a[rows].double().abs().cpu() @ w.double().abs().cpu().t()
+    assert bool(((got[rows].double().cpu() - want).abs() <= K * 2.0 ** -23 * mag).all())
+    for r in rows:
+        assert torch.equal(run(F32, w, a[r:r + 1].contiguous())[0], got[r])

@@ -15,7 +15,7 @@
  * rstd_kernel). Prefill's GEMMs (up to 16,384 rows a call) are prefill_gemm.hip's MFMA-tiled kernel over all the
  * call's rows at once, with the epilogue fused (bf16 out, the residual, ReLU^2 with the rstd); each row's sums run in
  * one fixed order, so they do not depend on how many rows the call holds. The o GEMM's residual sum needs its whole
- * row for the MLP's rstd, so it writes fp32 and rstd_kernel adds the residual. Every kernel covers the slots up to
+ * row for the MLP's rstd, so it also writes each 32 columns' sum of squares, which tile_rstd adds. Every kernel covers the slots up to
  * the highest active one (dec_set_active) and skips inactive slots.
  *
  * Numerics, op by op as decode.cu: the epilogues round once (bf16(s + residual)); the MLP reads the un-normed stream
@@ -204,12 +204,11 @@ __global__ void __launch_bounds__(256) norm_kernel(NormArgs a) {
     }
 }
 
-/* The MLP's rstd of o_proj's fp32 residual sum (decode.cu:149-154, 445-456), a wave per row: x = s + xm when xm is
- * given (then xo = bf16(x) is written here), else x = s (the GEMM wrote xo and x); rstd = 1 / sqrt(sum x^2 (1 / C)
- * + FLT_EPSILON). */
+/* The MLP's rstd of a step's fp32 residual sum x = s (decode.cu:149-154, 445-456; the o GEMM wrote its rounding), a wave
+ * per row: rstd = 1 / sqrt(sum x^2 (1 / C) + FLT_EPSILON). */
 template <int NJ>
-__global__ void __launch_bounds__(256) rstd_kernel(const float *s, const uint16_t *xm, uint16_t *xo, float *rstd,
-                                                   const unsigned long long *active, int rows, int C) {
+__global__ void __launch_bounds__(256) rstd_kernel(const float *s, float *rstd, const unsigned long long *active, int rows,
+                                                   int C) {
     const int lane = threadIdx.x & (WAVE - 1);
     const int b = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (b >= rows || (active && !live(active, b))) return;
@@ -220,23 +219,13 @@ __global__ void __launch_bounds__(256) rstd_kernel(const float *s, const uint16_
         const int i = j * ROW_CHUNK + lane * 8;
 #pragma unroll
         for (int e = 0; e < 8; e++) x[j][e] = 0.0f;
-        if (i >= C) continue;
-        load8(s + row + i, x[j]);
-        if (xm) {
-            float m[8];
-            load8(xm + row + i, m);
-#pragma unroll
-            for (int e = 0; e < 8; e++) x[j][e] = x[j][e] + m[e];
-        }
+        if (i < C) load8(s + row + i, x[j]);
     }
     float ss = 0.0f;
 #pragma unroll
-    for (int j = 0; j < NJ; j++) {
-        const int i = j * ROW_CHUNK + lane * 8;
-        if (xm && i < C) store8(xo + row + i, x[j]);
+    for (int j = 0; j < NJ; j++)
 #pragma unroll
         for (int e = 0; e < 8; e++) ss = __builtin_fmaf(x[j][e], x[j][e], ss);
-    }
     ss = wave_sum_butterfly(ss);
     if (lane == 0) rstd[b] = 1.0f / __builtin_sqrtf(ss * (1.0f / (float)C) + FLT_EPS);
 }
@@ -759,6 +748,18 @@ static Acts acts_from(const Decoder *d, const Acts &a, size_t b0) {
     return r;
 }
 
+/* A prefill's o GEMM: xo = bf16(in . W^T + resid) and, from each 32 columns' sum of squares of the fp32 sum (ssq), the
+ * rows' rstd for fc. With the fp32 sum written out and a pass over it for the residual and the rstd, 6,594 rows of 768
+ * took 21 + 8 us, this 24 + 5; 16,384 rows of 1,664 write 109 MB less a layer (8 layers: 12.84 -> 12.60 ms a prefill). */
+static void o_gemm(const Lane &ln, const uint16_t *w, int C, const uint16_t *in, int n, uint16_t *xo,
+                   const uint16_t *resid, float *ssq, float *rstd) {
+    if (n <= 0) return;
+    if (n > PREFILL_ROWS) die("o_gemm", "more rows than the prefill buffers hold", __LINE__);
+    PfGemm g = {in, w, n, C, C, xo, nullptr, resid, nullptr, ssq};
+    NC_CHECK(prefill_gemm(g, SG_RESID2, ln.stream));
+    HIP_CHECK((hipError_t)tile_rstd(ssq, n, C, rstd, ln.stream));
+}
+
 /* A prefill GEMM (prefill_gemm.hip) over all n rows of the call: out[r][rows] = epilogue(in[r][cols] . W[rows][cols]^T),
  * each row's sums in one fixed order whatever n is, so a row's result does not depend on how many rows share the call.
  * epi: SG_STORE (bf16), SG_RESID (bf16(s + resid)), SG_F32 (fp32) or SG_RELU2 (bf16(relu(p) p), p = s rstd[r]). */
@@ -767,7 +768,7 @@ static void gemm(const Lane &ln, const uint16_t *w, int rows, int cols, const ui
     if (n <= 0) return;
     if (n > PREFILL_ROWS) die("gemm", "more rows than the prefill buffers hold", __LINE__);
     PfGemm g = {in, w, n, rows, cols, epi == SG_F32 ? nullptr : (uint16_t *)out, epi == SG_F32 ? (float *)out : nullptr,
-                resid, rstd};
+                resid, rstd, nullptr};
     NC_CHECK(prefill_gemm(g, epi, ln.stream));
 }
 
@@ -795,16 +796,13 @@ static void launch_norm(const Lane &ln, const NormArgs &n) {
     else hipLaunchKernelGGL(norm_kernel<8>, grid, block, 0, ln.stream, n);
 }
 
-static void launch_rstd(Decoder *d, const Lane &ln, const float *s, const uint16_t *xm, uint16_t *xo, float *rstd,
-                        const unsigned long long *active, int rows) {
+static void launch_rstd(Decoder *d, const Lane &ln, const float *s, float *rstd, const unsigned long long *active,
+                        int rows) {
     const dim3 grid((rows + 3) / 4), block(256);
     const int C = d->C;
-    if (C <= 2 * ROW_CHUNK)
-        hipLaunchKernelGGL(rstd_kernel<2>, grid, block, 0, ln.stream, s, xm, xo, rstd, active, rows, C);
-    else if (C <= 4 * ROW_CHUNK)
-        hipLaunchKernelGGL(rstd_kernel<4>, grid, block, 0, ln.stream, s, xm, xo, rstd, active, rows, C);
-    else
-        hipLaunchKernelGGL(rstd_kernel<8>, grid, block, 0, ln.stream, s, xm, xo, rstd, active, rows, C);
+    if (C <= 2 * ROW_CHUNK) hipLaunchKernelGGL(rstd_kernel<2>, grid, block, 0, ln.stream, s, rstd, active, rows, C);
+    else if (C <= 4 * ROW_CHUNK) hipLaunchKernelGGL(rstd_kernel<4>, grid, block, 0, ln.stream, s, rstd, active, rows, C);
+    else hipLaunchKernelGGL(rstd_kernel<8>, grid, block, 0, ln.stream, s, rstd, active, rows, C);
 }
 
 static uint8_t *layer_k(Decoder *d, int l) { return d->k_pages + (size_t)l * d->layer_pages * d->H * PAGE_BYTES; }
@@ -813,8 +811,7 @@ static float *layer_s(Decoder *d, int l) { return d->kv_scale + (size_t)l * d->l
 
 /* A GEMM with its epilogue. A decode step (step): slot_gemm over the slots in blocks of SG_MAX_N, each slot's sums in
  * the same order whatever the block holds, so a slot's result does not depend on the others; its split-K partials (long
- * K) are reduced in slice order. Prefill rows: prefill_gemm with the epilogue fused, except the o GEMM's residual sum,
- * whose rstd needs the whole row (fp32 out; rstd_kernel adds the residual). */
+ * K) are reduced in slice order. Prefill rows: prefill_gemm with the epilogue fused (their o GEMM: o_gemm). */
 static void gemm_epi(Decoder *d, const Lane &ln, bool step, int epi, const uint16_t *w, int rows, int cols,
                      const uint16_t *in, int n, uint16_t *out, float *out_f32, const uint16_t *res, const float *rstd,
                      const unsigned long long *active, float *ssq = nullptr) {
@@ -837,9 +834,6 @@ static void gemm_epi(Decoder *d, const Lane &ln, bool step, int epi, const uint1
     case SG_STORE: gemm(ln, w, rows, cols, in, n, out, SG_STORE); break;
     case SG_RESID: gemm(ln, w, rows, cols, in, n, out, SG_RESID, res); break;
     case SG_F32: gemm(ln, w, rows, cols, in, n, out_f32, SG_F32); break;
-    case SG_RESID2:  /* fp32 s; the rstd kernel adds the residual and writes out */
-        gemm(ln, w, rows, cols, in, n, out_f32, SG_F32);
-        break;
     case SG_RELU2: gemm(ln, w, rows, cols, in, n, out, SG_RELU2, nullptr, rstd); break;
     }
 }
@@ -875,8 +869,12 @@ static void mlp(Decoder *d, const Lane &ln, bool step, const Layer &ly, const La
         proj_norm(d, ln, ly, next, a, n, active);
         return;
     }
-    gemm_epi(d, ln, step, SG_RESID2, ly.o, C, C, a.att, n, a.xo, a.acc, a.xm, nullptr, active);
-    launch_rstd(d, ln, a.acc, step ? nullptr : a.xm, a.xo, a.rstd, active, n);
+    if (step) {
+        gemm_epi(d, ln, step, SG_RESID2, ly.o, C, C, a.att, n, a.xo, a.acc, a.xm, nullptr, active);
+        launch_rstd(d, ln, a.acc, a.rstd, active, n);
+    } else {
+        o_gemm(ln, ly.o, C, a.att, n, a.xo, a.xm, a.acc, a.rstd);
+    }
     gemm_epi(d, ln, step, SG_RELU2, ly.fc, F, C, a.xo, n, a.u, a.acc, nullptr, a.rstd, active);
     if (step) proj_norm(d, ln, ly, next, a, n, active);
     else gemm_epi(d, ln, step, SG_RESID, ly.proj, C, F, a.u, n, a.x, nullptr, a.xo, nullptr, active);

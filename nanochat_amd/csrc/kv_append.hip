@@ -3,9 +3,8 @@
  * per-(token, KV head) absmax e4m3fn quantizer and the paged store; plus the training-form q/k prologue
  * (the reference's qkp_forward) on the same row math.
  *
- * One wave per (token, head) row: lane l holds the rotation pair (dims l, l + 64), so the rotation is
- * lane-local and the row's sum of squares is one xor butterfly over the wave. The row math (nc_row.h) is
- * shared with the fused decode step, which appends the step's token inside the attention kernel.
+ * Four (token, head) rows a wave, 16 lanes a row. The row math (nc_row.h) gives the
+ * same bits as the fused decode step's, which appends the step's token inside the attention kernel.
  */
 #include "nc_device.h"
 #include "nc_row.h"
@@ -45,14 +44,21 @@ static inline int append_pages_per_seq(int T) { return (T + PAGE - 2) / PAGE + 1
  * The new positions of b are [max(start, 0), start + min(T, num_new[b])), cut at rope_len when FUSED (the rest are
  * skipped, as are all of b's positions on a page past max_pages or whose table entry lies outside the pool). The
  * work-group takes those of them on page k: slots [s_lo, s_hi) of that page. Rows are computed four a wave, 16 lanes
- * a row (nc_row.h's 16-lane form, the same bits as the one-row-a-wave form of the fused decode step).
- * y < Hkv: KV head y. Wave w computes the k rows of slots 4 w .. 4 w + 3 (norm and rotation when FUSED, then the
- * quantizer), then their v rows (the value-embedding mix when given, then the quantizer), and writes the codes into an
- * LDS image of the page in the cache's layout. The work-group then stores the image with one 16-byte store a lane; a
- * K block holds one slot, a V block four (slots 4 g .. 4 g + 3), and a V block holding slots outside [s_lo, s_hi) is
- * stored byte by byte, so the page's other slots keep their bytes. The 16 scales of K and of V go out the same way.
- * y >= Hkv (FUSED only): q head 4 (y - Hkv) + w a wave, four of the page's slots at a time, normed and rotated into
- * q_out. */
+ * a row (nc_row.h's 16-lane form, the same bits as the one-row-a-wave form of the fused
+ * decode step), wave w slots 4 w .. 4 w + 3.
+ * y < Hkv: KV head y. The k rows (norm and rotation when FUSED, then the quantizer) and the v rows (the value-embedding
+ * mix when given, then the quantizer) leave their codes in an LDS image of the page in the cache's layout. The work-group
+ * then stores the image with one 16-byte store a lane; a K block holds one slot, a V block four (slots 4 g .. 4 g + 3),
+ * and a V block holding slots outside [s_lo, s_hi) is stored byte by byte, so the page's other slots keep their bytes.
+ * The 16 scales of K and of V go out the same way.
+ * y >= Hkv (FUSED only): q heads 4 (y - Hkv) .. + 3 of the page's slots, normed and rotated into q_out; a wave reads its
+ * slots' rotation once for the four.
+ * It is bound by the chain each work-group begins with (position, page, rows) more than by HBM: 46 MB in 12.8 us at
+ * 8 x 512 tokens of 16 / 4 heads (13.1 with eight 2-byte accesses a row and lane), 75 MB in 21.8 us at 3 x 1,501 tokens of
+ * 13 / 13 heads (22.4); with value embeddings, 6,594 rows of 6 heads, C = 768, 36 -> 24 us. Four KV heads a work-group, one
+ * chain for all, left too few of them: 17 us, 25 us and 37 us. */
+constexpr int Q_GROUP = 4;   /* q heads a work-group */
+
 template <bool FUSED>
 __global__ void __launch_bounds__(256) append_kernel(AppendArgs a) {
     __shared__ __align__(16) uint8_t img[2][PAGE_BYTES];
@@ -70,31 +76,29 @@ __global__ void __launch_bounds__(256) append_kernel(AppendArgs a) {
     const int s_lo = (int)(max(lo, pg0) - pg0), s_hi = (int)(min(hi, pg0 + PAGE) - pg0);
     if (s_lo >= s_hi) return;
     const long long tok_at = (a.row0 ? (long long)a.row0[b] : (long long)b * a.T) - sp;   /* + position = row */
+    const int slot = 4 * wave + r;
+    const bool live = slot >= s_lo && slot < s_hi;   /* rows of other slots compute a new one and store nothing */
+    const long long p = pg0 + min(max(slot, s_lo), s_hi - 1), tok = tok_at + p;
 
     if (FUSED && (int)blockIdx.y >= a.Hkv) {
-        const int h = 4 * ((int)blockIdx.y - a.Hkv) + wave;
-        if (h >= a.Hq) return;
-        float g[8];
+        const int h0 = Q_GROUP * ((int)blockIdx.y - a.Hkv);
+        const uint16_t *row = a.qkv + tok * a.token_stride + h0 * HEAD_DIM;
+        uint4 raw[Q_GROUP];
+        float g[8], c[4], s[4];
 #pragma unroll
-        for (int j = 0; j < 8; j++) g[j] = a.q_gain[i + 16 * j];
-        for (int s0 = s_lo; s0 < s_hi; s0 += 4) {
-            const int slot = s0 + r;   /* past s_hi: computes the last slot again and stores nothing */
-            const long long p = pg0 + min(slot, s_hi - 1), tok = tok_at + p;
-            const uint16_t *row = a.qkv + tok * a.token_stride + h * HEAD_DIM;
-            float x[8], c[4], sn[4], y[8];
+        for (int j = 0; j < Q_GROUP; j++)
+            if (h0 + j < a.Hq) raw[j] = load_row16(row + j * HEAD_DIM, i);
+        load4_f32(a.cos + p * HALF + 4 * i, c);
+        load4_f32(a.sin + p * HALF + 4 * i, s);
+        load_gain16(a.q_gain, i, g);
+        uint16_t *q = a.q_out + (tok * a.Hq + h0) * HEAD_DIM;
 #pragma unroll
-            for (int j = 0; j < 8; j++) x[j] = bf16_to_f32(row[i + 16 * j]);
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                c[j] = a.cos[p * HALF + i + 16 * j];
-                sn[j] = a.sin[p * HALF + i + 16 * j];
-            }
-            norm_rope_quad(x, g, c, sn, y);
-            if (slot < s_hi) {
-                uint16_t *q = a.q_out + (tok * a.Hq + h) * HEAD_DIM;
-#pragma unroll
-                for (int j = 0; j < 8; j++) q[i + 16 * j] = f32_to_bf16(y[j]);
-            }
+        for (int j = 0; j < Q_GROUP; j++) {
+            if (h0 + j >= a.Hq) break;
+            float x[8], y[8];
+            unpack8(raw[j], x);
+            norm_rope16(x, g, c, s, y);
+            if (live) store_row16(q + j * HEAD_DIM, i, y);
         }
         return;
     }
@@ -106,46 +110,37 @@ __global__ void __launch_bounds__(256) append_kernel(AppendArgs a) {
     if (page < 0 || page >= a.num_pages) return;
     const long long at = (long long)page * a.Hkv + kvh;
 
-    const int slot = 4 * wave + r;
-    const bool live = slot >= s_lo && slot < s_hi;   /* rows of other slots compute a new one and store nothing */
-    const long long p = pg0 + min(max(slot, s_lo), s_hi - 1), tok = tok_at + p;
     const uint16_t *kx = FUSED ? a.qkv + tok * a.token_stride + (a.Hq + kvh) * HEAD_DIM
                                : a.k + tok * a.token_stride + kvh * HEAD_DIM;
     const uint16_t *vx = FUSED ? a.qkv + tok * a.token_stride + (a.Hq + a.Hkv + kvh) * HEAD_DIM
                                : a.v + tok * a.token_stride + kvh * HEAD_DIM;
-    float kr[8], vr[8];
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-        kr[j] = bf16_to_f32(kx[i + 16 * j]);
-        vr[j] = bf16_to_f32(vx[i + 16 * j]);
-    }
+    const uint4 kraw = load_row16(kx, i), vraw = load_row16(vx, i);
+    float x[8];
+    unpack8(kraw, x);
     if (FUSED) {
-        float g[8], c[4], sn[4], y[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++) g[j] = a.k_gain[i + 16 * j];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            c[j] = a.cos[p * HALF + i + 16 * j];
-            sn[j] = a.sin[p * HALF + i + 16 * j];
-        }
-        norm_rope_quad(kr, g, c, sn, y);
-#pragma unroll
-        for (int j = 0; j < 8; j++) kr[j] = bf16_to_f32(f32_to_bf16(y[j]));
+        float g[8], c[4], s[4], y[8];
+        load4_f32(a.cos + p * HALF + 4 * i, c);
+        load4_f32(a.sin + p * HALF + 4 * i, s);
+        load_gain16(a.k_gain, i, g);
+        norm_rope16(x, g, c, s, y);
+        unpack8(pack8(y), x);
     }
-    uint32_t code[8];
-    float scale = quantize_quad(kr, code);
+    uint32_t code[2];
+    float scale = quantize16(x, code);
     if (live) {
-#pragma unroll
-        for (int j = 0; j < 8; j++) img[0][k_page_offset(slot, i + 16 * j)] = (uint8_t)code[j];
+        *reinterpret_cast<uint32_t *>(&img[0][k_page_offset(slot, 4 * i)]) = code[0];
+        *reinterpret_cast<uint32_t *>(&img[0][k_page_offset(slot, HALF + 4 * i)]) = code[1];
         if (i == 0) img_scale[0][slot] = scale;
     }
+    unpack8(vraw, x);
     if (FUSED && a.ve)
-        ve_mix_quad(a.ve_h + tok * a.C, a.ve_gate + (long long)kvh * a.C, a.C,
-                    a.ve + (long long)a.ve_tokens[tok] * a.C + kvh * HEAD_DIM, i, vr);
-    scale = quantize_quad(vr, code);
+        ve_mix16(a.ve_h + tok * a.C, a.ve_gate + (long long)kvh * a.C, a.C,
+                 a.ve + (long long)a.ve_tokens[tok] * a.C + kvh * HEAD_DIM, i, x);
+    scale = quantize16(x, code);
     if (live) {
 #pragma unroll
-        for (int j = 0; j < 8; j++) img[1][v_page_offset(slot, i + 16 * j)] = (uint8_t)code[j];
+        for (int e = 0; e < 8; e++)
+            img[1][v_page_offset(slot, (e < 4 ? 4 * i : HALF + 4 * i) + (e & 3))] = (uint8_t)(code[e >> 2] >> (8 * (e & 3)));
         if (i == 0) img_scale[1][slot] = scale;
     }
     __syncthreads();
@@ -159,13 +154,13 @@ __global__ void __launch_bounds__(256) append_kernel(AppendArgs a) {
     } else if (kind && s_first < s_hi && s_first + s_count > s_lo) {
 #pragma unroll
         for (int e = 0; e < 16; e++) {   /* byte e holds slot s_first + e % 4 */
-            const int s = s_first + (e & 3);
-            if (s >= s_lo && s < s_hi) dst[e] = src[e];
+            const int sl = s_first + (e & 3);
+            if (sl >= s_lo && sl < s_hi) dst[e] = src[e];
         }
     }
     if (t < 2 * PAGE) {
-        const int s = t & (PAGE - 1), kv = t >> 4;
-        if (s >= s_lo && s < s_hi) a.kv_scale[(at * 2 + kv) * PAGE + s] = img_scale[kv][s];
+        const int sl = t & (PAGE - 1), kv = t >> 4;
+        if (sl >= s_lo && sl < s_hi) a.kv_scale[(at * 2 + kv) * PAGE + sl] = img_scale[kv][sl];
     }
 }
 
@@ -173,22 +168,11 @@ __global__ void __launch_bounds__(256) append_kernel(AppendArgs a) {
  * token stride 3 H 128, output contiguous, position p % T for token p.
  *
  * Both directions are bound by HBM (forward: 2 x 256 bytes a row; backward: 3 x 256). 16 lanes take a row (nc_row.h's
- * form of eight consecutive dims a lane), a 16-lane group QK_HEADS heads of one token, so every access is 16 bytes a
- * lane, the rotation is read once for QK_HEADS rows and all of a group's rows are in flight together. Against one row a
- * wave with 2-byte accesses, 65,536 tokens of 6 heads: forward 179 -> 90 us, backward 242 -> 133 us (4.5 TB/s each; a
- * large copy reaches 4.8). */
+ * form), a 16-lane group QK_HEADS heads of one token, so an access is 8 or 16 bytes a lane, the rotation is read once for QK_HEADS rows and all of a group's rows are in flight together. Against one row a
+ * wave with 2-byte accesses, 65,536 tokens of 6 heads: forward 179 -> 87 us (4.6 TB/s), backward 242 -> 115 us (5.2
+ * TB/s); a large copy reaches 4.8. */
 constexpr int QK_HEADS = 3;
 static int qk_head_chunks(int H) { return (H + QK_HEADS - 1) / QK_HEADS; }
-
-/* The rotation of token p's pairs in lane i (see norm_rope_oct): sin is negated in the lanes of the half that `neg`
- * names. */
-__device__ __forceinline__ void load_rotation(const float *cos, const float *sin, long long pos, int i, bool neg,
-                                              float (&c)[8], float (&s)[8]) {
-    load8_f32(cos + pos * HALF + 8 * (i & 7), c);
-    load8_f32(sin + pos * HALF + 8 * (i & 7), s);
-#pragma unroll
-    for (int e = 0; e < 8; e++) s[e] = neg ? -s[e] : s[e];
-}
 
 /* Grid x = 16-token blocks times the head chunks of q then of k (chunk fastest), 256 threads. Indexes fit 32 bits: a row
  * takes 768 bytes of memory or more. */
@@ -202,22 +186,24 @@ __global__ void __launch_bounds__(256) qkp_forward_kernel(const uint16_t *q, con
     if (p >= tokens) return;   /* whole 16-lane groups */
     const bool isq = chunk < chunks;
     const int h0 = (chunk - (isq ? 0 : chunks)) * QK_HEADS;
-    const uint16_t *x = (isq ? q : k) + (p * 3 * H + h0) * HEAD_DIM + 8 * i;
-    uint16_t *y = (isq ? qo : ko) + (p * H + h0) * HEAD_DIM + 8 * i;
+    const uint16_t *x = (isq ? q : k) + (p * 3 * H + h0) * HEAD_DIM;
+    uint16_t *y = (isq ? qo : ko) + (p * H + h0) * HEAD_DIM;
+    const long long tab = (long long)((unsigned)p % (unsigned)T) * HALF + 4 * i;
     uint4 raw[QK_HEADS];
-    float g[8], c[8], s[8];
+    float g[8], c[4], s[4];
 #pragma unroll
     for (int j = 0; j < QK_HEADS; j++)
-        if (h0 + j < H) raw[j] = load8_raw(x + j * HEAD_DIM);
-    load_rotation(cos, sin, (unsigned)p % (unsigned)T, i, i >= 8, c, s);
-    load8_f32((isq ? gq : gk) + 8 * i, g);
+        if (h0 + j < H) raw[j] = load_row16(x + j * HEAD_DIM, i);
+    load4_f32(cos + tab, c);
+    load4_f32(sin + tab, s);
+    load_gain16(isq ? gq : gk, i, g);
 #pragma unroll
     for (int j = 0; j < QK_HEADS; j++) {
         if (h0 + j >= H) break;
         float xr[8], yr[8];
         unpack8(raw[j], xr);
-        norm_rope_oct(xr, g, c, s, yr);
-        store8_bf16(y + j * HEAD_DIM, yr);
+        norm_rope16(xr, g, c, s, yr);
+        store_row16(y + j * HEAD_DIM, i, yr);
     }
 }
 
@@ -241,48 +227,51 @@ __global__ void __launch_bounds__(256) qkp_backward_kernel(const uint16_t *q, co
     uint16_t *dxout = isq ? dq : dk;
     const unsigned chunks = (H + QK_HEADS - 1) / QK_HEADS;
     float g[8], acc[8];
-    load8_f32((isq ? gq : gk) + 8 * i, g);
+    load_gain16(isq ? gq : gk, i, g);
 #pragma unroll
     for (int e = 0; e < 8; e++) acc[e] = 0.0f;
     const unsigned units = (unsigned)(tokens * chunks);
     for (unsigned u = (isq ? blockIdx.x : blockIdx.x - QKB_BLOCKS) * 16 + grp; u < units; u += QKB_GROUPS) {
         const unsigned t = u / chunks;
         const int h0 = (int)(u - t * chunks) * QK_HEADS;
-        const long long at = ((long long)t * 3 * H + h0) * HEAD_DIM + 8 * i, row = ((long long)t * H + h0) * HEAD_DIM + 8 * i;
+        const long long at = ((long long)t * 3 * H + h0) * HEAD_DIM, row = ((long long)t * H + h0) * HEAD_DIM;
+        const long long tab = (long long)(t % (unsigned)T) * HALF + 4 * i;
         uint4 xraw[QK_HEADS], draw[QK_HEADS];
-        float c[8], s[8];
+        float c[4], s[4];
 #pragma unroll
         for (int j = 0; j < QK_HEADS; j++)
             if (h0 + j < H) {
-                xraw[j] = load8_raw(xin + at + j * HEAD_DIM);
-                draw[j] = load8_raw(dyin + row + j * HEAD_DIM);
+                xraw[j] = load_row16(xin + at + j * HEAD_DIM, i);
+                draw[j] = load_row16(dyin + row + j * HEAD_DIM, i);
             }
-        load_rotation(cos, sin, t % (unsigned)T, i, i < 8, c, s);
+        load4_f32(cos + tab, c);
+        load4_f32(sin + tab, s);
 #pragma unroll
         for (int j = 0; j < QK_HEADS; j++) {
             if (h0 + j >= H) break;
-            float xr[8], d[8], n[8], dn[8], part8[8];
-            unpack8(xraw[j], xr);
+            float x[8], d[8], n[8], dn[8], prod[4], dx[8];
+            unpack8(xraw[j], x);
             unpack8(draw[j], d);
-            const float r = rstd_oct(xr);
+            const float r = rstd16(x);
 #pragma unroll
-            for (int e = 0; e < 8; e++) {
-                n[e] = xr[e] * r;
-                const float dm = d[e] * c[e] + lane_xor_dpp<8>(d[e]) * s[e];
-                acc[e] = acc[e] + dm * n[e];
-                dn[e] = dm * g[e];
-                const float w = dn[e] * n[e];
-                part8[e] = w + lane_xor_dpp<8>(w);
+            for (int e = 0; e < 8; e++) n[e] = x[e] * r;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float dm1 = d[e] * c[e] - d[e + 4] * s[e], dm2 = d[e] * s[e] + d[e + 4] * c[e];
+                acc[e] = acc[e] + dm1 * n[e];
+                acc[e + 4] = acc[e + 4] + dm2 * n[e + 4];
+                dn[e] = dm1 * g[e];
+                dn[e + 4] = dm2 * g[e + 4];
+                prod[e] = dn[e] * n[e] + dn[e + 4] * n[e + 4];
             }
-            const float b = oct_row_sum(part8) / 128.0f;
-            float dx[8];
+            const float b = lane16_sum(prod) / 128.0f;
 #pragma unroll
             for (int e = 0; e < 8; e++) dx[e] = r * (dn[e] - n[e] * b);
-            store8_bf16(dxout + at + j * HEAD_DIM, dx);
+            store_row16(dxout + at + j * HEAD_DIM, i, dx);
         }
     }
 #pragma unroll
-    for (int e = 0; e < 8; e++) gpart[grp][8 * i + e] = acc[e];
+    for (int e = 0; e < 8; e++) gpart[grp][(e < 4 ? 0 : HALF) + 4 * i + (e & 3)] = acc[e];
     __syncthreads();
     if (threadIdx.x < HEAD_DIM) {
         float sum = gpart[0][threadIdx.x];
@@ -319,7 +308,7 @@ static int launch_append(AppendArgs a, bool fused, hipStream_t stream) {
     a.pages_per_seq = append_pages_per_seq(a.T);
     const long long x = (long long)a.B * a.pages_per_seq;
     if (x * 256 >= (1LL << 32)) return NC_ERR_SHAPE;
-    const dim3 grid((unsigned)x, (unsigned)(fused ? a.Hkv + (a.Hq + 3) / 4 : a.Hkv));
+    const dim3 grid((unsigned)x, (unsigned)(a.Hkv + (fused ? (a.Hq + Q_GROUP - 1) / Q_GROUP : 0)));
     if (fused)
         hipLaunchKernelGGL(append_kernel<true>, grid, dim3(256), 0, stream, a);
     else

@@ -72,37 +72,39 @@ __device__ __forceinline__ void ve_mix_pair(const uint16_t *h, const float *w, i
     v2 = bf16_to_f32(f32_to_bf16(v2 + g * bf16_to_f32(e[lane + HALF])));
 }
 
-/* The same row math with 16 lanes a row, four rows a wave (the append kernel's form). Lane i of a 16-lane group
- * holds its row's dims i + 16 j, j = 0..7, as x[j]: its rotation pairs (x[j], x[j + 4]) are dims (i + 16 j, i + 16 j
- * + 64), and it stands for lanes l = i + 16 j (j < 4) of the one-row-a-wave form above. That form's butterfly steps 32
- * and 16 pair l with l ^ 32 (j with j ^ 2) and l ^ 16 (j with j ^ 1), so they are lane-local here, and steps 8 .. 1
- * are the same DPP exchanges within the group's 16 lanes: every sum is formed in the same order, and every result
- * has the same bits as the one-row-a-wave form's. All 64 lanes of the wave must call these together. */
-__device__ __forceinline__ float quad_row_sum(const float (&p)[4]) {
-    float v = (p[0] + p[2]) + (p[1] + p[3]);
-    v = v + lane_xor_dpp<8>(v);
-    v = v + lane_xor_dpp<4>(v);
-    v = v + lane_xor_dpp<2>(v);
-    return v + lane_xor_dpp<1>(v);
+/* The same row math with 16 lanes a row, four rows a wave: lane i of a 16-lane group holds dims 4 i .. 4 i + 3 (elements
+ * 0 .. 3) and 64 + 4 i .. 64 + 4 i + 3 (elements 4 .. 7) of its row, so a row moves by two 8-byte accesses a lane and its
+ * rotation pairs (elements j, j + 4) are lane-local. Pair j of lane i stands for lane l = 4 i + j of the one-row-a-wave
+ * form: its butterfly steps 32, 16, 8 and 4 pair lanes i with i ^ 8, i ^ 4, i ^ 2 and i ^ 1, and steps 2 and 1 pair
+ * elements, so every sum is formed in the same order and has the same bits. All 16 lanes of a group must call these
+ * together. (Eight consecutive dims a lane, by 16-byte accesses, spread the order's first steps over eight values a lane
+ * and the pairs over lanes: the append of 8 x 512
+ * tokens took 15 us that way, 12.8 this way.) */
+__device__ __forceinline__ float lane16_sum(float (&d)[4]) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) d[j] = d[j] + lane_xor_dpp<8>(d[j]);
+#pragma unroll
+    for (int j = 0; j < 4; j++) d[j] = d[j] + lane_xor_dpp<4>(d[j]);
+#pragma unroll
+    for (int j = 0; j < 4; j++) d[j] = d[j] + lane_xor_dpp<2>(d[j]);
+#pragma unroll
+    for (int j = 0; j < 4; j++) d[j] = d[j] + lane_xor_dpp<1>(d[j]);
+    return (d[0] + d[2]) + (d[1] + d[3]);
 }
 
-__device__ __forceinline__ float quad_row_max(const float (&m)[4]) {
-    float v = fmaxf(fmaxf(m[0], m[2]), fmaxf(m[1], m[3]));
-    v = fmaxf(v, lane_xor_dpp<8>(v));
-    v = fmaxf(v, lane_xor_dpp<4>(v));
-    v = fmaxf(v, lane_xor_dpp<2>(v));
-    return fmaxf(v, lane_xor_dpp<1>(v));
-}
-
-/* norm_rope_pair in the 16-lane form: g, the gains of the lane's dims; c, s the rotation of its pairs. */
-__device__ __forceinline__ void norm_rope_quad(const float (&x)[8], const float (&g)[8], const float (&c)[4],
-                                               const float (&s)[4], float (&y)[8]) {
+/* 1 / sqrt(mean x^2 + FLT_EPSILON) of the row, as norm_rope_pair's r. */
+__device__ __forceinline__ float rstd16(const float (&x)[8]) {
     float part[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) part[j] = x[j] * x[j] + x[j + 4] * x[j + 4];
-    const float ss = quad_row_sum(part);
-    const float v = ss / 128.0f + FLT_EPS;
-    const float r = 1.0f / __builtin_sqrtf(v);
+    const float v = lane16_sum(part) / 128.0f + FLT_EPS;
+    return 1.0f / __builtin_sqrtf(v);
+}
+
+/* norm_rope_pair in this form. g: the lane's gains; c, s: cos and sin of its four pairs. */
+__device__ __forceinline__ void norm_rope16(const float (&x)[8], const float (&g)[8], const float (&c)[4],
+                                            const float (&s)[4], float (&y)[8]) {
+    const float r = rstd16(x);
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const float n1 = (x[j] * r) * g[j];
@@ -112,82 +114,14 @@ __device__ __forceinline__ void norm_rope_quad(const float (&x)[8], const float 
     }
 }
 
-/* quantize_pair in the 16-lane form: the row's scale, and the lane's eight codes. */
-__device__ __forceinline__ float quantize_quad(const float (&x)[8], uint32_t (&code)[8]) {
-    float m[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) m[j] = fmaxf(fabsf(x[j]), fabsf(x[j + 4]));
-    const float amax = quad_row_max(m);
-    const float scale = amax > 0.0f ? amax / FP8_MAX : 1.0f;
-    const bool fast = scale >= QUANT_FAST_SCALE;
-    const float r = 1.0f / scale;
-#pragma unroll
-    for (int j = 0; j < 8; j++) code[j] = quant_code(x[j], scale, r, fast);
-    return scale;
-}
-
-/* ve_mix_pair in the 16-lane form (i: the lane's index in its group): the lane runs the FMA chains of the four
- * one-row-a-wave lanes it stands for. */
-__device__ __forceinline__ void ve_mix_quad(const uint16_t *h, const float *w, int C, const uint16_t *e, int i,
-                                            float (&v)[8]) {
-    float d[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        d[j] = 0.0f;
-        for (int k = i + 16 * j; k < C; k += WAVE) d[j] = __builtin_fmaf(bf16_to_f32(h[k]), w[k], d[j]);
-    }
-    const float t = quad_row_sum(d);
-    const float g = 2.0f * (1.0f / (1.0f + exp_rn(-t)));
-#pragma unroll
-    for (int j = 0; j < 8; j++) v[j] = bf16_to_f32(f32_to_bf16(v[j] + g * bf16_to_f32(e[i + 16 * j])));
-}
-
-/* The row math a third way: 16 lanes a row, lane i of a 16-lane group holding the eight consecutive dims 8 i .. 8 i + 7,
- * so a row moves by one 16-byte access a lane. Lane i's rotation partners (dim +- 64) are lane i ^ 8's elements of the
- * same index. The element e of lanes i and i ^ 8 stands for lane l = 8 (i % 8) + e of the one-row-a-wave form: its
- * butterfly steps 32, 16 and 8 pair lanes i with i ^ 4, i ^ 2 and i ^ 1, and steps 4, 2 and 1 pair elements, so every
- * sum is formed in the same order and has the same bits. All 16 lanes of a group must call these together. */
-__device__ __forceinline__ float oct_row_sum(float (&p)[8]) {
-#pragma unroll
-    for (int e = 0; e < 8; e++) p[e] = p[e] + lane_xor_dpp<4>(p[e]);
-#pragma unroll
-    for (int e = 0; e < 8; e++) p[e] = p[e] + lane_xor_dpp<2>(p[e]);
-#pragma unroll
-    for (int e = 0; e < 8; e++) p[e] = p[e] + lane_xor_dpp<1>(p[e]);
-    return ((p[0] + p[4]) + (p[2] + p[6])) + ((p[1] + p[5]) + (p[3] + p[7]));
-}
-
-/* 1 / sqrt(mean x^2 + FLT_EPSILON) of the row, as norm_rope_pair's r. */
-__device__ __forceinline__ float rstd_oct(const float (&x)[8]) {
-    float part[8];
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-        const float sq = x[e] * x[e];
-        part[e] = sq + lane_xor_dpp<8>(sq);
-    }
-    const float v = oct_row_sum(part) / 128.0f + FLT_EPS;
-    return 1.0f / __builtin_sqrtf(v);
-}
-
-/* norm_rope_pair in this form. g: the lane's gains; c, s: cos and sin of the lane's pairs, s negated in the upper half's
- * lanes (i >= 8: y = n2 c - n1 s). */
-__device__ __forceinline__ void norm_rope_oct(const float (&x)[8], const float (&g)[8], const float (&c)[8],
-                                              const float (&s)[8], float (&y)[8]) {
-    const float r = rstd_oct(x);
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-        const float n = (x[e] * r) * g[e];
-        y[e] = n * c[e] + lane_xor_dpp<8>(n) * s[e];
-    }
-}
-
-/* Eight consecutive elements by 16-byte accesses at any element alignment (the declared alignment is the element's). */
-typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+/* A lane's elements of a row at any element alignment (the declared alignment is the element's). */
+typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
 typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
-__device__ __forceinline__ uint4 load8_raw(const uint16_t *p) {
-    const u32x4_a2 u = *reinterpret_cast<const u32x4_a2 *>(p);
-    return uint4{u[0], u[1], u[2], u[3]};
+__device__ __forceinline__ uint4 load_row16(const uint16_t *row, int i) {
+    const u32x2_a2 a = *reinterpret_cast<const u32x2_a2 *>(row + 4 * i);
+    const u32x2_a2 b = *reinterpret_cast<const u32x2_a2 *>(row + HALF + 4 * i);
+    return uint4{a[0], a[1], b[0], b[1]};
 }
 
 __device__ __forceinline__ void unpack8(const uint4 &r, float (&x)[8]) {
@@ -199,22 +133,83 @@ __device__ __forceinline__ void unpack8(const uint4 &r, float (&x)[8]) {
     }
 }
 
-__device__ __forceinline__ void load8_f32(const float *p, float (&x)[8]) {
-    const u32x4_a4 a = reinterpret_cast<const u32x4_a4 *>(p)[0], b = reinterpret_cast<const u32x4_a4 *>(p)[1];
+__device__ __forceinline__ void load4_f32(const float *p, float (&x)[4]) {
+    const u32x4_a4 a = *reinterpret_cast<const u32x4_a4 *>(p);
+#pragma unroll
+    for (int k = 0; k < 4; k++) x[k] = __uint_as_float(a[k]);
+}
+
+/* fp32 [128] (a gain) as a lane's elements. */
+__device__ __forceinline__ void load_gain16(const float *g, int i, float (&x)[8]) {
+    float a[4], b[4];
+    load4_f32(g + 4 * i, a);
+    load4_f32(g + HALF + 4 * i, b);
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-        x[k] = __uint_as_float(a[k]);
-        x[4 + k] = __uint_as_float(b[k]);
+        x[k] = a[k];
+        x[4 + k] = b[k];
     }
 }
 
-/* Rounded to bf16 (nearest even, v_cvt_pk_bf16_f32) and stored. */
-__device__ __forceinline__ void store8_bf16(uint16_t *p, const float (&x)[8]) {
+/* Rounded to bf16 (nearest even, v_cvt_pk_bf16_f32), packed. */
+__device__ __forceinline__ uint4 pack8(const float (&x)[8]) {
     bf16x8 v;
 #pragma unroll
     for (int e = 0; e < 8; e++) v[e] = (__bf16)x[e];
-    const uint4 u = __builtin_bit_cast(uint4, v);
-    *reinterpret_cast<u32x4_a2 *>(p) = u32x4_a2{u.x, u.y, u.z, u.w};
+    return __builtin_bit_cast(uint4, v);
+}
+
+__device__ __forceinline__ void store_row16(uint16_t *row, int i, const float (&x)[8]) {
+    const uint4 u = pack8(x);
+    *reinterpret_cast<u32x2_a2 *>(row + 4 * i) = u32x2_a2{u.x, u.y};
+    *reinterpret_cast<u32x2_a2 *>(row + HALF + 4 * i) = u32x2_a2{u.z, u.w};
+}
+
+/* quantize_pair in this form: the row's scale, and the lane's codes of its two runs of four dims, packed. */
+__device__ __forceinline__ float quantize16(const float (&x)[8], uint32_t (&code)[2]) {
+    float m = fabsf(x[0]);
+#pragma unroll
+    for (int e = 1; e < 8; e++) m = fmaxf(m, fabsf(x[e]));
+    m = fmaxf(m, lane_xor_dpp<8>(m));
+    m = fmaxf(m, lane_xor_dpp<4>(m));
+    m = fmaxf(m, lane_xor_dpp<2>(m));
+    const float amax = fmaxf(m, lane_xor_dpp<1>(m));
+    const float scale = amax > 0.0f ? amax / FP8_MAX : 1.0f;
+    const bool fast = scale >= QUANT_FAST_SCALE;
+    const float r = 1.0f / scale;
+    code[0] = code[1] = 0u;
+#pragma unroll
+    for (int e = 0; e < 8; e++) code[e >> 2] |= quant_code(x[e], scale, r, fast) << (8 * (e & 3));
+    return scale;
+}
+
+/* ve_mix_pair in this form: the gate's 64 FMA chains (chain l: elements l, l + 64, ...) run four a lane, lane i chains
+ * 4 i .. 4 i + 3, so h and w move by 8- and 16-byte loads. */
+__device__ __forceinline__ void ve_mix16(const uint16_t *h, const float *w, int C, const uint16_t *e, int i,
+                                         float (&v)[8]) {
+    const uint4 emb = load_row16(e, i);
+    float d[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    const int whole = C / WAVE * WAVE;
+#pragma unroll 4
+    for (int k = 4 * i; k < whole; k += WAVE) {
+        const u32x2_a2 x = *reinterpret_cast<const u32x2_a2 *>(h + k);
+        float y[4];
+        load4_f32(w + k, y);
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            d[j] = __builtin_fmaf(__uint_as_float(j & 1 ? x[j >> 1] & 0xFFFF0000u : x[j >> 1] << 16), y[j], d[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int k = whole + 4 * i + j;
+        if (k < C) d[j] = __builtin_fmaf(bf16_to_f32(h[k]), w[k], d[j]);
+    }
+    const float g = 2.0f * (1.0f / (1.0f + exp_rn(-lane16_sum(d))));
+    float ev[8];
+    unpack8(emb, ev);
+#pragma unroll
+    for (int j = 0; j < 8; j++) v[j] = v[j] + g * ev[j];
+    unpack8(pack8(v), v);
 }
 
 }  // namespace nc

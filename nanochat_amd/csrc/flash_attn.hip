@@ -341,158 +341,215 @@ __device__ __forceinline__ void store4(uint16_t *p, const f32x4 &v, float mul) {
 
 struct alignas(16) DkvStage {
     uint16_t q[FA_BN * HEAD_DIM], dout[FA_BN * HEAD_DIM];   /* k_lds layout; Q^T and dO^T read transposed */
-    float lse2[FA_BN], dd[FA_BN];              /* the block's rows: lse log2(e) (+inf past the segment), D */
+    float nlse[FA_BN], nd[FA_BN];              /* the block's rows: -lse / scale (-inf past the segment), -D */
 };
 
-/* dK, dV of 128 keys: eight waves (two a SIMD) of 16 keys share each staged query block, so a CU takes in half the
- * Q and dO bytes per product that four waves of 16 would. S = Q K^T and dP = dO V^T with queries as rows (a lane holds
- * one key's column), so P and dS feed dV^T += dO^T P and dK^T += Q^T dS directly as B operands, with dO^T and Q^T read
- * from transposed LDS tiles. */
-constexpr int DKV_WAVES = 8;
-constexpr int DKV_KEYS = 16 * DKV_WAVES;
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+__device__ __forceinline__ f32x16 mfma32x32x16(const bf16x8 &a, const bf16x8 &b, const f32x16 &c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+/* A lane's byte offsets into a row-major (k_lds) tile for the A operands of 32 x 32 products; every operand lies at an
+ * offset's xor with a constant, plus a constant, so two registers address them all.
+ * rows_at: the products over the dimension; lane (hf, c) = (lane / 32, lane % 32) holds dims 16 cc + 8 hf .. +7 of row
+ * 32 rt + c. tr_at: the products over 16 rows r0 .. r0 + 15, in the row order of a score tile's registers: lane (hf, c) gets
+ * rows r0 + 4 hf .. + 3, then r0 + 8 + 4 hf .. + 3, of dim 32 dt + c (ds_read_b64_tr_b16 as in tr_operand: a lane points at
+ * row base + (lane % 16) / 4, dims 4 (lane % 4) .. + 3 of its 16). */
+__device__ __forceinline__ uint32_t rows_at(int lane) { return 2 * k_lds(lane & 31, lane >> 5); }
+
+__device__ __forceinline__ uint32_t tr_at(int lane) {
+    const int i = lane & 15, row = 4 * (lane >> 5) + (i >> 2), dim = (lane & 16) + 4 * (i & 3);
+    return 2 * (k_lds(row, dim >> 3) + (dim & 4));
+}
+
+typedef __attribute__((address_space(3))) const unsigned char LdsByte;
+typedef __attribute__((address_space(3))) const bf16x8 LdsOp;
+
+__device__ __forceinline__ bf16x8 rows_operand32(const uint16_t *tile, uint32_t at, int rt, int cc) {
+    return *(LdsOp *)((LdsByte *)tile + (at ^ (cc << 5)) + rt * 32 * HEAD_DIM * 2);
+}
+
+__device__ __forceinline__ bf16x8 tr_operand32(const uint16_t *tile, uint32_t at, int dt, int r0) {
+    LdsByte *p = (LdsByte *)tile + r0 * HEAD_DIM * 2;
+    const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsV4 *)(p + (at ^ (dt << 6))));
+    const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsV4 *)(p + (at ^ (dt << 6) ^ 128) + 8 * HEAD_DIM * 2));
+    const uint2 x = __builtin_bit_cast(uint2, lo), y = __builtin_bit_cast(uint2, hi);
+    return __builtin_bit_cast(bf16x8, uint4{x.x, x.y, y.x, y.y});
+}
+
+/* dK, dV of 128 keys, 32 a wave: S = Q K^T and dP = dO V^T in 32 x 32 tiles with queries as rows (a lane holds one key's
+ * column), so P and dS feed dV^T += dO^T P and dK^T += Q^T dS directly as B operands, with dO^T and Q^T read transposed from
+ * the staged tiles. A wave's 32 columns make every operand read from LDS feed twice the products that 16 x 16 tiles of 16
+ * keys a wave did: those read 64 KiB a wave and block for 64 products, twice the time of the products themselves.
+ * Two blocks of four waves share a CU. At 65,536 tokens of 2,048-token segments x 6 heads dK/dV takes 546 us by trace (16 x 16
+ * tiles in blocks of eight waves: 675), the backward 912 -> 810; at 2 x 8,192 tokens 762 -> 690, at 8 x 2,048 x 10 heads with
+ * a window of 512 232 -> 208. */
+constexpr int DKV_WAVES = 4;
+constexpr int DKV_KEYS = 32 * DKV_WAVES;
+constexpr int DKV_PARKED = 3;   /* K's last operand and V's last two wait in LDS: 256 registers hold the other 13 */
 
 __global__ void __launch_bounds__(64 * DKV_WAVES, 2) flash_bwd_dkv_kernel(FlashBwd a) {
     __shared__ DkvStage s0, s1;   /* distinct objects: a read of one never waits for DMA into the other */
+    __shared__ uint4 parked[DKV_WAVES][DKV_PARKED][WAVE];   /* the operands the registers do not hold */
     const FaBlock fb = fa_block_order();
     const int seg = fb.seg, h = fb.h;
     const long long start = a.cu[seg];
     const int seglen = a.cu[seg + 1] - a.cu[seg];
     const int k0 = fb.rank * DKV_KEYS;          /* the most query blocks first */
     if (seglen <= 0 || k0 >= seglen) return;
-    const int t = threadIdx.x, lane = t & (WAVE - 1), wave = t >> 6, g = lane >> 4, c = lane & 15;
-    const int kw = k0 + wave * 16;              /* the wave's first key */
+    const int t = threadIdx.x, lane = t & (WAVE - 1), hf = lane >> 5, c = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);   /* in a scalar register, as are the bounds made of it */
+    const int kw = k0 + wave * 32;              /* the wave's first key */
     const bool active = kw < seglen;
     const int key = kw + c;
 
-    /* the wave's K and V as B operands: lane (g, c) holds dims 32 cc + 8 g .. +7 of key c */
-    bf16x8 kb_[4], vb_[4];
+    /* the wave's K and V as B operands: lane (hf, c) holds dims 16 cc + 8 hf .. +7 of key c */
+    bf16x8 kb_[8], vb_[8];
     {
-        const int n = active ? min(16, seglen - kw) : 0;
+        const int n = active ? min(32, seglen - kw) : 0;
         const Rsrc rk = rows_rsrc(a.k, start + kw, a.k_stride, h, n), rv = rows_rsrc(a.v, start + kw, a.v_stride, h, n);
 #pragma unroll
-        for (int cc = 0; cc < 4; cc++) {
-            kb_[cc] = __builtin_bit_cast(bf16x8, bload(rk, (int)((c * a.k_stride + cc * 32 + g * 8) * 2)));
-            vb_[cc] = __builtin_bit_cast(bf16x8, bload(rv, (int)((c * a.v_stride + cc * 32 + g * 8) * 2)));
+        for (int cc = 0; cc < 8; cc++) {
+            kb_[cc] = __builtin_bit_cast(bf16x8, bload(rk, (int)((c * a.k_stride + cc * 16 + hf * 8) * 2)));
+            vb_[cc] = __builtin_bit_cast(bf16x8, bload(rv, (int)((c * a.v_stride + cc * 16 + hf * 8) * 2)));
         }
+        parked[wave][0][lane] = __builtin_bit_cast(uint4, kb_[7]);
+        parked[wave][1][lane] = __builtin_bit_cast(uint4, vb_[6]);
+        parked[wave][2][lane] = __builtin_bit_cast(uint4, vb_[7]);
     }
-    f32x4 dk[8], dv[8];
+    const auto unpark = [&](int i) { return __builtin_bit_cast(bf16x8, parked[wave][i][lane]); };
+    f32x16 dk[4], dv[4];
 #pragma unroll
-    for (int d = 0; d < 8; d++) dk[d] = dv[d] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int d = 0; d < 4; d++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) dk[d][i] = dv[d][i] = 0.0f;
 
     const int qhi = a.window >= 0 ? min(seglen - 1, k0 + DKV_KEYS - 1 + a.window) : seglen - 1;
     /* query block qbk + 1 (Q and dO by LDS DMA, the row statistics through registers) is fetched into the other stage
      * while block qbk is computed; the barrier after the compute makes it visible and frees the one just read */
-    float rl = INFINITY, rd = 0.0f;
+    float rl = 0.0f, rd = 0.0f;
+    const float inv_scale = FA_LOG2E / a.scale_log2;
     auto fetch = [&](int qbk, DkvStage &stg) {
         const int qs = qbk * FA_BN, nq = min(FA_BN, seglen - qs);
-        tile_dma<DKV_WAVES>(a.q, start + qs, a.q_stride, h, nq, stg.q, wave, lane);
-        tile_dma<DKV_WAVES>(a.dout, start + qs, a.do_stride, h, nq, stg.dout, wave, lane);
-        if (t < FA_BN) {
-            const bool ok = t < nq;
-            rl = ok ? a.lse[(long long)h * a.lse_stride + start + qs + t] * FA_LOG2E : INFINITY;
-            rd = ok ? a.dpsum[(start + qs + t) * a.H + h] : 0.0f;
+        int ln = lane;
+        asm volatile("" : "+v"(ln));   /* the DMA's addresses are made here, not held across the loop */
+        tile_dma<DKV_WAVES>(a.q, start + qs, a.q_stride, h, nq, stg.q, wave, ln);
+        tile_dma<DKV_WAVES>(a.dout, start + qs, a.do_stride, h, nq, stg.dout, wave, ln);
+        if (wave == 0) {
+            const long long row0 = start + qs;
+            const Rsrc rs = make_rsrc(a.lse + (long long)h * a.lse_stride + row0, (unsigned)nq * 4);
+            const Rsrc rr = make_rsrc(a.dpsum + row0 * a.H + h, (unsigned)((nq - 1) * a.H + 1) * 4);
+            rl = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, ln * 4, 0, 0));
+            rd = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rr, ln * a.H * 4, 0, 0));
         }
     };
-    auto put_stats = [&](DkvStage &stg) {
-        if (t < FA_BN) {
-            stg.lse2[t] = rl;
-            stg.dd[t] = rd;
+    auto put_stats = [&](int qbk, DkvStage &stg) {
+        if (wave == 0) {
+            stg.nlse[lane] = qbk * FA_BN + lane < seglen ? -rl * inv_scale : -INFINITY;
+            stg.nd[lane] = -rd;   /* rows past the segment: 0 */
         }
     };
+    uint32_t rat = rows_at(lane), tat = tr_at(lane);
     auto compute = [&](int qbk, const DkvStage &s) {
         if (!active) return;
         const int qs = qbk * FA_BN;
-        const int kw1 = kw + 15, qe = qs + FA_BN - 1;
-        if (kw > qe || (a.window >= 0 && qs - kw1 > a.window)) return;   /* no row of the block sees the wave's keys */
-        const bool interior = kw1 <= qs && qe < seglen && kw1 < seglen && (a.window < 0 || qe - kw <= a.window);
-        /* the four query tiles' S and dP first (eight independent accumulators, so the products pipeline), then
-         * P and dS, then the dV and dK products of k-step 0 (query tiles 0, 1) and 1 (tiles 2, 3): each dv, dk element
-         * adds k-step 0, then 1 */
-        f32x4 sc[4], dp[4];
 #pragma unroll
-        for (int qt = 0; qt < 4; qt++) sc[qt] = dp[qt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        /* step st = (cc, qt), cc-major; its Q and dO operands are read one step ahead of the products */
-        bf16x8 qn = rows_operand(s.q, 0, 0, g, c), on = rows_operand(s.dout, 0, 0, g, c);
+        for (int qt = 0; qt < 2; qt++) {
+            asm volatile("" : "+v"(rat), "+v"(tat));   /* operand addresses are made here, not held across the loop */
+            const int q0 = qs + 32 * qt, q1 = q0 + 31, kw1 = kw + 31;
+            if (kw > q1 || q0 >= seglen || (a.window >= 0 && q0 - kw1 > a.window)) continue;   /* no row sees the keys */
+            const bool interior = kw1 <= q0 && q1 < seglen && kw1 < seglen && (a.window < 0 || q1 - kw <= a.window);
+            /* the products start from the rows' statistics (rows q0 + 8 j + 4 hf + i in registers 4 j + i): S - lse / scale,
+             * dP - D. The groups keep four operands ahead of their products; two to four measured the same, six 3 % slower,
+             * and the dV and dK products' first operands read ahead of the exponentials spilled 20 registers (+ 20 %). */
+            f32x16 sc, dp;
 #pragma unroll
-        for (int st = 0; st < 16; st++) {
-            const int cc = st >> 2, qt = st & 3;
-            const bf16x8 qo = qn, oo = on;
-            if (st + 1 < 16) {
-                qn = rows_operand(s.q, (st + 1) & 3, (st + 1) >> 2, g, c);
-                on = rows_operand(s.dout, (st + 1) & 3, (st + 1) >> 2, g, c);
+            for (int j = 0; j < 4; j++) {
+                const f32x4 l4 = *reinterpret_cast<const f32x4 *>(&s.nlse[32 * qt + 8 * j + 4 * hf]);
+#pragma unroll
+                for (int i = 0; i < 4; i++) sc[4 * j + i] = l4[i];
             }
-            sc[qt] = mfma16x16x32(qo, kb_[cc], sc[qt]);
-            dp[qt] = mfma16x16x32(oo, vb_[cc], dp[qt]);
-        }
-        /* the row statistics of the lane's 16 rows: one 16-byte LDS read per tile each, all issued together */
-        float4 l2[4], dd[4];
 #pragma unroll
-        for (int qt = 0; qt < 4; qt++) {
-            l2[qt] = *reinterpret_cast<const float4 *>(&s.lse2[qt * 16 + 4 * g]);
-            dd[qt] = *reinterpret_cast<const float4 *>(&s.dd[qt * 16 + 4 * g]);
-        }
-        bf16x8 pb[2], db[2];
-        /* P and dS of the lane's 16 (key, row) pairs; only a block on the diagonal, the window edge or the segment end
-         * tests each pair (interior is uniform over the wave: one scalar branch) */
-        auto stats = [&](bool masked) {
+            for (int cc = 0; cc < 8; cc++)
+                sc = mfma32x32x16(rows_operand32(s.q, rat, qt, cc), cc < 7 ? kb_[cc] : unpark(0), sc);
 #pragma unroll
-            for (int qt = 0; qt < 4; qt++) {
-                /* lane (g, c): key c, query rows qs + 16 qt + 4 g + i */
-                const float lv[4] = {l2[qt].x, l2[qt].y, l2[qt].z, l2[qt].w};
-                const float dv_[4] = {dd[qt].x, dd[qt].y, dd[qt].z, dd[qt].w};
+            for (int j = 0; j < 4; j++) {
+                const f32x4 d4 = *reinterpret_cast<const f32x4 *>(&s.nd[32 * qt + 8 * j + 4 * hf]);
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int r = qt * 16 + 4 * g + i;
-                    const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[qt][i], a.scale_log2, -lv[i]));
-                    const float p = !masked || visible(key, qs + r, seglen, a.window) ? e : 0.0f;
-                    const float ds = p * (dp[qt][i] - dv_[i]);
-                    pb[qt >> 1][(qt & 1) * 4 + i] = (__bf16)p;
-                    db[qt >> 1][(qt & 1) * 4 + i] = (__bf16)ds;
+                for (int i = 0; i < 4; i++) dp[4 * j + i] = d4[i];
+            }
+#pragma unroll
+            for (int cc = 0; cc < 8; cc++)
+                dp = mfma32x32x16(rows_operand32(s.dout, rat, qt, cc), cc < 6 ? vb_[cc] : unpark(cc - 5), dp);
+            __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);   /* S's statistics, four operands */
+#pragma unroll
+            for (int m = 0; m < 16; m++) {   /* product m, then the reads of product m + 4: its row operand, a parked one */
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                if (m == 4) __builtin_amdgcn_sched_group_barrier(0x100, 5, 0);   /* dP's statistics with its first */
+                else if (m == 3 || m == 10 || m == 11) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+                else if (m < 12) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            }
+            bf16x8 pb[2], db[2];
+            /* P and dS of the lane's 16 (key, row) pairs; only a tile on the diagonal, the window edge or the segment end
+             * tests each pair (interior is uniform over the wave: one scalar branch) */
+            auto stats = [&](bool masked) {
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const float e = __builtin_amdgcn_exp2f(sc[4 * j + i] * a.scale_log2);
+                        const float p = !masked || visible(key, q0 + 8 * j + 4 * hf + i, seglen, a.window) ? e : 0.0f;
+                        const float ds = p * dp[4 * j + i];
+                        pb[j >> 1][(j & 1) * 4 + i] = (__bf16)p;
+                        db[j >> 1][(j & 1) * 4 + i] = (__bf16)ds;
+                    }
+            };
+            if (interior)
+                stats(false);
+            else
+                stats(true);
+#pragma unroll
+            for (int s2 = 0; s2 < 2; s2++)
+#pragma unroll
+                for (int d = 0; d < 4; d++) {
+                    dv[d] = mfma32x32x16(tr_operand32(s.dout, tat, d, 32 * qt + 16 * s2), pb[s2], dv[d]);
+                    dk[d] = mfma32x32x16(tr_operand32(s.q, tat, d, 32 * qt + 16 * s2), db[s2], dk[d]);
                 }
-            }
-        };
-        if (interior)
-            stats(false);
-        else
-            stats(true);
-        /* step st = (s2, d); its dO^T and Q^T operands are read one step ahead of the products */
-        bf16x8 vn = tr_operand(s.dout, 0, 0, g, c), kn = tr_operand(s.q, 0, 0, g, c);
+            __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);   /* two steps' operands ahead of their products */
 #pragma unroll
-        for (int st = 0; st < 16; st++) {
-            const int s2 = st >> 3, d = st & 7;
-            const bf16x8 vo = vn, ko = kn;
-            if (st + 1 < 16) {
-                vn = tr_operand(s.dout, (st + 1) & 7, (st + 1) >> 3, g, c);
-                kn = tr_operand(s.q, (st + 1) & 7, (st + 1) >> 3, g, c);
+            for (int st = 0; st < 8; st++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+                if (st < 6) __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
             }
-            dv[d] = mfma16x16x32(vo, pb[s2], dv[d]);
-            dk[d] = mfma16x16x32(ko, db[s2], dk[d]);
         }
     };
     const int qb_lo = k0 / FA_BN, qb_hi = qhi / FA_BN;
     fetch(qb_lo, s0);
-    put_stats(s0);
+    put_stats(qb_lo, s0);
     __syncthreads();
     for (int qbk = qb_lo; qbk <= qb_hi; qbk += 2) {
         if (qbk + 1 <= qb_hi) fetch(qbk + 1, s1);
         compute(qbk, s0);
-        if (qbk + 1 <= qb_hi) put_stats(s1);
+        if (qbk + 1 <= qb_hi) put_stats(qbk + 1, s1);
         __syncthreads();
         if (qbk + 1 > qb_hi) break;
         if (qbk + 2 <= qb_hi) fetch(qbk + 2, s0);
         compute(qbk + 1, s1);
-        if (qbk + 2 <= qb_hi) put_stats(s0);
+        if (qbk + 2 <= qb_hi) put_stats(qbk + 2, s0);
         __syncthreads();
     }
     if (!active || key >= seglen) return;
-    /* dK^T, dV^T tile d: lane (g, c) holds dims 16 d + 4 g .. +3 of key c */
-    uint16_t *pk = a.dk + (start + key) * a.dk_stride + (long long)h * HEAD_DIM + 4 * g;
-    uint16_t *pv = a.dv + (start + key) * a.dv_stride + (long long)h * HEAD_DIM + 4 * g;
+    /* dK^T, dV^T tile d: lane (hf, c) holds dims 32 d + 8 j + 4 hf .. +3 of key c in registers 4 j .. + 3 */
+    uint16_t *pk = a.dk + (start + key) * a.dk_stride + (long long)h * HEAD_DIM + 4 * hf;
+    uint16_t *pv = a.dv + (start + key) * a.dv_stride + (long long)h * HEAD_DIM + 4 * hf;
 #pragma unroll
-    for (int d = 0; d < 8; d++) {
-        store4(pk + d * 16, dk[d], a.scale);
-        store4(pv + d * 16, dv[d], 1.0f);
-    }
+    for (int d = 0; d < 4; d++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            store4(pk + d * 32 + 8 * j, f32x4{dk[d][4 * j], dk[d][4 * j + 1], dk[d][4 * j + 2], dk[d][4 * j + 3]}, a.scale);
+            store4(pv + d * 32 + 8 * j, f32x4{dv[d][4 * j], dv[d][4 * j + 1], dv[d][4 * j + 2], dv[d][4 * j + 3]}, 1.0f);
+        }
 }
 
 struct DqStage {
@@ -718,7 +775,8 @@ extern "C" int nc_flash_attn_bwd(const void *q, const void *k, const void *v, co
     a.q_stride = q_stride; a.k_stride = k_stride; a.v_stride = v_stride; a.do_stride = do_stride;
     a.lse = lse; a.lse_stride = lse_stride; a.dpsum = dpsum;
     a.cu = cu_seqlens; a.segments = segments; a.H = heads; a.window = window < 0 ? -1 : window;
-    a.scale = softmax_scale; a.scale_log2 = softmax_scale * FA_LOG2E;
+    /* dK/dV divides lse by the exponent's scale: kept where that quotient is finite; below, scale S vanishes beside lse */
+    a.scale = softmax_scale; a.scale_log2 = fmaxf(softmax_scale, 0x1p-116f) * FA_LOG2E;
     a.dq = (uint16_t *)dq; a.dk = (uint16_t *)dk; a.dv = (uint16_t *)dv;
     a.dq_stride = dq_stride; a.dk_stride = dk_stride; a.dv_stride = dv_stride;
     hipLaunchKernelGGL(flash_bwd_dkv_kernel, dim3((unsigned)((max_seqlen + DKV_KEYS - 1) / DKV_KEYS),

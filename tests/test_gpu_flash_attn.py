@@ -97,6 +97,36 @@ def test_backward_matches_oracle(device, lengths, H, window):
         rel_check(got.float().cpu().numpy(), ref)
 
 
+@pytest.mark.parametrize("scale", [None, 1e-39])
+@pytest.mark.parametrize("window", [None, 0, 1, 31, 32, 33, 95])
+def test_key_gradients_at_tile_edges(device, window, scale):
+    """dK, dV around the 32 x 32 tiles' edges (keys a wave, rows a tile, keys a workgroup), window ends inside and on a
+    tile, and a scale whose lse / scale would overflow (every weight then 1 / the row's keys). Each against float64 from
+    the same inputs within one bf16 rounding (8 significant bits: 2^-8) of each term's P or dS and one of the result, and
+    2^-16 of the terms' magnitudes for the fp32 lse, exponentials and sums."""
+    lengths, H = [1, 31, 32, 33, 63, 65, 96, 127, 128, 129, 161], 1
+    q, k, v, cu, _ = make(lengths, H, seed=77)
+    dout = torch.randn(q.shape, generator=torch.Generator().manual_seed(78)).bfloat16()
+    qd, kd, vd, dod, cud = (t.to(device) for t in (q, k, v, dout, cu))
+    out, lse = flash_attn_fwd(qd, kd, vd, cud, max(lengths), window_left=window, softmax_scale=scale)
+    rows = flash_attn_bwd_rows(out, dod)
+    _, dk, dv = flash_attn_bwd(qd, kd, vd, out, dod, lse, cud, max(lengths), rows=rows, window_left=window,
+                               softmax_scale=scale)
+    rows, dk, dv = (t.double().cpu() for t in (rows, dk, dv))
+    sc = 128 ** -0.5 if scale is None else scale
+    for s, e in zip(cu[:-1].tolist(), cu[1:].tolist()):
+        Q, K, V, dO = (t[s:e, 0].double() for t in (q, k, v, dout))
+        i = torch.arange(e - s)
+        seen = (i[:, None] >= i) & (i[:, None] - i <= (window if window is not None else e - s))
+        P = torch.softmax((Q @ K.T * sc).masked_fill(~seen, -float("inf")), -1)
+        dP = dO @ V.T
+        dS = P * (dP - rows[s:e])
+        mag = P * (dP.abs() + (dO.abs() @ V.abs().T) + rows[s:e].abs())
+        for got, want, terms in ((dv[s:e, 0], P.T @ dO, P.T @ dO.abs()), (dk[s:e, 0], sc * dS.T @ Q, sc * mag.T @ Q.abs())):
+            tol = 2.0 ** -8 * want.abs() + (2.0 ** -8 + 2.0 ** -16) * terms + 2.0 ** -133
+            assert bool(((got - want).abs() <= tol).all()), (s, e, float(((got - want).abs() / tol).max()))
+
+
 def test_backward_rows_and_strided_dv(device):
     """rows given (the reference passes D from the o_proj epilogue), dv written into the v block of a fused
     gradient, v a view of the fused projection."""

@@ -8,10 +8,10 @@
  *   out[i] = sum_j softmax_j(scale q_i . k_j) v_j          bf16, fp32 accumulation
  *   lse[h][i] = ln sum_j exp(scale q_i . k_j)              fp32 (FA4's (H, total) layout)
  *
- * Mapping: a workgroup of four waves owns 128 query rows of one (segment, head), each wave two 16-row tiles. Keys
+ * Mapping: a workgroup of four waves owns 128 query rows of one (segment, head), each wave 32. Keys
  * are visited in blocks of 64, staged in LDS for the four waves (K and V row-major with 16-byte chunks XOR-swizzled
  * by the key) by LDS DMA straight from HBM, in two LDS stages: block b+1 is fetched into one while block b is read
- * from the other, with no registers held for the fetch. Scores are S^T = K Q^T (v_mfma_f32_16x16x32_bf16, keys as
+ * from the other, with no registers held for the fetch. Scores are S^T = K Q^T (v_mfma_f32_32x32x16_bf16, keys as
  * rows, queries as columns), so a lane's scores all belong to one query; the online softmax runs in the log2 domain
  * with the lazy rescale of the decode kernels (the reference max moves only when a column's max passes it by 2^8);
  * P^T then feeds O^T += V^T P^T with no shuffle: the V^T operand is read from the row-major tile by gfx950's
@@ -46,11 +46,17 @@ struct FlashFwd {
 };
 
 struct FaStage {
-    uint16_t k[FA_BN * HEAD_DIM];   /* [key][128], 16-byte chunk c of key j at chunk c ^ (j & 15) */
+    uint16_t k[FA_BN * HEAD_DIM];   /* [key][128], 16-byte chunk c of key j at chunk c ^ k_swizzle(j) */
     uint16_t v[FA_BN * HEAD_DIM];   /* the same layout: read transposed by ds_read_b64_tr_b16 */
 };
 
-__device__ __forceinline__ int k_lds(int key, int chunk) { return key * HEAD_DIM + ((chunk ^ (key & 15)) << 3); }
+/* A row is 256 bytes, all 64 banks, so where rows meet in one access they need different chunks. A row operand's 16 lanes
+ * read one chunk of 16 rows: any one-to-one map of row % 16 does. A transposing read's 32 lanes read the same four chunks
+ * of four rows r0 .. r0 + 3 (r0 a multiple of 4), so the row's low two bits pick the group of four chunks. With chunk
+ * c ^ (row & 15) those rows met in one group: each such read waited 6 cycles, 53 % of the dK/dV kernel's LDS cycles
+ * (none now). */
+__device__ __forceinline__ int k_swizzle(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
+__device__ __forceinline__ int k_lds(int row, int chunk) { return row * HEAD_DIM + ((chunk ^ k_swizzle(row)) << 3); }
 
 __device__ __forceinline__ Rsrc make_rsrc(const void *p, unsigned bytes) {
     const unsigned long long u = (unsigned long long)p;
@@ -82,7 +88,7 @@ typedef __attribute__((address_space(3))) v4i16 LdsV4;
 
 /* A 64-row tile of one head straight into LDS in the k_lds layout by LDS DMA (no registers held), shared by NW
  * waves: instruction i of a wave writes rows 4 i' .. 4 i' + 3 (i' = wave + NW i), lane l the 16 bytes at LDS chunk
- * l % 16 of row 4 i' + l / 16, fetched from the row's chunk (l % 16) ^ (row & 15). Rows past the descriptor's range
+ * l % 16 of row 4 i' + l / 16, fetched from the row's chunk (l % 16) ^ k_swizzle(row). Rows past the descriptor's range
  * read zeros. */
 template <int NW = 4>
 __device__ __forceinline__ void tile_dma(const uint16_t *base, long long row0, long long stride, int h, int rows,
@@ -91,15 +97,15 @@ __device__ __forceinline__ void tile_dma(const uint16_t *base, long long row0, l
 #pragma unroll
     for (int k = 0; k < FA_BN / 4 / NW; k++) {
         const int i = wave + NW * k, r = 4 * i + (lane >> 4), p = lane & 15;
-        const int off = (int)((r * stride + ((p ^ (r & 15)) << 3)) * 2);
+        const int off = (int)((r * stride + ((p ^ k_swizzle(r)) << 3)) * 2);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (LdsVoid *)(lds + i * 4 * HEAD_DIM), 16, off, 0, 0, 0);
     }
 }
 
 /* The A operand of a product over 32 rows of a row-major (k_lds) tile (V^T in O^T += V^T P^T; dO^T, Q^T, K^T in the
  * backward) for dim tile d and k-step s2, in the row order of a score MFMA's output pair: lane (g, c) gets rows
- * 32 s2 + 4 g .. + 3, then 32 s2 + 16 + 4 g .. + 3, of dim 16 d + c. ds_read_b64_tr_b16 hands lane i of a 16-lane group element i % 4 of the 8 bytes lane 4 t + i / 4 points
- * at, for t = 0..3: so lane j of group g points at dims 16 d + 4 (j % 4) .. + 3 of key base + j / 4. */
+ * 32 s2 + 4 g .. + 3, then 32 s2 + 16 + 4 g .. + 3, of dim 16 d + c. ds_read_b64_tr_b16 hands lane i of a 16-lane group
+ * element i % 4 of the 8 bytes lane 4 t + i / 4 points at, for t = 0..3: so lane j of group g points at dims 16 d + 4 (j % 4) .. + 3 of key base + j / 4. */
 __device__ __forceinline__ bf16x8 tr_operand(const uint16_t *v, int d, int s2, int g, int c) {
     const int dim = 16 * d + 4 * (c & 3), chunk = dim >> 3, half = (dim >> 2) & 1;
     const int r0 = 32 * s2 + 4 * g + (c >> 2), r1 = r0 + 16;
@@ -110,239 +116,6 @@ __device__ __forceinline__ bf16x8 tr_operand(const uint16_t *v, int d, int s2, i
     const uint2 a = __builtin_bit_cast(uint2, lo), b = __builtin_bit_cast(uint2, hi);
     return __builtin_bit_cast(bf16x8, uint4{a.x, a.y, b.x, b.y});
 }
-
-struct FaState {
-    f32x4 o[2][8];   /* O^T tile d of query tile j: dims 16d + 4g + i of column (lane & 15) */
-    float m[2];      /* the column's reference max (log2 domain), equal in the four groups */
-    float l[2];      /* sum of exp2(s - m) over the keys this lane's group holds */
-};
-
-/* One key block for the wave's two query tiles. kb0: the block's first key (segment-relative); q0: the wave's first
- * query row (segment-relative). MASKED: apply causal, window and segment-end bounds per score. */
-template <bool MASKED>
-__device__ __forceinline__ void fa_block(const FlashFwd &a, const FaStage &s, const bf16x8 (&qb)[2][4], FaState &st,
-                                         int kb0, int q0, int seglen, int lane) {
-    const int g = lane >> 4, c = lane & 15;
-    f32x4 sc[2][4];
-#pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-        for (int kt = 0; kt < 4; kt++) sc[j][kt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    /* raised priority while the scores issue: the SIMD's other wave runs its softmax between them (fa forward
-     * 464 -> 471.5 TFLOP/s; the same around the PV products, or around the backward's S / dP products, was slower) */
-    __builtin_amdgcn_s_setprio(1);
-    /* tile 0's scores, then tile 1's (K operands read from LDS once per tile), so tile 1's products can issue among
-     * tile 0's scale, mask and max instructions (the groups below): 471.8 -> 476.6 TFLOP/s; without the groups the
-     * compiler issued them all first and the forward fell to 343.6 */
-#pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-        for (int kt = 0; kt < 4; kt++)
-#pragma unroll
-            for (int cc = 0; cc < 4; cc++) sc[j][kt] = mfma16x16x32(rows_operand(s.k, kt, cc, g, c), qb[j][cc], sc[j][kt]);
-    __builtin_amdgcn_s_setprio(0);
-    bf16x8 pv[2][2];
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int qi = q0 + 16 * j + c;
-        /* raw scores: the scale is positive, so the max of the scaled scores is the scaled max, and it is folded into
-         * one FMA per exponential below */
-        float sv[16];
-#pragma unroll
-        for (int kt = 0; kt < 4; kt++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                float x = sc[j][kt][i];
-                if (MASKED) {
-                    const int key = kb0 + kt * 16 + 4 * g + i;
-                    const bool ok = (key <= qi) & (key < seglen) & ((a.window < 0) | (qi - key <= a.window));
-                    x = ok ? x : -INFINITY;
-                }
-                sv[kt * 4 + i] = x;
-            }
-        float mt = sv[0];
-#pragma unroll
-        for (int i = 1; i < 16; i++) mt = fmaxf(mt, sv[i]);
-        mt = pair_max32(pair_max16(mt)) * a.scale_log2;
-        if (j == 0) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 16, 0);
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
-            }
-        }
-        const float mnew = fmaxf(st.m[j], mt);
-        if (__any(mnew > st.m[j] + FA_RESCALE)) {
-            const float alpha = mnew == st.m[j] ? 1.0f : __builtin_amdgcn_exp2f(st.m[j] - mnew);
-#pragma unroll
-            for (int d = 0; d < 8; d++) st.o[j][d] *= alpha;
-            st.l[j] *= alpha;
-            st.m[j] = mnew;
-        }
-        const float mbase = st.m[j] == -INFINITY ? 0.0f : st.m[j];
-        float psum = 0.0f;
-        float p[16];
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            p[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[i], a.scale_log2, -mbase));
-            psum += p[i];
-        }
-        st.l[j] += psum;
-        /* k-step s2 covers key tiles 2 s2 and 2 s2 + 1: the group's keys 4g..4g+3 of each */
-#pragma unroll
-        for (int s2 = 0; s2 < 2; s2++)
-#pragma unroll
-            for (int i = 0; i < 8; i++) pv[j][s2][i] = (__bf16)p[(2 * s2 + (i >> 2)) * 4 + (i & 3)];
-    }
-#pragma unroll
-    for (int d = 0; d < 8; d++) {
-#pragma unroll
-        for (int s2 = 0; s2 < 2; s2++) {
-            const bf16x8 vop = tr_operand(s.v, d, s2, g, c);
-#pragma unroll
-            for (int j = 0; j < 2; j++) st.o[j][d] = mfma16x16x32(vop, pv[j][s2], st.o[j][d]);
-        }
-    }
-}
-
-/* A workgroup's (rank, segment, head) from its place in the launch order: work-groups start in linear order (x,
- * then y, then z), so rank r = L / (segments heads) takes the r-th tile of every (segment, head) before any takes
- * the (r + 1)-th. The kernels map rank 0 to their longest tile, so the short ones of every head come last, where they
- * fill the CUs the long ones leave (the grid keeps x = tiles, y = segments, z = heads). */
-struct FaBlock {
-    int rank, seg, h;
-};
-
-__device__ __forceinline__ FaBlock fa_block_order() {
-    const int yz = (int)(gridDim.y * gridDim.z);
-    const int L = (int)blockIdx.x + (int)gridDim.x * ((int)blockIdx.y + (int)gridDim.y * (int)blockIdx.z);
-    const int r = L % yz;
-    return FaBlock{L / yz, r % (int)gridDim.y, r / (int)gridDim.y};
-}
-
-__global__ void __launch_bounds__(FA_THREADS, 2) flash_fwd_kernel(FlashFwd a) {
-    __shared__ FaStage st0, st1;   /* distinct objects: a read of one never waits for DMA into the other */
-    const FaBlock fb = fa_block_order();
-    const int seg = fb.seg, h = fb.h;
-    const long long start = a.cu[seg];
-    const int seglen = a.cu[seg + 1] - a.cu[seg];
-    const int tile = (int)gridDim.x - 1 - fb.rank;   /* the longest key ranges first */
-    const int qa = tile * FA_BM;
-    if (seglen <= 0 || qa >= seglen) return;
-    const int t = threadIdx.x, lane = t & (WAVE - 1), wave = t >> 6, g = lane >> 4, c = lane & 15;
-    const int qb = min(qa + FA_BM, seglen) - 1;
-    const int q0 = qa + wave * 32;                                 /* the wave's first row */
-    const bool active = q0 < seglen;
-    const int qw1 = min(q0 + 31, seglen - 1);                       /* the wave's last valid row */
-
-    /* the wave's queries: B operand of S^T = K Q^T, lane (g, c) holds dims 32 cc + 8 g .. +7 of row c */
-    bf16x8 qb_[2][4];
-    {
-        const Rsrc rq = rows_rsrc(a.q, start + q0, a.q_stride, h, active ? min(32, seglen - q0) : 0);
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int cc = 0; cc < 4; cc++)
-                qb_[j][cc] = __builtin_bit_cast(bf16x8, bload(rq, (int)(((16 * j + c) * a.q_stride + cc * 32 + g * 8) * 2)));
-    }
-    FaState st;
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-#pragma unroll
-        for (int d = 0; d < 8; d++) st.o[j][d] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        st.m[j] = -INFINITY;
-        st.l[j] = 0.0f;
-    }
-
-    const int klo = a.window >= 0 ? max(0, qa - a.window) : 0;
-    const int kb_lo = klo / FA_BN, kb_hi = qb / FA_BN;
-    /* block kb + 1 is fetched by LDS DMA into the other stage while block kb is computed; the barrier after the
-     * compute (its fence waits for this wave's DMA) makes the fetched block visible and frees the one just read */
-    auto fetch = [&](int kb, FaStage &stg) {
-        const int n = min(FA_BN, seglen - kb * FA_BN);
-        tile_dma(a.k, start + kb * FA_BN, a.k_stride, h, n, stg.k, wave, lane);
-        tile_dma(a.v, start + kb * FA_BN, a.v_stride, h, n, stg.v, wave, lane);
-    };
-    auto compute = [&](int kb, const FaStage &stg) {
-        if (!active) return;
-        const int k0 = kb * FA_BN, k1 = k0 + FA_BN - 1;
-        /* unmasked iff every key of the block is visible to every row of the wave */
-        const bool interior = k1 <= q0 && k1 < seglen && (a.window < 0 || qw1 - k0 <= a.window);
-        if (interior)
-            fa_block<false>(a, stg, qb_, st, k0, q0, seglen, lane);
-        else
-            fa_block<true>(a, stg, qb_, st, k0, q0, seglen, lane);
-    };
-    fetch(kb_lo, st0);
-    __syncthreads();
-    for (int kb = kb_lo; kb <= kb_hi; kb += 2) {
-        if (kb + 1 <= kb_hi) fetch(kb + 1, st1);
-        compute(kb, st0);
-        __syncthreads();
-        if (kb + 1 > kb_hi) break;
-        if (kb + 2 <= kb_hi) fetch(kb + 2, st0);
-        compute(kb + 1, st1);
-        __syncthreads();
-    }
-    if (!active) return;
-
-    /* out = O^T / l, lse = (m + log2 l) ln 2 */
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int row = q0 + 16 * j + c;
-        const float l = pair_sum32(pair_sum16(st.l[j]));
-        if (row >= seglen) continue;
-        const long long tok = start + row;
-        const float inv = 1.0f / l;
-        uint16_t *o = a.out + (tok * a.H + h) * HEAD_DIM + 4 * g;
-#pragma unroll
-        for (int d = 0; d < 8; d++) {
-            const f32x4 v = st.o[j][d];
-            *reinterpret_cast<uint2 *>(o + d * 16) =
-                uint2{(uint32_t)f32_to_bf16(v[0] * inv) | ((uint32_t)f32_to_bf16(v[1] * inv) << 16),
-                      (uint32_t)f32_to_bf16(v[2] * inv) | ((uint32_t)f32_to_bf16(v[3] * inv) << 16)};
-        }
-        if (g == 0) a.lse[(long long)h * a.lse_stride + tok] = (st.m[j] + __log2f(l)) * FA_LN2;
-    }
-}
-
-/* ---------------------------------------------------------------------------------------------------------------
- * Backward (the reference's _flash_attn_bwd / bwd_bf16dq, model/ops/flash_attn.py:367-391), per segment and head:
- *   P = exp(scale S - lse), dV = P^T dO, dP = dO V^T, dS = P (dP - D) with D_i = dO_i . O_i (the caller's row
- *   statistics: the reference's `rows`, from the o_proj backward epilogue), dQ = scale dS K, dK = scale dS^T Q.
- * Two kernels and no atomics: flash_bwd_dkv_kernel owns 128 keys (a wave 16) and walks the query blocks that see them;
- * flash_bwd_dq_kernel owns 128 queries (a wave 32, as the forward) and walks their key blocks. S and dP are computed
- * in both (seven 128-deep products per (query, key) pair instead of five), the price of writing dQ once.
- * ------------------------------------------------------------------------------------------------------------- */
-
-struct FlashBwd {
-    const uint16_t *q, *k, *v, *dout;         /* (total, H, 128) at token strides */
-    long long q_stride, k_stride, v_stride, do_stride;
-    const float *lse;                          /* [H][lse_stride], natural log */
-    long long lse_stride;
-    const float *dpsum;                        /* (total, H): D = dO . O per row */
-    const int32_t *cu;
-    int segments, H, window;
-    float scale, scale_log2;
-    uint16_t *dq, *dk, *dv;                    /* (total, H, 128) at their token strides */
-    long long dq_stride, dk_stride, dv_stride;
-};
-
-/* bitwise, not short-circuit: evaluated per element inside unrolled loops, a branch per term would split the wave */
-__device__ __forceinline__ bool visible(int key, int q, int seglen, int window) {
-    return (key <= q) & (q < seglen) & ((window < 0) | (q - key <= window));
-}
-
-__device__ __forceinline__ void store4(uint16_t *p, const f32x4 &v, float mul) {
-    *reinterpret_cast<uint2 *>(p) = uint2{(uint32_t)f32_to_bf16(v[0] * mul) | ((uint32_t)f32_to_bf16(v[1] * mul) << 16),
-                                          (uint32_t)f32_to_bf16(v[2] * mul) | ((uint32_t)f32_to_bf16(v[3] * mul) << 16)};
-}
-
-struct alignas(16) DkvStage {
-    uint16_t q[FA_BN * HEAD_DIM], dout[FA_BN * HEAD_DIM];   /* k_lds layout; Q^T and dO^T read transposed */
-    float nlse[FA_BN], nd[FA_BN];              /* the block's rows: -lse / scale (-inf past the segment), -D */
-};
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -373,10 +146,221 @@ __device__ __forceinline__ bf16x8 rows_operand32(const uint16_t *tile, uint32_t 
 __device__ __forceinline__ bf16x8 tr_operand32(const uint16_t *tile, uint32_t at, int dt, int r0) {
     LdsByte *p = (LdsByte *)tile + r0 * HEAD_DIM * 2;
     const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsV4 *)(p + (at ^ (dt << 6))));
-    const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsV4 *)(p + (at ^ (dt << 6) ^ 128) + 8 * HEAD_DIM * 2));
+    const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsV4 *)(p + (at ^ (dt << 6) ^ 32) + 8 * HEAD_DIM * 2));
     const uint2 x = __builtin_bit_cast(uint2, lo), y = __builtin_bit_cast(uint2, hi);
     return __builtin_bit_cast(bf16x8, uint4{x.x, x.y, y.x, y.y});
 }
+
+__device__ __forceinline__ void store4(uint16_t *p, const f32x4 &v, float mul) {
+    *reinterpret_cast<uint2 *>(p) = uint2{(uint32_t)f32_to_bf16(v[0] * mul) | ((uint32_t)f32_to_bf16(v[1] * mul) << 16),
+                                          (uint32_t)f32_to_bf16(v[2] * mul) | ((uint32_t)f32_to_bf16(v[3] * mul) << 16)};
+}
+
+struct FaState {
+    f32x16 o[4];   /* O^T tile d: dims 32 d + 8 j + 4 hf + i of column (lane & 31) in registers 4 j + i */
+    float m;       /* the column's reference max (log2 domain), equal in both halves */
+    float l;       /* sum of exp2(s - m) over the keys this lane's half holds */
+};
+
+/* One key block for the wave's 32 queries. kb0: the block's first key (segment-relative); qi: the lane's query row
+ * (segment-relative). MASKED: apply causal, window and segment-end bounds per score.
+ * Bound by the matrix cores and the exponentials' issue together, at the clock the power limit leaves. 32 x 32 products
+ * read K from LDS once for the wave's 32 queries (two 16-wide tiles read it twice) and a column's maximum needs one
+ * exchange, not two; blocks no row of a wave sees are skipped. 2 segments of 8,192 tokens x 6 heads: 280 -> 234 us;
+ * 8 x 2,048 x 10 heads, window 512: 80 -> 73; 5 x 3,000 x 4: 89 -> 71; 32 x 2,048 x 6, where HBM traffic takes its share of
+ * the power: 346 -> 338. Measured slower: the second tile's products among the first one's maxima, the second half's
+ * exponentials among the first half's PV products (+ 3 %), a raised wave priority around the scores (+ 4 %). */
+template <bool MASKED>
+__device__ __forceinline__ void fa_block(const FlashFwd &a, const FaStage &s, const bf16x8 (&qb)[8], FaState &st,
+                                         uint32_t rat, uint32_t tat, int kb0, int qi, int seglen, int hf) {
+    f32x16 sc[2];
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) sc[kt][i] = 0.0f;
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+        for (int cc = 0; cc < 8; cc++) sc[kt] = mfma32x32x16(rows_operand32(s.k, rat, kt, cc), qb[cc], sc[kt]);
+    /* tile 0's scores, then tile 1's, each operand read four products ahead */
+    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+    for (int m = 0; m < 16; m++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if (m < 12) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    /* raw scores: the scale is positive, so the max of the scaled scores is the scaled max, and it is folded into
+     * one FMA per exponential below */
+    if (MASKED) {
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int key = kb0 + 32 * kt + 8 * (i >> 2) + 4 * hf + (i & 3);
+                const bool ok = (key <= qi) & (key < seglen) & ((a.window < 0) | (qi - key <= a.window));
+                sc[kt][i] = ok ? sc[kt][i] : -INFINITY;
+            }
+    }
+    float mt = sc[0][0];
+#pragma unroll
+    for (int i = 1; i < 32; i++) mt = fmaxf(mt, sc[i >> 4][i & 15]);
+    mt = pair_max32(mt) * a.scale_log2;
+    const float mnew = fmaxf(st.m, mt);
+    if (__any(mnew > st.m + FA_RESCALE)) {
+        const float alpha = mnew == st.m ? 1.0f : __builtin_amdgcn_exp2f(st.m - mnew);
+#pragma unroll
+        for (int d = 0; d < 4; d++) st.o[d] *= alpha;
+        st.l *= alpha;
+        st.m = mnew;
+    }
+    const float mbase = st.m == -INFINITY ? 0.0f : st.m;
+    bf16x8 pv[4];
+    float psum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 32; i++) {
+        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i >> 4][i & 15], a.scale_log2, -mbase));
+        psum += p;
+        pv[i >> 3][i & 7] = (__bf16)p;
+    }
+    st.l += psum;
+    /* k-step s2: the half's keys 16 s2 + 4 hf .. + 3 and 16 s2 + 8 + 4 hf .. + 3 */
+#pragma unroll
+    for (int s2 = 0; s2 < 4; s2++)
+#pragma unroll
+        for (int d = 0; d < 4; d++) st.o[d] = mfma32x32x16(tr_operand32(s.v, tat, d, 16 * s2), pv[s2], st.o[d]);
+    __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+#pragma unroll
+    for (int m = 0; m < 16; m++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if (m < 12) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+    }
+}
+
+/* A workgroup's (rank, segment, head) from its place in the launch order: work-groups start in linear order (x,
+ * then y, then z), so rank r = L / (segments heads) takes the r-th tile of every (segment, head) before any takes
+ * the (r + 1)-th. The kernels map rank 0 to their longest tile, so the short ones of every head come last, where they
+ * fill the CUs the long ones leave (the grid keeps x = tiles, y = segments, z = heads). */
+struct FaBlock {
+    int rank, seg, h;
+};
+
+__device__ __forceinline__ FaBlock fa_block_order() {
+    const int yz = (int)(gridDim.y * gridDim.z);
+    const int L = (int)blockIdx.x + (int)gridDim.x * ((int)blockIdx.y + (int)gridDim.y * (int)blockIdx.z);
+    const int r = L % yz;
+    return FaBlock{L / yz, r % (int)gridDim.y, r / (int)gridDim.y};
+}
+
+__global__ void __launch_bounds__(FA_THREADS, 2) flash_fwd_kernel(FlashFwd a) {
+    __shared__ FaStage st0, st1;   /* distinct objects: a read of one never waits for DMA into the other */
+    const FaBlock fb = fa_block_order();
+    const int seg = fb.seg, h = fb.h;
+    const long long start = a.cu[seg];
+    const int seglen = a.cu[seg + 1] - a.cu[seg];
+    const int tile = (int)gridDim.x - 1 - fb.rank;   /* the longest key ranges first */
+    const int qa = tile * FA_BM;
+    if (seglen <= 0 || qa >= seglen) return;
+    const int t = threadIdx.x, lane = t & (WAVE - 1), hf = lane >> 5, c = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);   /* in a scalar register, as are the bounds made of it */
+    const int qb = min(qa + FA_BM, seglen) - 1;
+    const int q0 = qa + wave * 32;                                 /* the wave's first row */
+    const bool active = q0 < seglen;
+    const int qw1 = min(q0 + 31, seglen - 1);                       /* the wave's last valid row */
+
+    /* the wave's queries: B operand of S^T = K Q^T, lane (hf, c) holds dims 16 cc + 8 hf .. +7 of row c */
+    bf16x8 qb_[8];
+    {
+        const Rsrc rq = rows_rsrc(a.q, start + q0, a.q_stride, h, active ? min(32, seglen - q0) : 0);
+#pragma unroll
+        for (int cc = 0; cc < 8; cc++)
+            qb_[cc] = __builtin_bit_cast(bf16x8, bload(rq, (int)((c * a.q_stride + cc * 16 + hf * 8) * 2)));
+    }
+    FaState st;
+#pragma unroll
+    for (int d = 0; d < 4; d++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) st.o[d][i] = 0.0f;
+    st.m = -INFINITY;
+    st.l = 0.0f;
+
+    const int klo = a.window >= 0 ? max(0, qa - a.window) : 0;
+    const int kb_lo = klo / FA_BN, kb_hi = qb / FA_BN;
+    /* block kb + 1 is fetched by LDS DMA into the other stage while block kb is computed; the barrier after the
+     * compute (its fence waits for this wave's DMA) makes the fetched block visible and frees the one just read */
+    auto fetch = [&](int kb, FaStage &stg) {
+        const int n = min(FA_BN, seglen - kb * FA_BN);
+        tile_dma(a.k, start + kb * FA_BN, a.k_stride, h, n, stg.k, wave, lane);
+        tile_dma(a.v, start + kb * FA_BN, a.v_stride, h, n, stg.v, wave, lane);
+    };
+    const uint32_t rat = rows_at(lane), tat = tr_at(lane);
+    auto compute = [&](int kb, const FaStage &stg) {
+        const int k0 = kb * FA_BN, k1 = k0 + FA_BN - 1;
+        if (!active || k0 > qw1 || (a.window >= 0 && q0 - k1 > a.window)) return;   /* no row sees the keys */
+        /* unmasked iff every key of the block is visible to every row of the wave */
+        const bool interior = k1 <= q0 && k1 < seglen && (a.window < 0 || qw1 - k0 <= a.window);
+        if (interior)
+            fa_block<false>(a, stg, qb_, st, rat, tat, k0, q0 + c, seglen, hf);
+        else
+            fa_block<true>(a, stg, qb_, st, rat, tat, k0, q0 + c, seglen, hf);
+    };
+    fetch(kb_lo, st0);
+    __syncthreads();
+    for (int kb = kb_lo; kb <= kb_hi; kb += 2) {
+        if (kb + 1 <= kb_hi) fetch(kb + 1, st1);
+        compute(kb, st0);
+        __syncthreads();
+        if (kb + 1 > kb_hi) break;
+        if (kb + 2 <= kb_hi) fetch(kb + 2, st0);
+        compute(kb + 1, st1);
+        __syncthreads();
+    }
+    if (!active) return;
+
+    /* out = O^T / l, lse = (m + log2 l) ln 2 */
+    const float l = pair_sum32(st.l);
+    if (q0 + c >= seglen) return;
+    const long long tok = start + q0 + c;
+    const float inv = 1.0f / l;
+    uint16_t *o = a.out + (tok * a.H + h) * HEAD_DIM + 4 * hf;
+#pragma unroll
+    for (int d = 0; d < 4; d++)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            store4(o + d * 32 + 8 * j, f32x4{st.o[d][4 * j], st.o[d][4 * j + 1], st.o[d][4 * j + 2], st.o[d][4 * j + 3]}, inv);
+    if (hf == 0) a.lse[(long long)h * a.lse_stride + tok] = (st.m + __log2f(l)) * FA_LN2;
+}
+
+/* ---------------------------------------------------------------------------------------------------------------
+ * Backward (the reference's _flash_attn_bwd / bwd_bf16dq, model/ops/flash_attn.py:367-391), per segment and head:
+ *   P = exp(scale S - lse), dV = P^T dO, dP = dO V^T, dS = P (dP - D) with D_i = dO_i . O_i (the caller's row
+ *   statistics: the reference's `rows`, from the o_proj backward epilogue), dQ = scale dS K, dK = scale dS^T Q.
+ * Two kernels and no atomics: flash_bwd_dkv_kernel owns 128 keys (a wave 16) and walks the query blocks that see them;
+ * flash_bwd_dq_kernel owns 128 queries (a wave 32, as the forward) and walks their key blocks. S and dP are computed
+ * in both (seven 128-deep products per (query, key) pair instead of five), the price of writing dQ once.
+ * ------------------------------------------------------------------------------------------------------------- */
+
+struct FlashBwd {
+    const uint16_t *q, *k, *v, *dout;         /* (total, H, 128) at token strides */
+    long long q_stride, k_stride, v_stride, do_stride;
+    const float *lse;                          /* [H][lse_stride], natural log */
+    long long lse_stride;
+    const float *dpsum;                        /* (total, H): D = dO . O per row */
+    const int32_t *cu;
+    int segments, H, window;
+    float scale, scale_log2;
+    uint16_t *dq, *dk, *dv;                    /* (total, H, 128) at their token strides */
+    long long dq_stride, dk_stride, dv_stride;
+};
+
+/* bitwise, not short-circuit: evaluated per element inside unrolled loops, a branch per term would split the wave */
+__device__ __forceinline__ bool visible(int key, int q, int seglen, int window) {
+    return (key <= q) & (q < seglen) & ((window < 0) | (q - key <= window));
+}
+
+struct alignas(16) DkvStage {
+    uint16_t q[FA_BN * HEAD_DIM], dout[FA_BN * HEAD_DIM];   /* k_lds layout; Q^T and dO^T read transposed */
+    float nlse[FA_BN], nd[FA_BN];              /* the block's rows: -lse / scale (-inf past the segment), -D */
+};
 
 /* dK, dV of 128 keys, 32 a wave: S = Q K^T and dP = dO V^T in 32 x 32 tiles with queries as rows (a lane holds one key's
  * column), so P and dS feed dV^T += dO^T P and dK^T += Q^T dS directly as B operands, with dO^T and Q^T read transposed from

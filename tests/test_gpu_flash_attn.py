@@ -71,6 +71,27 @@ def test_training_shape_against_float32_sdpa(device):
     assert err.max().item() <= MAX_ABS and err.mean().item() <= MEAN_ABS
 
 
+@pytest.mark.parametrize("window", [None, 0, 1, 31, 32, 33, 95])
+def test_forward_at_tile_edges(device, window):
+    """Around the wave's 32 rows, the 32-key tiles, the 64-key blocks and the workgroup's 128 rows. Output against
+    float64 of the same inputs within one bf16 rounding (2^-8) of each weight's term and one of the result, and 2^-16 of
+    the terms' magnitudes for the fp32 scores, exponentials and sums; lse within 1e-5 of its size."""
+    lengths, H = [1, 31, 32, 33, 63, 65, 96, 127, 128, 129, 161], 1
+    q, k, v, cu, _ = make(lengths, H, seed=79)
+    out, lse = run(device, q, k, v, cu, max(lengths), window)
+    for s, e in zip(cu[:-1].tolist(), cu[1:].tolist()):
+        Q, K, V = (t[s:e, 0].double() for t in (q, k, v))
+        i = torch.arange(e - s)
+        seen = (i[:, None] >= i) & (i[:, None] - i <= (window if window is not None else e - s))
+        S = (Q @ K.T * 128 ** -0.5).masked_fill(~seen, -float("inf"))
+        P = torch.softmax(S, -1)
+        want, ref = P @ V, torch.logsumexp(S, -1)
+        tol = 2.0 ** -8 * want.abs() + (2.0 ** -8 + 2.0 ** -16) * (P @ V.abs())
+        got = torch.from_numpy(out[s:e, 0]).double()
+        assert bool(((got - want).abs() <= tol).all()), (s, e, float(((got - want).abs() / tol).max()))
+        assert bool(((torch.from_numpy(lse[0, s:e]).double() - ref).abs() <= 1e-5 * (1 + ref.abs())).all()), (s, e)
+
+
 def rel_check(got, ref, max_rel=2e-2, mean_rel=1e-2):
     """bf16 gradients: max error against the largest reference value, mean error against the mean magnitude (floors
     of 1e-3 and 1e-4: with window 0 dq and dk are exactly zero and the device's are rounding noise)."""

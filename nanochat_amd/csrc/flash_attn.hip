@@ -76,12 +76,6 @@ __device__ __forceinline__ Rsrc rows_rsrc(const uint16_t *base, long long row0, 
     return make_rsrc(base + row0 * stride + (long long)h * HEAD_DIM, bytes);
 }
 
-/* The A operand of a product over the dimension from a row-major tile: lane (g, c) holds dims 32 cc + 8 g .. +7 of
- * row 16 rt + c. */
-__device__ __forceinline__ bf16x8 rows_operand(const uint16_t *lds, int rt, int cc, int g, int c) {
-    return *reinterpret_cast<const bf16x8 *>(&lds[k_lds(rt * 16 + c, cc * 4 + g)]);
-}
-
 typedef __attribute__((address_space(3))) void LdsVoid;
 typedef short v4i16 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) v4i16 LdsV4;
@@ -102,21 +96,6 @@ __device__ __forceinline__ void tile_dma(const uint16_t *base, long long row0, l
     }
 }
 
-/* The A operand of a product over 32 rows of a row-major (k_lds) tile (V^T in O^T += V^T P^T; dO^T, Q^T, K^T in the
- * backward) for dim tile d and k-step s2, in the row order of a score MFMA's output pair: lane (g, c) gets rows
- * 32 s2 + 4 g .. + 3, then 32 s2 + 16 + 4 g .. + 3, of dim 16 d + c. ds_read_b64_tr_b16 hands lane i of a 16-lane group
- * element i % 4 of the 8 bytes lane 4 t + i / 4 points at, for t = 0..3: so lane j of group g points at dims 16 d + 4 (j % 4) .. + 3 of key base + j / 4. */
-__device__ __forceinline__ bf16x8 tr_operand(const uint16_t *v, int d, int s2, int g, int c) {
-    const int dim = 16 * d + 4 * (c & 3), chunk = dim >> 3, half = (dim >> 2) & 1;
-    const int r0 = 32 * s2 + 4 * g + (c >> 2), r1 = r0 + 16;
-    const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-        (LdsV4 *)(v + k_lds(r0, chunk) + 4 * half));
-    const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-        (LdsV4 *)(v + k_lds(r1, chunk) + 4 * half));
-    const uint2 a = __builtin_bit_cast(uint2, lo), b = __builtin_bit_cast(uint2, hi);
-    return __builtin_bit_cast(bf16x8, uint4{a.x, a.y, b.x, b.y});
-}
-
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ f32x16 mfma32x32x16(const bf16x8 &a, const bf16x8 &b, const f32x16 &c) {
@@ -127,8 +106,9 @@ __device__ __forceinline__ f32x16 mfma32x32x16(const bf16x8 &a, const bf16x8 &b,
  * offset's xor with a constant, plus a constant, so two registers address them all.
  * rows_at: the products over the dimension; lane (hf, c) = (lane / 32, lane % 32) holds dims 16 cc + 8 hf .. +7 of row
  * 32 rt + c. tr_at: the products over 16 rows r0 .. r0 + 15, in the row order of a score tile's registers: lane (hf, c) gets
- * rows r0 + 4 hf .. + 3, then r0 + 8 + 4 hf .. + 3, of dim 32 dt + c (ds_read_b64_tr_b16 as in tr_operand: a lane points at
- * row base + (lane % 16) / 4, dims 4 (lane % 4) .. + 3 of its 16). */
+ * rows r0 + 4 hf .. + 3, then r0 + 8 + 4 hf .. + 3, of dim 32 dt + c. ds_read_b64_tr_b16 hands lane i of a 16-lane group
+ * element i % 4 of the 8 bytes lane 4 t + i / 4 points at, for t = 0..3: so lane i points at row base + i / 4, dims
+ * 4 (i % 4) .. + 3 of its group's 16. */
 __device__ __forceinline__ uint32_t rows_at(int lane) { return 2 * k_lds(lane & 31, lane >> 5); }
 
 __device__ __forceinline__ uint32_t tr_at(int lane) {
@@ -154,6 +134,19 @@ __device__ __forceinline__ bf16x8 tr_operand32(const uint16_t *tile, uint32_t at
 __device__ __forceinline__ void store4(uint16_t *p, const f32x4 &v, float mul) {
     *reinterpret_cast<uint2 *>(p) = uint2{(uint32_t)f32_to_bf16(v[0] * mul) | ((uint32_t)f32_to_bf16(v[1] * mul) << 16),
                                           (uint32_t)f32_to_bf16(v[2] * mul) | ((uint32_t)f32_to_bf16(v[3] * mul) << 16)};
+}
+
+/* The schedule of N products in source order, each with the READS LDS reads of its row or transposed operand four products
+ * ahead (two to four measured the same in the dK/dV kernel, six 3 % slower). Left to itself the compiler read an operand
+ * right before its product. */
+template <int N, int READS>
+__device__ __forceinline__ void products_in_order() {
+    __builtin_amdgcn_sched_group_barrier(0x100, 4 * READS, 0);
+#pragma unroll
+    for (int m = 0; m < N; m++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if (m < N - 4) __builtin_amdgcn_sched_group_barrier(0x100, READS, 0);
+    }
 }
 
 struct FaState {
@@ -182,13 +175,7 @@ __device__ __forceinline__ void fa_block(const FlashFwd &a, const FaStage &s, co
     for (int kt = 0; kt < 2; kt++)
 #pragma unroll
         for (int cc = 0; cc < 8; cc++) sc[kt] = mfma32x32x16(rows_operand32(s.k, rat, kt, cc), qb[cc], sc[kt]);
-    /* tile 0's scores, then tile 1's, each operand read four products ahead */
-    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-#pragma unroll
-    for (int m = 0; m < 16; m++) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        if (m < 12) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-    }
+    products_in_order<16, 1>();   /* tile 0's scores, then tile 1's */
     /* raw scores: the scale is positive, so the max of the scaled scores is the scaled max, and it is folded into
      * one FMA per exponential below */
     if (MASKED) {
@@ -228,12 +215,7 @@ __device__ __forceinline__ void fa_block(const FlashFwd &a, const FaStage &s, co
     for (int s2 = 0; s2 < 4; s2++)
 #pragma unroll
         for (int d = 0; d < 4; d++) st.o[d] = mfma32x32x16(tr_operand32(s.v, tat, d, 16 * s2), pv[s2], st.o[d]);
-    __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
-#pragma unroll
-    for (int m = 0; m < 16; m++) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        if (m < 12) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-    }
+    products_in_order<16, 2>();
 }
 
 /* A workgroup's (rank, segment, head) from its place in the launch order: work-groups start in linear order (x,
@@ -541,7 +523,10 @@ struct DqStage {
 };
 
 /* dQ of 128 queries: as the forward, S^T = K Q^T and dP^T = V dO^T with queries as columns, so dS^T feeds
- * dQ^T += K^T dS^T as the B operand with K^T read from a transposed LDS tile. */
+ * dQ^T += K^T dS^T as the B operand with K^T read from a transposed LDS tile. Bound as the forward is. 32 x 32 products
+ * read the same operand bytes as two 16-wide tiles a wave did; they win by the lse and D they start from (a column's two
+ * scalars, so P and dS are one multiplication each) and by skipping 32-key tiles no row sees. The backward's share
+ * of 1 x 8,192 tokens x 6 heads: 499 -> 468 us, 32 x 2,048 x 6 800 -> 781, 8 x 2,048 x 10 with window 512 206 -> 196. */
 __global__ void __launch_bounds__(FA_THREADS, 2) flash_bwd_dq_kernel(FlashBwd a) {
     __shared__ DqStage s0, s1;   /* distinct objects: a read of one never waits for DMA into the other */
     const FaBlock fb = fa_block_order();
@@ -551,36 +536,34 @@ __global__ void __launch_bounds__(FA_THREADS, 2) flash_bwd_dq_kernel(FlashBwd a)
     const int tile = (int)gridDim.x - 1 - fb.rank;
     const int qa = tile * FA_BM;
     if (seglen <= 0 || qa >= seglen) return;
-    const int t = threadIdx.x, lane = t & (WAVE - 1), wave = t >> 6, g = lane >> 4, c = lane & 15;
+    const int t = threadIdx.x, lane = t & (WAVE - 1), hf = lane >> 5, c = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);   /* in a scalar register, as are the bounds made of it */
     const int qb = min(qa + FA_BM, seglen) - 1;
     const int q0 = qa + wave * 32;
     const bool active = q0 < seglen;
     const int qw1 = min(q0 + 31, seglen - 1);
 
-    /* queries and dO as B operands (lane (g, c): dims 32 cc + 8 g .. +7 of row c), each column's lse and D */
-    bf16x8 qb_[2][4], ob_[2][4];
-    float lse2[2], dd[2];
+    /* queries and dO as B operands (lane (hf, c): dims 16 cc + 8 hf .. +7 of row c); the column's -lse / scale and -D,
+     * from which its S and dP products start */
+    bf16x8 qb_[8], ob_[8];
+    float nlse, nd;
     {
         const int n = active ? min(32, seglen - q0) : 0;
         const Rsrc rq = rows_rsrc(a.q, start + q0, a.q_stride, h, n), ro = rows_rsrc(a.dout, start + q0, a.do_stride, h, n);
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-#pragma unroll
-            for (int cc = 0; cc < 4; cc++) {
-                qb_[j][cc] = __builtin_bit_cast(bf16x8, bload(rq, (int)(((16 * j + c) * a.q_stride + cc * 32 + g * 8) * 2)));
-                ob_[j][cc] = __builtin_bit_cast(bf16x8, bload(ro, (int)(((16 * j + c) * a.do_stride + cc * 32 + g * 8) * 2)));
-            }
-            const int row = q0 + 16 * j + c;
-            const bool ok = active && row < seglen;
-            lse2[j] = ok ? a.lse[(long long)h * a.lse_stride + start + row] * FA_LOG2E : INFINITY;
-            dd[j] = ok ? a.dpsum[(start + row) * a.H + h] : 0.0f;
+        for (int cc = 0; cc < 8; cc++) {
+            qb_[cc] = __builtin_bit_cast(bf16x8, bload(rq, (int)((c * a.q_stride + cc * 16 + hf * 8) * 2)));
+            ob_[cc] = __builtin_bit_cast(bf16x8, bload(ro, (int)((c * a.do_stride + cc * 16 + hf * 8) * 2)));
         }
+        const bool ok = c < n;
+        nlse = ok ? a.lse[(long long)h * a.lse_stride + start + q0 + c] * (-FA_LOG2E / a.scale_log2) : -INFINITY;
+        nd = ok ? -a.dpsum[(start + q0 + c) * a.H + h] : 0.0f;
     }
-    f32x4 dq[2][8];
+    f32x16 dq[4];
 #pragma unroll
-    for (int j = 0; j < 2; j++)
+    for (int d = 0; d < 4; d++)
 #pragma unroll
-        for (int d = 0; d < 8; d++) dq[j][d] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int i = 0; i < 16; i++) dq[d][i] = 0.0f;
 
     const int klo = a.window >= 0 ? max(0, qa - a.window) : 0;
     /* key block kb + 1 (K and V by LDS DMA) is fetched into the other stage while block kb is computed */
@@ -589,52 +572,46 @@ __global__ void __launch_bounds__(FA_THREADS, 2) flash_bwd_dq_kernel(FlashBwd a)
         tile_dma(a.k, start + kb * FA_BN, a.k_stride, h, nk, stg.k, wave, lane);
         tile_dma(a.v, start + kb * FA_BN, a.v_stride, h, nk, stg.v, wave, lane);
     };
+    uint32_t rat = rows_at(lane), tat = tr_at(lane);
     auto compute = [&](int kb, const DqStage &s) {
         if (!active) return;
-        const int k0 = kb * FA_BN, k1 = k0 + FA_BN - 1;
-        const bool interior = k1 <= q0 && k1 < seglen && (a.window < 0 || qw1 - k0 <= a.window);
-        /* k-step s2 (key tiles 2 s2, 2 s2 + 1): its dS^T half is formed, then consumed by the dQ products at once, so
-         * only one half is ever live; each dq element still adds k-step 0, then 1 */
 #pragma unroll
-        for (int s2 = 0; s2 < 2; s2++) {
+        for (int kt = 0; kt < 2; kt++) {
+            asm volatile("" : "+v"(rat), "+v"(tat));   /* operand addresses are made here, not held across the loop */
+            const int k0 = kb * FA_BN + 32 * kt, k1 = k0 + 31;
+            if (k0 > qw1 || (a.window >= 0 && q0 - k1 > a.window)) continue;   /* no row sees the keys */
+            const bool interior = k1 <= q0 && k1 < seglen && (a.window < 0 || qw1 - k0 <= a.window);
+            f32x16 sc, dp;
+#pragma unroll
+            for (int i = 0; i < 16; i++) { sc[i] = nlse; dp[i] = nd; }
+#pragma unroll
+            for (int cc = 0; cc < 8; cc++) {
+                sc = mfma32x32x16(rows_operand32(s.k, rat, kt, cc), qb_[cc], sc);
+                dp = mfma32x32x16(rows_operand32(s.v, rat, kt, cc), ob_[cc], dp);
+            }
+            products_in_order<16, 1>();
+            /* lane (hf, c): query column c, keys k0 + 8 j + 4 hf + i; only a tile on the diagonal, the window edge or the
+             * segment end tests each pair (interior is uniform: one scalar branch) */
             bf16x8 db[2];
+            auto pds = [&](bool masked) {
 #pragma unroll
-            for (int kk = 0; kk < 2; kk++) {
-                const int kt = 2 * s2 + kk;
-                f32x4 sc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}}, dp[2] = {sc[0], sc[1]};
-#pragma unroll
-                for (int cc = 0; cc < 4; cc++) {
-                    const bf16x8 kop = rows_operand(s.k, kt, cc, g, c), vop = rows_operand(s.v, kt, cc, g, c);
-#pragma unroll
-                    for (int j = 0; j < 2; j++) {
-                        sc[j] = mfma16x16x32(kop, qb_[j][cc], sc[j]);
-                        dp[j] = mfma16x16x32(vop, ob_[j][cc], dp[j]);
-                    }
+                for (int i = 0; i < 16; i++) {
+                    const float e = __builtin_amdgcn_exp2f(sc[i] * a.scale_log2);
+                    const float p =
+                        !masked || visible(k0 + 8 * (i >> 2) + 4 * hf + (i & 3), q0 + c, seglen, a.window) ? e : 0.0f;
+                    db[i >> 3][i & 7] = (__bf16)(p * dp[i]);
                 }
-                /* lane (g, c): query column c of tile j, keys k0 + 16 kt + 4 g + i; only a block on the diagonal, the
-                 * window edge or the segment end tests each pair (interior is uniform: one scalar branch) */
-                auto pds = [&](bool masked) {
+            };
+            if (interior)
+                pds(false);
+            else
+                pds(true);
 #pragma unroll
-                    for (int j = 0; j < 2; j++)
+            for (int s2 = 0; s2 < 2; s2++)
 #pragma unroll
-                        for (int i = 0; i < 4; i++) {
-                            const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[j][i], a.scale_log2, -lse2[j]));
-                            const float p =
-                                !masked || visible(k0 + 16 * kt + 4 * g + i, q0 + 16 * j + c, seglen, a.window) ? e : 0.0f;
-                            db[j][kk * 4 + i] = (__bf16)(p * (dp[j][i] - dd[j]));
-                        }
-                };
-                if (interior)
-                    pds(false);
-                else
-                    pds(true);
-            }
-#pragma unroll
-            for (int d = 0; d < 8; d++) {
-                const bf16x8 kop = tr_operand(s.k, d, s2, g, c);
-#pragma unroll
-                for (int j = 0; j < 2; j++) dq[j][d] = mfma16x16x32(kop, db[j], dq[j][d]);
-            }
+                for (int d = 0; d < 4; d++)
+                    dq[d] = mfma32x32x16(tr_operand32(s.k, tat, d, 32 * kt + 16 * s2), db[s2], dq[d]);
+            products_in_order<8, 2>();
         }
     };
     const int kb_lo = klo / FA_BN, kb_hi = qb / FA_BN;
@@ -649,15 +626,13 @@ __global__ void __launch_bounds__(FA_THREADS, 2) flash_bwd_dq_kernel(FlashBwd a)
         compute(kb + 1, s1);
         __syncthreads();
     }
-    if (!active) return;
+    if (!active || q0 + c >= seglen) return;
+    uint16_t *p = a.dq + (start + q0 + c) * a.dq_stride + (long long)h * HEAD_DIM + 4 * hf;
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int row = q0 + 16 * j + c;
-        if (row >= seglen) continue;
-        uint16_t *p = a.dq + (start + row) * a.dq_stride + (long long)h * HEAD_DIM + 4 * g;
+    for (int d = 0; d < 4; d++)
 #pragma unroll
-        for (int d = 0; d < 8; d++) store4(p + d * 16, dq[j][d], a.scale);
-    }
+        for (int j = 0; j < 4; j++)
+            store4(p + d * 32 + 8 * j, f32x4{dq[d][4 * j], dq[d][4 * j + 1], dq[d][4 * j + 2], dq[d][4 * j + 3]}, a.scale);
 }
 
 /* D[row][h] = sum_d dO . O in fp32, bound by HBM (512 bytes a row): 16 lanes a (row, head), eight consecutive dims a lane by

@@ -120,8 +120,8 @@ def test_backward_matches_oracle(device, lengths, H, window):
 
 @pytest.mark.parametrize("scale", [None, 1e-39])
 @pytest.mark.parametrize("window", [None, 0, 1, 31, 32, 33, 95])
-def test_key_gradients_at_tile_edges(device, window, scale):
-    """dK, dV around the 32 x 32 tiles' edges (keys a wave, rows a tile, keys a workgroup), window ends inside and on a
+def test_gradients_at_tile_edges(device, window, scale):
+    """dQ, dK, dV around the 32 x 32 tiles' edges (keys or rows a wave, rows or keys a tile, a workgroup), window ends inside and on a
     tile, and a scale whose lse / scale would overflow (every weight then 1 / the row's keys). Each against float64 from
     the same inputs within one bf16 rounding (8 significant bits: 2^-8) of each term's P or dS and one of the result, and
     2^-16 of the terms' magnitudes for the fp32 lse, exponentials and sums."""
@@ -131,9 +131,9 @@ def test_key_gradients_at_tile_edges(device, window, scale):
     qd, kd, vd, dod, cud = (t.to(device) for t in (q, k, v, dout, cu))
     out, lse = flash_attn_fwd(qd, kd, vd, cud, max(lengths), window_left=window, softmax_scale=scale)
     rows = flash_attn_bwd_rows(out, dod)
-    _, dk, dv = flash_attn_bwd(qd, kd, vd, out, dod, lse, cud, max(lengths), rows=rows, window_left=window,
+    dq, dk, dv = flash_attn_bwd(qd, kd, vd, out, dod, lse, cud, max(lengths), rows=rows, window_left=window,
                                softmax_scale=scale)
-    rows, dk, dv = (t.double().cpu() for t in (rows, dk, dv))
+    rows, dq, dk, dv = (t.double().cpu() for t in (rows, dq, dk, dv))
     sc = 128 ** -0.5 if scale is None else scale
     for s, e in zip(cu[:-1].tolist(), cu[1:].tolist()):
         Q, K, V, dO = (t[s:e, 0].double() for t in (q, k, v, dout))
@@ -143,7 +143,8 @@ def test_key_gradients_at_tile_edges(device, window, scale):
         dP = dO @ V.T
         dS = P * (dP - rows[s:e])
         mag = P * (dP.abs() + (dO.abs() @ V.abs().T) + rows[s:e].abs())
-        for got, want, terms in ((dv[s:e, 0], P.T @ dO, P.T @ dO.abs()), (dk[s:e, 0], sc * dS.T @ Q, sc * mag.T @ Q.abs())):
+        for got, want, terms in ((dv[s:e, 0], P.T @ dO, P.T @ dO.abs()), (dk[s:e, 0], sc * dS.T @ Q, sc * mag.T @ Q.abs()),
+                                 (dq[s:e, 0], sc * dS @ K, sc * mag @ K.abs())):
             tol = 2.0 ** -8 * want.abs() + (2.0 ** -8 + 2.0 ** -16) * terms + 2.0 ** -133
             assert bool(((got - want).abs() <= tol).all()), (s, e, float(((got - want).abs() / tol).max()))
 

@@ -172,6 +172,26 @@ def test_backward_rows_and_strided_dv(device):
         rel_check(got.float().cpu().numpy(), ref)
 
 
+@pytest.mark.parametrize("lengths,H", [([256] * 16, 8), ([300] * 30, 3), ([130, 300, 257] * 20, 3)])
+def test_every_tile_is_taken_once(device, lengths, H):
+    """256 workgroups (one per CU), 270 (some in the reversed second round) and 540 (a third round): every segment and
+    head gives the bits it gives in a call of its own."""
+    q, k, v, cu, _ = make(lengths, H, seed=len(lengths))
+    dout = torch.randn(q.shape, generator=torch.Generator().manual_seed(6)).bfloat16()
+
+    def both(q, k, v, dout, cu, longest):
+        out, lse = flash_attn_fwd(q, k, v, cu, longest)
+        return (out, lse.t()) + tuple(flash_attn_bwd(q, k, v, out, dout, lse, cu, longest))
+
+    qd, kd, vd, dod = (t.to(device) for t in (q, k, v, dout))
+    full = both(qd, kd, vd, dod, cu.to(device), max(lengths))
+    for s, e in list(zip(cu[:-1].tolist(), cu[1:].tolist())):
+        one = both(*(t[s:e].contiguous() for t in (qd, kd, vd, dod)),
+                   torch.tensor([0, e - s], dtype=torch.int32, device=device), e - s)
+        for a, b in zip(full, one):
+            assert torch.equal(a[s:e], b), (s, e)
+
+
 def test_backward_training_shape_against_autograd(device):
     """One 2048-token segment, 6 heads: gradients against float32 autograd of causal SDPA on the GPU."""
     gen = torch.Generator().manual_seed(12)

@@ -12,9 +12,8 @@
  * fragments already in registers, and between them reads the next stage's 4 weight and 8 activation fragments (one
  * 16-byte LDS read each) into a second register set. Lane (g, i) of a
  * result tile holds columns n .. n + 3 (n = 16 t + 4 g) of row m = 16 u + i, and every epilogue writes 4 adjacent
- * columns of a row. In LDS a row's 64 bytes (4 blocks of 16) keep block b at position b ^ ((row / 4) % 4), so the 16
- * rows of a fragment read fall in distinct banks; each DMA lane fetches the global block that belongs at its LDS
- * position.
+ * columns of a row. In LDS a row's 64 bytes (4 blocks of 16) keep block b at position b ^ pg_swizzle(row), so a fragment
+ * read meets no bank conflicts; each DMA lane fetches the global block that belongs at its LDS position.
  *
  * Workgroups take their tiles in an XCD-aware order (pg_order), so the workgroups an XCD runs together share operand
  * tiles in its L2. The tiles that would leave the last (or only) round of workgroups part-filled (T mod CUs of T tiles) are
@@ -72,9 +71,17 @@ __device__ __forceinline__ Rsrc pg_rsrc(const void *p, long long bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes, 0x00020000);
 }
 
+/* Four rows lie side by side over the 64 banks, so the block's place among its row's four depends on row / 4. A 16-byte
+ * LDS read is served 16 lanes at a time: lanes 0-3, 12-15, 20-23 and 24-27, then 4-7, 8-11, 16-19 and 28-31, and the
+ * same of the upper half. Of a fragment read (lane 16 g + i: row i, block g) those are rows 0-3 and 12-15 of one block
+ * with 4-11 of its neighbour, and the negated row / 4 puts the four groups in four places. With row / 4 itself they met
+ * in pairs: every read took 8 cycles, not 4 (o of d1664 at 150 rows 18.6 -> 15.8 us, fc
+ * at 150 rows 19.7 -> 16.8, d768 proj 30.8 -> 25.3; whole tiles, which wait for little, 1-2 %). */
+__device__ __forceinline__ int pg_swizzle(int row) { return -(row >> 2) & 3; }
+
 /* Stage j's DMA into buf (j >= stages: offsets past the range, zeros and no memory access). Instruction q fills the
  * buffer's rows 16 q .. 16 q + 15 (rows below TM: a rows m0 + r; the rest: w rows n0 + r - TM); lane l writes row
- * 16 q + l / 4 at position l % 4 and fetches the global block (l % 4) ^ ((row / 4) % 4). Wave w issues q = w, w + 8,
+ * 16 q + l / 4 at position l % 4 and fetches the global block (l % 4) ^ pg_swizzle(row). Wave w issues q = w, w + 8,
  * ... (its first A_LOADS are a's). */
 template <class P>
 __device__ __forceinline__ void pg_fetch(Rsrc ra, Rsrc rw, unsigned char *buf, int j, int stages, int m0, int n0,
@@ -86,7 +93,7 @@ __device__ __forceinline__ void pg_fetch(Rsrc ra, Rsrc rw, unsigned char *buf, i
         const int q = wave + PG_WAVES * s, row = 16 * q + (lane >> 2);
         const bool is_a = s < P::A_LOADS;
         const int grow = (is_a ? m0 : n0 - P::TM) + row;
-        const int off = live ? grow * rowb + kb + ((pos ^ ((row >> 2) & 3)) << 4) : PG_PAST;
+        const int off = live ? grow * rowb + kb + ((pos ^ pg_swizzle(row)) << 4) : PG_PAST;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(is_a ? ra : rw, (LdsPtr *)(buf + q * 1024), 16, off, 0, 0, 0);
     }
 }
@@ -127,7 +134,7 @@ __device__ __forceinline__ void pg_mfma(f32x4 &c, const bf16x8 &a, const bf16x8 
  * 16, so rows 16 f on from it have the same swizzle and fragment f lies 16 f rows = 1 KiB further on). */
 __device__ __forceinline__ uint32_t pg_base(const unsigned char *buf, int row0, int i16, int grp) {
     const int row = row0 + i16;
-    const LdsPtr *p = (const LdsPtr *)(buf + row * PG_ROWB + ((grp ^ ((row >> 2) & 3)) << 4));
+    const LdsPtr *p = (const LdsPtr *)(buf + row * PG_ROWB + ((grp ^ pg_swizzle(row)) << 4));
     return (uint32_t)reinterpret_cast<uintptr_t>(p);
 }
 

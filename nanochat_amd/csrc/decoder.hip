@@ -8,8 +8,9 @@
  *          attention.hip), o GEMM (+ residual: the bf16 rounding of the fp32 sum, and each 16-row tile's sum of
  *          squares), fc GEMM (+ ReLU^2 of the sum scaled by the rstd it takes from those tile sums), proj GEMM
  *          (K-slice partials), proj_norm_kernel (the partials + residual, then the next layer's residual norm) }
- *   head   norm_kernel(FINAL), lm_head GEMM (fp32 logits; prefill_gemm.hip's tiled kernel), choose_kernel (greedy,
- *          Gumbel-max or nucleus choice within the allowed tokens, then the commit), the tokens to pinned host memory.
+ *   head   norm_kernel(FINAL), lm_head GEMM (fp32 logits; prefill_gemm.hip's tiled kernel), choose_kernel (greedy
+ *          choice within the allowed tokens, nucleus thresholds), sample_kernel where a slot is sampled (Gumbel-max over
+ *          many blocks a slot), each with the commit of its slots; the tokens to pinned host memory.
  * A step's GEMMs are slot_gemm.hip's weight-streaming MFMA kernel with the epilogue fused (long-K GEMMs split into
  * K-slices whose partials a second kernel adds in order; a model wider than 2,048 computes the MLP's rstd in
  * rstd_kernel). Prefill's GEMMs (up to 16,384 rows a call) are prefill_gemm.hip's MFMA-tiled kernel over all the
@@ -353,7 +354,26 @@ struct ChoiceArgs {
     int32_t *tokens, *alt_tokens, *pos;
     float softcap;
     int vocab, lazy;
+    uint32_t *cut;              /* [B]: a nucleus slot's threshold, from choose_kernel to sample_kernel */
+    unsigned long long *keys;   /* [B][2]: the best and the alternative key of sample_kernel's blocks so far; 0 between calls */
+    int32_t *arrived;           /* [B]: its blocks that have added theirs; 0 between calls */
 };
+
+/* The end of slot b's choice (one thread): tokens of the two keys, key 0 (nothing allowed) giving -1. */
+__device__ __forceinline__ void commit_choice(const ChoiceArgs &c, int b, unsigned long long best, unsigned long long alt) {
+    c.tokens[b] = (int32_t)(0xFFFFFFFFu - (uint32_t)best);
+    c.alt_tokens[b] = (int32_t)(0xFFFFFFFFu - (uint32_t)alt);
+    c.pos[b] += 1;
+}
+
+__device__ __forceinline__ bool row_allowed(const uint32_t *allow, bool masked, int r) {
+    return !masked || ((allow[r / WORD_BITS] >> (r % WORD_BITS)) & 1u);
+}
+
+/* z / T of a logit, z = c tanh(s / c) */
+__device__ __forceinline__ float capped_over_t(const ChoiceArgs &c, float s, float T) {
+    return c.softcap * tanhf(s / c.softcap) / T;
+}
 
 /* Block reductions: the wave butterfly, then the waves in order; every thread gets the result. */
 __device__ float block_max(float v, float *scratch) {
@@ -477,10 +497,9 @@ __global__ void __launch_bounds__(CHOICE_THREADS) nucleus_cut_kernel(const float
     if (threadIdx.x == 0) cut[blockIdx.x] = u;
 }
 
-/* A block per slot: its token among the allowed rows of its logits, then the commit (decode.cu:170-229, 361-411,
- * 677-688). Temperature 0: the largest logit. T > 0: the largest z / T + gumbel, z = c tanh(s / c) (Gumbel-max
- * sampling of softmax(z / T)). T > 0 and top_p < 1: Gumbel-max within the nucleus that nucleus_cut fixes. The
- * alternative is the best key but the lazy row's (none for a nucleus slot). */
+/* A block per slot: a greedy slot's token among the allowed rows of its logits, then the commit (decode.cu:170-229,
+ * 361-411, 677-688): the largest logit, the alternative being the best but the lazy row. A nucleus slot (T > 0 and
+ * top_p < 1) gets its probabilities and threshold here, for sample_kernel; any other sampled slot is sample_kernel's. */
 __global__ void __launch_bounds__(CHOICE_THREADS) choose_kernel(ChoiceArgs c) {
     __shared__ float fscratch[CHOICE_WAVES];
     __shared__ unsigned long long kscratch[CHOICE_WAVES];
@@ -491,52 +510,89 @@ __global__ void __launch_bounds__(CHOICE_THREADS) choose_kernel(ChoiceArgs c) {
     const float T = c.temperature[b], top_p = c.top_p[b];
     const bool masked = live(c.active + MASK_WORDS, b);
     const uint32_t *allow = c.allow + (long long)b * (c.vocab / WORD_BITS);
-    const int gen = c.pos[b] - c.first[b];
-    const unsigned long long seed = c.seed[b];
-    auto allowed = [&](int r) { return !masked || ((allow[r / WORD_BITS] >> (r % WORD_BITS)) & 1u); };
-    auto capped = [&](int r) { return c.softcap * tanhf(s[r] / c.softcap); };
-    unsigned long long best = 0, alt = 0;
-    if (T > 0.0f && top_p < 1.0f) {
-        /* the slot's probabilities go to its row of c.probs; every pass over them visits a thread's own rows */
+    if (T > 0.0f) {
+        if (!(top_p < 1.0f)) return;
+        /* the slot's probabilities go to its row of c.probs; every pass over them here visits a thread's own rows */
         float *prob = c.probs + (long long)b * c.vocab;
         float zmax = -INFINITY;
         for (int r = tid; r < c.vocab; r += CHOICE_THREADS)
-            if (allowed(r)) zmax = fmaxf(zmax, capped(r) / T);
+            if (row_allowed(allow, masked, r)) zmax = fmaxf(zmax, capped_over_t(c, s[r], T));
         zmax = block_max(zmax, fscratch);
-        for (int r = tid; r < c.vocab; r += CHOICE_THREADS) prob[r] = allowed(r) ? expf(capped(r) / T - zmax) : 0.0f;
+        for (int r = tid; r < c.vocab; r += CHOICE_THREADS)
+            prob[r] = row_allowed(allow, masked, r) ? expf(capped_over_t(c, s[r], T) - zmax) : 0.0f;
         const uint32_t cut = nucleus_cut(prob, c.vocab, top_p, nucleus);
-        for (int r = tid; r < c.vocab; r += CHOICE_THREADS) {
-            const float pr = prob[r];
-            if (pr == 0.0f || __float_as_uint(pr) < cut) continue;
-            const unsigned long long key = choice_key(capped(r) / T + gumbel(seed, gen, r), r);
-            best = key > best ? key : best;
-        }
-    } else {
-        /* four logits a thread a step by 16-byte reads, four reads in flight (the vocab is a multiple of 32); the result
-         * is a maximum over keys unique per row, so the visiting order does not matter */
-        const float4 *s4 = reinterpret_cast<const float4 *>(s);
+        if (tid == 0) c.cut[b] = cut;
+        return;
+    }
+    unsigned long long best = 0, alt = 0;
+    /* four logits a thread a step by 16-byte reads, four reads in flight (the vocab is a multiple of 32); the result
+     * is a maximum over keys unique per row, so the visiting order does not matter */
+    const float4 *s4 = reinterpret_cast<const float4 *>(s);
 #pragma unroll 4
-        for (int q = tid; q < c.vocab / 4; q += CHOICE_THREADS) {
-            const float4 v4 = s4[q];
-            const float v[4] = {v4.x, v4.y, v4.z, v4.w};
+    for (int q = tid; q < c.vocab / 4; q += CHOICE_THREADS) {
+        const float4 v4 = s4[q];
+        const float v[4] = {v4.x, v4.y, v4.z, v4.w};
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int r = 4 * q + e;
-                if (!allowed(r)) continue;
-                const float score = T > 0.0f ? c.softcap * tanhf(v[e] / c.softcap) / T + gumbel(seed, gen, r) : v[e];
-                const unsigned long long key = choice_key(score, r);
-                best = key > best ? key : best;
-                if (r != c.lazy) alt = key > alt ? key : alt;
-            }
+        for (int e = 0; e < 4; e++) {
+            const int r = 4 * q + e;
+            if (!row_allowed(allow, masked, r)) continue;
+            const unsigned long long key = choice_key(v[e], r);
+            best = key > best ? key : best;
+            if (r != c.lazy) alt = key > alt ? key : alt;
         }
     }
     best = block_max_key(best, kscratch);
     alt = block_max_key(alt, kscratch);
-    if (tid == 0) {
-        c.tokens[b] = (int32_t)(0xFFFFFFFFu - (uint32_t)best);   /* key 0 (nothing allowed) gives -1 */
-        c.alt_tokens[b] = (int32_t)(0xFFFFFFFFu - (uint32_t)alt);
-        c.pos[b] += 1;
+    if (tid == 0) commit_choice(c, b, best, alt);
+}
+
+/* The sampled slots' tokens (T > 0), SAMPLE_SPLIT blocks a slot: the row with the largest z / T + gumbel among the allowed
+ * rows (Gumbel-max sampling of softmax(z / T)), or among those a nucleus slot's threshold keeps (no alternative then).
+ * A row costs a Philox block and two fp64 logarithms, about 2 us for a block of 1,024 rows, so one block a slot took
+ * 135 us of a vocabulary of 65,536 (12 layers of d768, a step of 4 sampled slots 580 -> 460 us, with a nucleus 716 -> 596,
+ * of 128 sampled slots 728 -> 687; the same greedy steps 460 and 605). A block adds its best keys to the slot's by agent-scope maxima and then counts itself; the last to
+ * count takes the keys, clears them for the next call and commits. Keys are unique per row, so the order does not
+ * matter. Launched only where a slot is sampled. */
+constexpr int SAMPLE_SPLIT = 16;
+
+__global__ void __launch_bounds__(CHOICE_THREADS) sample_kernel(ChoiceArgs c) {
+    __shared__ unsigned long long kscratch[CHOICE_WAVES];
+    const int b = blockIdx.y, tid = threadIdx.x;
+    const float T = c.temperature[b];
+    if (!live(c.active, b) || !(T > 0.0f)) return;
+    const float *s = c.logits + (long long)b * c.vocab, *prob = c.probs + (long long)b * c.vocab;
+    const bool masked = live(c.active + MASK_WORDS, b), kept = c.top_p[b] < 1.0f;
+    const uint32_t *allow = c.allow + (long long)b * (c.vocab / WORD_BITS);
+    const uint32_t cut = kept ? c.cut[b] : 0u;
+    const int gen = c.pos[b] - c.first[b];
+    const unsigned long long seed = c.seed[b];
+    unsigned long long best = 0, alt = 0;
+    for (int r = blockIdx.x * CHOICE_THREADS + tid; r < c.vocab; r += SAMPLE_SPLIT * CHOICE_THREADS) {
+        if (kept) {
+            const float pr = prob[r];
+            if (pr == 0.0f || __float_as_uint(pr) < cut) continue;
+        } else if (!row_allowed(allow, masked, r)) {
+            continue;
+        }
+        const unsigned long long key = choice_key(capped_over_t(c, s[r], T) + gumbel(seed, gen, r), r);
+        best = key > best ? key : best;
+        if (!kept && r != c.lazy) alt = key > alt ? key : alt;
     }
+    best = block_max_key(best, kscratch);
+    alt = block_max_key(alt, kscratch);
+    if (tid != 0) return;
+    unsigned long long *keys = c.keys + 2 * b;
+    __hip_atomic_fetch_max(keys, best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_fetch_max(keys + 1, alt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0);   /* both maxima have reached the coherent level before the block is counted */
+    asm volatile("" ::: "memory");
+    const int prior = __hip_atomic_fetch_add(c.arrived + b, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (prior != SAMPLE_SPLIT - 1) return;
+    best = __hip_atomic_exchange(keys, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    alt = __hip_atomic_exchange(keys + 1, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(c.arrived + b, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    commit_choice(c, b, best, alt);
 }
 
 /* ---------------------------------------------------------------- small state kernels */
@@ -675,7 +731,11 @@ struct Decoder {
     std::vector<int32_t> hpos;           /* host copy of pos: the position a live slot's next step writes */
     std::vector<unsigned long long> live;  /* host copy of the live-slot mask of dec_set_active */
     int32_t *tokens, *alt_tokens, *pos, *first, *seq_lens, *num_new;  /* [B] */
+    std::vector<bool> sampled;           /* host copy of temperature > 0 */
     float *temperature, *top_p;
+    uint32_t *cut;                       /* [B], with keys [B][2] and arrived [B]: ChoiceArgs */
+    unsigned long long *keys;
+    int32_t *arrived;
     unsigned long long *seed;
     unsigned long long *active;          /* [2][MASK_WORDS] */
     uint32_t *allow;                     /* [B][vocab / 32] */
@@ -1021,8 +1081,11 @@ static void enqueue_head(Decoder *d) {
             gemm_epi(d, d->lane[0], true, SG_F32, d->lm_head, d->vocab, d->C, a.hn, R, nullptr, d->logits, nullptr,
                      nullptr, d->active);
         ChoiceArgs c = {d->logits, d->probs, d->active, d->allow, d->temperature, d->top_p, d->seed, d->first,
-                        d->tokens, d->alt_tokens, d->pos, d->softcap, d->vocab, d->lazy};
+                        d->tokens, d->alt_tokens, d->pos, d->softcap, d->vocab, d->lazy, d->cut, d->keys, d->arrived};
         hipLaunchKernelGGL(choose_kernel, dim3(R), dim3(CHOICE_THREADS), 0, d->stream, c);
+        bool sampled = false;
+        for (int b = 0; b < R; b++) sampled |= d->sampled[b];
+        if (sampled) hipLaunchKernelGGL(sample_kernel, dim3(SAMPLE_SPLIT, R), dim3(CHOICE_THREADS), 0, d->stream, c);
     }
     HIP_CHECK(hipMemcpyAsync(d->host_tokens, d->tokens, (size_t)d->B * 4, hipMemcpyDeviceToHost, d->stream));
     HIP_CHECK(hipMemcpyAsync(d->host_tokens + d->B, d->alt_tokens, (size_t)d->B * 4, hipMemcpyDeviceToHost, d->stream));
@@ -1112,6 +1175,10 @@ static Decoder *create(const int *cfg, const uint64_t *ptrs, const float *scal, 
     d->seq_lens = state + 4 * B; d->num_new = state + 5 * B;
     d->temperature = (float *)device_alloc(d, B * sizeof(float));
     d->top_p = (float *)device_alloc(d, B * sizeof(float));
+    d->sampled.assign(d->B, false);
+    d->cut = (uint32_t *)device_alloc(d, B * sizeof(uint32_t));
+    d->keys = (unsigned long long *)device_alloc(d, 2 * B * sizeof(unsigned long long));
+    d->arrived = (int32_t *)device_alloc(d, B * sizeof(int32_t));
     d->seed = (unsigned long long *)device_alloc(d, B * sizeof(unsigned long long));
     d->allow = (uint32_t *)device_alloc(d, B * (d->vocab / WORD_BITS) * sizeof(uint32_t));
     d->logits = (float *)device_alloc(d, B * d->vocab * sizeof(float));
@@ -1443,6 +1510,7 @@ extern "C" void dec_set_prompt(void *handle, int b, int32_t token, int32_t last,
                        d->temperature, d->top_p, d->seed, b, token, last, temperature, top_p, seed);
     HIP_CHECK(hipGetLastError());
     d->hpos[b] = last;
+    d->sampled[b] = temperature > 0.0f;
     nc::dec::release_pages(d, b, last / nc::PAGE + 1);   /* pages past the slot's position hold an older sequence */
     nc::dec::flush_table(d);
 }

@@ -310,6 +310,42 @@ def test_sampling_matches_oracle_choice(device):
         dec.close()
 
 
+@pytest.mark.parametrize("vocab", [1024, 16352, 16416, 50016])
+def test_split_sampling_matches_oracle_choice(device, vocab):
+    """The sampled slots' rows over 16 blocks of 1,024: one block with rows, the last one short, a second turn, and a
+    vocabulary of several turns; greedy, plain and nucleus slots side by side, over steps (the blocks' shared keys are
+    cleared for the next)."""
+    m = model_tensors(1, 256, 1024, vocab, 64, seed=3, std=0.05, theta=10000.0, ve_layers=(), windows=[64], device=device)
+    params = [(0.9, 1.0, 7), (0.7, 0.8, 11), (0.0, 1.0, 1), (1.7, 1.0, 2 ** 63 + 5)]
+    dec = DecoderRuntime(m, bos_token_id=0, max_length=64, prompt_store=0, max_slots=8)
+    try:
+        for b, ids in enumerate(prompts([10, 14, 18, 22], vocab, seed=5)):
+            dec.place(b, ids, temperature=params[b][0], top_p=params[b][1], seed=params[b][2])
+        dec.prefill()
+        dec.activate(range(4))
+        for step in range(3):
+            tokens, got = dec.step(), dec.logits(4)
+            for b, (T, p, seed) in enumerate(params):
+                tok, alt = sampling.choose(got[b], temperature=T, top_p=p, seed=seed, gen=step, lazy=0, softcap=m.softcap)
+                if T == 0:
+                    assert tokens[b] == tok and dec.alternatives[b] == alt
+                    continue
+                z = sampling.capped(got[b], m.softcap)
+                scores = (z / np.float32(T)).astype(np.float32) + sampling.gumbel(seed, step, np.arange(vocab))
+                if p < 1:
+                    keep, e = sampling.nucleus_keep(z, T, p, np.ones(vocab, bool))
+                    if not keep[tokens[b]]:   # only a row at the nucleus boundary may differ
+                        assert abs(e[tokens[b]] - e[keep].min()) <= 1e-5 * e[keep].min(), (step, b)
+                    else:
+                        assert near_tie_ok(int(tokens[b]), tok, scores), (step, b)
+                    assert dec.alternatives[b] == -1
+                else:
+                    assert near_tie_ok(int(tokens[b]), tok, scores), (step, b)
+                    assert near_tie_ok(int(dec.alternatives[b]), alt, scores), (step, b)
+    finally:
+        dec.close()
+
+
 def test_inactive_slot_holds_still(device):
     m, w, max_length = build(device, "tiny")
     ids = prompts([15, 25, 35], m.vocab, seed=6)

@@ -324,7 +324,7 @@ __global__ void __launch_bounds__(FA_THREADS, 2) flash_fwd_kernel(FlashFwd a) {
  * Backward (the reference's _flash_attn_bwd / bwd_bf16dq, model/ops/flash_attn.py:367-391), per segment and head:
  *   P = exp(scale S - lse), dV = P^T dO, dP = dO V^T, dS = P (dP - D) with D_i = dO_i . O_i (the caller's row
  *   statistics: the reference's `rows`, from the o_proj backward epilogue), dQ = scale dS K, dK = scale dS^T Q.
- * Two kernels and no atomics: flash_bwd_dkv_kernel owns 128 keys (a wave 16) and walks the query blocks that see them;
+ * Two kernels and no atomics: flash_bwd_dkv_kernel owns 128 keys (a wave 32) and walks the query blocks that see them;
  * flash_bwd_dq_kernel owns 128 queries (a wave 32, as the forward) and walks their key blocks. S and dP are computed
  * in both (seven 128-deep products per (query, key) pair instead of five), the price of writing dQ once.
  * ------------------------------------------------------------------------------------------------------------- */
@@ -356,9 +356,9 @@ struct alignas(16) DkvStage {
  * column), so P and dS feed dV^T += dO^T P and dK^T += Q^T dS directly as B operands, with dO^T and Q^T read transposed from
  * the staged tiles. A wave's 32 columns make every operand read from LDS feed twice the products that 16 x 16 tiles of 16
  * keys a wave did: those read 64 KiB a wave and block for 64 products, twice the time of the products themselves.
- * Two blocks of four waves share a CU. At 65,536 tokens of 2,048-token segments x 6 heads dK/dV takes 546 us by trace (16 x 16
- * tiles in blocks of eight waves: 675), the backward 912 -> 810; at 2 x 8,192 tokens 762 -> 690, at 8 x 2,048 x 10 heads with
- * a window of 512 232 -> 208. */
+ * Two blocks of four waves share a CU. At 65,536 tokens of 2,048-token segments x 6 heads dK/dV went from 675 us by trace (16 x
+ * 16 tiles in blocks of eight waves) to 546, and with k_swizzle to 464; the backward with these tiles alone 912 -> 810, at
+ * 2 x 8,192 tokens 762 -> 690, at 8 x 2,048 x 10 heads with a window of 512 232 -> 208. */
 constexpr int DKV_WAVES = 4;
 constexpr int DKV_KEYS = 32 * DKV_WAVES;
 constexpr int DKV_PARKED = 3;   /* K's last operand and V's last two wait in LDS: 256 registers hold the other 13 */

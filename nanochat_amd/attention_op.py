@@ -110,13 +110,24 @@ def _plain(t: Tensor, dtype: torch.dtype, alignment: int) -> bool:
 SSQ_COLS = 32   # columns of one of nc_linear_residual_rms's sums of squares
 
 
+def _projection_fits(x: Tensor, o_weight: Tensor, residual: Tensor) -> bool:
+    """Whether nc_linear_residual_rms may take project's operands: it trusts the sizes it is given, so they are those of
+    all three tensors, on one device."""
+    if x.dim() != 2 or o_weight.dim() != 2:
+        return False
+    (tokens, K), C = x.shape, o_weight.size(0)
+    return (o_weight.size(1) == K and residual.shape == (tokens, C) and x.device == o_weight.device == residual.device
+            and _plain(x, BF16, 16) and _plain(o_weight, BF16, 16) and _plain(residual, BF16, 8)
+            and K % 128 == 0 and C % 4 == 0 and max(C, K) <= 32768)
+
+
 def project(x: Tensor, o_weight: Tensor, residual: Tensor) -> tuple[Tensor, Tensor]:
     """x [tokens, K] bf16 (dense), residual [tokens, C] -> (bf16(x o_weight^T + residual), the fp32 sum's rstd
     [tokens]). Dense bf16 operands of the kernel's sizes (K of 128, C of 4) take one GEMM whose epilogue does all of it
-    (65,536 tokens, C = 768: 350 -> 146 us); anything else a library GEMM and elementwise passes."""
-    tokens, (C, K) = x.size(0), o_weight.shape
-    if (_plain(x, BF16, 16) and _plain(o_weight, BF16, 16) and _plain(residual, BF16, 8) and K % 128 == 0 and C % 4 == 0
-            and residual.shape == (tokens, C) and max(C, K) <= 32768):
+    (65,536 tokens, C = 768: 350 -> 146 us); anything else a library GEMM and elementwise passes, which raise where the
+    sizes or devices do not agree."""
+    if _projection_fits(x, o_weight, residual):
+        (tokens, K), C = x.shape, o_weight.size(0)
         h, rstd = torch.empty_like(residual), x.new_empty(tokens, dtype=F32)
         ssq = x.new_empty(tokens * (-(-C // SSQ_COLS)), dtype=F32)
         check(hip_library().nc_linear_residual_rms(pointer(x), pointer(o_weight), pointer(residual), tokens, C, K,

@@ -91,3 +91,14 @@ def test_operands_the_kernels_do_not_take(device):
     op.add_weight_grad(grad, dd[:0], xd[:0])
     assert bool((grad == 1).all())
     assert op.project(xd[:0], wd, rd[:0])[0].shape == (0, 256)
+
+
+def test_projection_sizes_that_do_not_agree(device):
+    """x of another width than the weight, a residual of other rows or columns: an error, as from the library's product."""
+    x = torch.zeros(70, 256, dtype=torch.bfloat16, device=device)
+    w, res = x.new_zeros(128, 256), x.new_zeros(70, 128)
+    for args in ((x, w[:, :128].contiguous(), res), (x[:, :128].contiguous(), w, res), (x, w, res[:69]),
+                 (x, w, x), (x.view(70, 2, 128), w, res)):
+        with pytest.raises(RuntimeError):
+            op.project(*args)
+    torch.cuda.synchronize()

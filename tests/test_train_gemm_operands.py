@@ -1,0 +1,58 @@
+"""Which operands of the training block's projection and weight gradients reach their HIP kernels, which trust the sizes
+and addresses they are given: without a GPU, CPU tensors stand for device tensors and a kernel call is an exception of its
+own. Operands whose sizes or devices do not agree must meet the library GEMM instead, which raises."""
+import pytest
+import torch
+
+from nanochat_amd import attention_op as op
+
+
+class Reached(BaseException):
+    """A kernel entry point would have been called."""
+
+
+class Library(BaseException):
+    """The library GEMM would have been called."""
+
+
+def library_gemm(*args, **kwargs):
+    raise Library
+
+
+class NoLibrary:
+    def __getattr__(self, name):
+        raise Reached(name)
+
+
+@pytest.fixture(autouse=True)
+def device_operands(monkeypatch):
+    """Every dense aligned tensor counts as a device tensor, and neither kind of product runs."""
+    monkeypatch.setattr(op, "_plain", lambda t, dtype, alignment: (t.dtype == dtype and t.is_contiguous()
+                                                                   and t.data_ptr() % alignment == 0))
+    monkeypatch.setattr(op, "hip_library", NoLibrary)
+    monkeypatch.setattr(op, "stream", lambda: 0)
+    monkeypatch.setattr(torch, "mm", library_gemm)
+
+
+def bf(*shape, device="cpu"):
+    return torch.zeros(*shape, dtype=torch.bfloat16, device=device)
+
+
+def test_agreeing_operands_reach_the_projection():
+    with pytest.raises(Reached):
+        op.project(bf(24, 256), bf(128, 256), bf(24, 128))
+
+
+@pytest.mark.parametrize("x,w,res", [((24, 256), (128, 128), (24, 128)), ((24, 128), (128, 256), (24, 128)),
+                                     ((24, 2, 128), (128, 256), (24, 128)), ((24, 256), (128, 256), (23, 128)),
+                                     ((24, 256), (128, 256), (24, 256)), ((24, 256), (256,), (24, 128))])
+def test_projection_sizes_that_do_not_agree(x, w, res):
+    with pytest.raises(Library):
+        op.project(bf(*x), bf(*w), bf(*res))
+
+
+@pytest.mark.parametrize("elsewhere", [0, 1, 2])
+def test_projection_operands_on_two_devices(elsewhere):
+    args = [bf(*s, device="meta" if i == elsewhere else "cpu") for i, s in enumerate([(24, 256), (128, 256), (24, 128)])]
+    with pytest.raises(Library):
+        op.project(*args)

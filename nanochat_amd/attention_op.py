@@ -139,12 +139,19 @@ def project(x: Tensor, o_weight: Tensor, residual: Tensor) -> tuple[Tensor, Tens
     return total.to(BF16), rstd
 
 
+def _weight_grad_fits(o_grad: Tensor, dh: Tensor, x: Tensor) -> bool:
+    """Whether nc_weight_grad may take add_weight_grad's operands: one number of tokens, one device."""
+    return (dh.dim() == 2 and x.dim() == 2 and dh.size(0) == x.size(0) and o_grad.shape == (dh.size(1), x.size(1))
+            and dh.device == x.device == o_grad.device
+            and _plain(dh, BF16, 16) and _plain(x, BF16, 16) and _plain(o_grad, F32, 16))
+
+
 def add_weight_grad(o_grad: Tensor, dh: Tensor, x: Tensor) -> None:
     """o_grad += dh^T x over the tokens, fp32 sums: dh [tokens, C], x [tokens, K] bf16. Dense 16-byte aligned operands
     take the HIP kernel, which cuts the long sum over the tokens across the chip (65,536 tokens, 768 x 768: 302 -> 111 us);
-    others a library GEMM."""
-    tokens, C, K = dh.size(0), dh.size(1), x.size(1)
-    if _plain(dh, BF16, 16) and _plain(x, BF16, 16) and _plain(o_grad, F32, 16) and o_grad.shape == (C, K):
+    others a library GEMM, which raises where the sizes or devices do not agree."""
+    if _weight_grad_fits(o_grad, dh, x):
+        (tokens, C), K = dh.shape, x.size(1)
         need = hip_library().nc_weight_grad_workspace_bytes(tokens, C, K)
         if need >= 0:
             ws = x.new_empty(need, dtype=torch.uint8)

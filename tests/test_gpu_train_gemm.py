@@ -102,3 +102,14 @@ def test_projection_sizes_that_do_not_agree(device):
         with pytest.raises(RuntimeError):
             op.project(*args)
     torch.cuda.synchronize()
+
+
+def test_weight_gradient_sizes_that_do_not_agree(device):
+    """Other token counts or another gradient's shape: an error, and the gradient keeps its values."""
+    dh = torch.zeros(70, 128, dtype=torch.bfloat16, device=device)
+    x, grad = dh.new_zeros(70, 256), torch.ones(128, 256, device=device)
+    for args in ((grad, dh, x[:69]), (grad, dh[:69], x), (grad, dh, dh), (grad[:64], dh, x)):
+        with pytest.raises(RuntimeError):
+            op.add_weight_grad(*args)
+    torch.cuda.synchronize()
+    assert bool((grad == 1).all())

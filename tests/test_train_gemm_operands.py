@@ -56,3 +56,23 @@ def test_projection_operands_on_two_devices(elsewhere):
     args = [bf(*s, device="meta" if i == elsewhere else "cpu") for i, s in enumerate([(24, 256), (128, 256), (24, 128)])]
     with pytest.raises(Library):
         op.project(*args)
+
+
+def test_agreeing_operands_reach_the_weight_gradient():
+    with pytest.raises(Reached):
+        op.add_weight_grad(torch.zeros(128, 256), bf(24, 128), bf(24, 256))
+
+
+@pytest.mark.parametrize("grad,dh,x", [((128, 256), (24, 128), (23, 256)), ((128, 256), (23, 128), (24, 256)),
+                                       ((128, 256), (24, 128), (24, 2, 128)), ((128, 256), (24, 128), (24, 128)),
+                                       ((256,), (24, 128), (24, 256))])
+def test_weight_gradient_sizes_that_do_not_agree(grad, dh, x):
+    with pytest.raises(Library):
+        op.add_weight_grad(torch.zeros(*grad), bf(*dh), bf(*x))
+
+
+@pytest.mark.parametrize("elsewhere", [0, 1, 2])
+def test_weight_gradient_operands_on_two_devices(elsewhere):
+    d = ["meta" if i == elsewhere else "cpu" for i in range(3)]
+    with pytest.raises(Library):
+        op.add_weight_grad(torch.zeros(128, 256, device=d[0]), bf(24, 128, device=d[1]), bf(24, 256, device=d[2]))

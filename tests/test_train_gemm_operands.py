@@ -51,6 +51,14 @@ def test_projection_sizes_that_do_not_agree(x, w, res):
         op.project(bf(*x), bf(*w), bf(*res))
 
 
+@pytest.mark.parametrize("C,K,met", [(32768, 32640, Reached), (32764, 32768, Reached), (32768, 32768, Library),
+                                     (32772, 128, Library)])
+def test_projection_weights_at_the_kernels_limit(C, K, met):
+    """The kernel's 32-bit offsets end below a 2 GiB weight; that one and wider ones take the library."""
+    with pytest.raises(met):
+        op.project(bf(1, K), torch.empty(C, K, dtype=torch.bfloat16), bf(1, C))   # never touched
+
+
 @pytest.mark.parametrize("elsewhere", [0, 1, 2])
 def test_projection_operands_on_two_devices(elsewhere):
     args = [bf(*s, device="meta" if i == elsewhere else "cpu") for i, s in enumerate([(24, 256), (128, 256), (24, 128)])]

@@ -118,7 +118,7 @@ def _projection_fits(x: Tensor, o_weight: Tensor, residual: Tensor) -> bool:
     (tokens, K), C = x.shape, o_weight.size(0)
     return (o_weight.size(1) == K and residual.shape == (tokens, C) and x.device == o_weight.device == residual.device
             and _plain(x, BF16, 16) and _plain(o_weight, BF16, 16) and _plain(residual, BF16, 8)
-            and K % 128 == 0 and C % 4 == 0 and max(C, K) <= 32768 and C * K * 2 < 2 ** 31)   # 32-bit offsets into it
+            and K % 128 == 0 and C % 4 == 0 and max(C, K) <= 32768 and 0 < C * K * 2 < 2 ** 31)   # 32-bit offsets into it
 
 
 def project(x: Tensor, o_weight: Tensor, residual: Tensor) -> tuple[Tensor, Tensor]:

@@ -59,6 +59,13 @@ def test_projection_weights_at_the_kernels_limit(C, K, met):
         op.project(bf(1, K), torch.empty(C, K, dtype=torch.bfloat16), bf(1, C))   # never touched
 
 
+@pytest.mark.parametrize("C,K", [(0, 128), (128, 0)])
+def test_empty_projection(C, K):
+    """No columns or no inner size: the kernel refuses it, the library gives its empty or zero product."""
+    with pytest.raises(Library):
+        op.project(bf(3, K), bf(C, K), bf(3, C))
+
+
 @pytest.mark.parametrize("elsewhere", [0, 1, 2])
 def test_projection_operands_on_two_devices(elsewhere):
     args = [bf(*s, device="meta" if i == elsewhere else "cpu") for i, s in enumerate([(24, 256), (128, 256), (24, 128)])]

@@ -47,9 +47,11 @@ def ve_backward(dv: Tensor, n: Tensor, ids: Tensor, order: Tensor, table: Tensor
 
 
 def _weight_grad(dz: Tensor, n: Tensor, w: Tensor) -> Tensor:
-    """dw = dz^T n over the rows, fp32 sums, like w: the HIP kernel for dense bf16 rows and fp32 w, else a library GEMM."""
+    """dw = dz^T n over the rows, fp32 sums, like w: the HIP kernel for dense bf16 rows and fp32 w on one device, else a
+    library GEMM."""
     rows = dz.size(0)
-    if (rows and n.dtype == torch.bfloat16 and n.is_contiguous() and n.data_ptr() % 8 == 0 and w.dtype == torch.float32
+    if (rows and dz.device == n.device == w.device and n.dtype == torch.bfloat16 and n.is_contiguous()
+            and n.data_ptr() % 8 == 0 and w.dtype == torch.float32
             and tuple(n.shape) == (rows, w.size(1)) and w.size(1) == w.size(0) * 128 and dz.size(1) == w.size(0)):
         lib = hip_library()
         need = lib.nc_ve_weight_grad_workspace_bytes(rows, w.size(0))

@@ -1,10 +1,11 @@
-"""Which operands of the training block's projection and weight gradients reach their HIP kernels, which trust the sizes
+"""Which operands of the training block's projection and weight gradients (the value-embedding gate's too) reach their HIP kernels, which trust the sizes
 and addresses they are given: without a GPU, CPU tensors stand for device tensors and a kernel call is an exception of its
 own. Operands whose sizes or devices do not agree must meet the library GEMM instead, which raises."""
 import pytest
 import torch
 
 from nanochat_amd import attention_op as op
+from nanochat_amd import ve_gate
 
 
 class Reached(BaseException):
@@ -30,6 +31,7 @@ def device_operands(monkeypatch):
     monkeypatch.setattr(op, "_plain", lambda t, dtype, alignment: (t.dtype == dtype and t.is_contiguous()
                                                                    and t.data_ptr() % alignment == 0))
     monkeypatch.setattr(op, "hip_library", NoLibrary)
+    monkeypatch.setattr(ve_gate, "hip_library", NoLibrary)
     monkeypatch.setattr(op, "stream", lambda: 0)
     monkeypatch.setattr(torch, "mm", library_gemm)
 
@@ -91,3 +93,11 @@ def test_weight_gradient_operands_on_two_devices(elsewhere):
     d = ["meta" if i == elsewhere else "cpu" for i in range(3)]
     with pytest.raises(Library):
         op.add_weight_grad(torch.zeros(128, 256, device=d[0]), bf(24, 128, device=d[1]), bf(24, 256, device=d[2]))
+
+
+@pytest.mark.parametrize("elsewhere,met", [(None, Reached), (0, Library), (1, Library), (2, Library)])
+def test_gate_weight_gradient_operands_on_two_devices(elsewhere, met):
+    """n is an operand of this product alone, so its place is checked nowhere before."""
+    d = ["meta" if i == elsewhere else "cpu" for i in range(3)]
+    with pytest.raises(met):
+        ve_gate._weight_grad(bf(24, 2, device=d[0]), bf(24, 256, device=d[1]), torch.zeros(2, 256, device=d[2]))

@@ -240,6 +240,7 @@ def _(dh: Tensor, qkv: Tensor, q_norm_weight: Tensor, k_norm_weight: Tensor, cos
 def _setup_context(ctx: FunctionCtx, inputs: tuple, output: tuple) -> None:
     named = dict(zip(FORWARD_INPUTS, inputs)) | dict(zip(FORWARD_OUTPUTS, output))
     ctx.window_left = named["window_left"]
+    ctx.h_spec = (named["h"].shape, named["h"].dtype)
     # no zero gradients for the seven outputs that have none (65,536 tokens, C = 768: 7 fills, 77 us a pass)
     ctx.set_materialize_grads(False)
     ctx.mark_non_differentiable(*(named[o] for o in FORWARD_OUTPUTS if o not in DIFFERENTIABLE_OUTPUTS))
@@ -247,9 +248,9 @@ def _setup_context(ctx: FunctionCtx, inputs: tuple, output: tuple) -> None:
 
 
 def _backward(ctx: FunctionCtx, dh: Tensor | None, *_: Tensor | None) -> tuple:
-    if dh is None:                                  # nothing flows back through h
-        return (None,) * len(FORWARD_INPUTS)
-    named = dict(zip(SAVED, ctx.saved_tensors), dh=dh, window_left=ctx.window_left)
+    named = dict(zip(SAVED, ctx.saved_tensors), window_left=ctx.window_left)
+    # nothing flows back through h: the inputs' gradients are zeros, not absent
+    named["dh"] = named["qkv"].new_zeros(ctx.h_spec[0], dtype=ctx.h_spec[1]) if dh is None else dh
     got = dict(zip(BACKWARD_OUTPUTS, attention_bwd(*(named[name] for name in BACKWARD_INPUTS))))
     if named["table"] is None:                      # no value embeddings: n and w_gate took no part
         del got["n"], got["w_gate"]

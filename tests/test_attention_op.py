@@ -74,3 +74,28 @@ def test_gradients_reach_the_reference_positions():
         outs[0].backward(torch.empty_like(outs[0]))
         got = {k: tuple(v.grad.shape) for k, v in inputs.items() if isinstance(v, torch.Tensor) and v.grad is not None}
         assert got == wanted, (with_table, got)
+
+
+class _Stop(torch.autograd.Function):
+    """The identity, with no gradient for its input."""
+
+    @staticmethod
+    def forward(ctx, x):
+        return x.clone()
+
+    @staticmethod
+    def backward(ctx, g):
+        return None
+
+
+def test_no_gradient_for_the_block_gives_zeros():
+    """What follows the block may send it no gradient; its inputs' are then zeros, as for any op, not absent."""
+    for with_table in (False, True):
+        a, ve = fake_inputs(2, 48, 2, 40, with_table, d="meta")
+        inputs = {**a, **ve}
+        wanted = ["qkv", "q_norm_weight", "k_norm_weight", "residual"] + (["n", "w_gate"] if with_table else [])
+        for name in wanted:
+            inputs[name].requires_grad_()
+        h = torch.ops.nanochat_amd.attention(*inputs.values())[0]
+        got = torch.autograd.grad(_Stop.apply(h).sum(), [inputs[name] for name in wanted])
+        assert [g.shape for g in got] == [inputs[name].shape for name in wanted]

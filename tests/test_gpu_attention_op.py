@@ -129,3 +129,27 @@ def test_attention_op_matches_float64_autograd(device, with_table, window):
         rel_check(tab_d.grad, r_tab.grad, "table.grad")
     else:
         assert outs[6].numel() == 0 and outs[7].numel() == 0
+
+
+def test_no_gradient_for_the_block_gives_zeros(device):
+    """A block whose result receives no gradient: zero gradients for its inputs, nothing added to the weight's."""
+    B, T, H = 1, 40, 1
+    gen = torch.Generator().manual_seed(5)
+    bf = lambda *s: torch.randn(*s, generator=gen).bfloat16().to(device)
+    cos, sin = (t.to(device) for t in rotary_tables(T))
+    qkv, residual = bf(B, T, 3 * 128).requires_grad_(), bf(B, T, 128).requires_grad_()
+    gains, o_grad = torch.ones(2, 128, device=device), torch.ones(128, 128, device=device)
+    h = attention(qkv, gains[0].clone(), gains[1].clone(), cos, sin, T, torch.tensor([0, T], dtype=torch.int32, device=device),
+                  torch.tensor(1), bf(128, 128), o_grad, residual, *(None,) * 6)[0]
+
+    class Stop(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x):
+            return x.clone()
+
+        @staticmethod
+        def backward(ctx, g):
+            return None
+
+    got = torch.autograd.grad(Stop.apply(h).sum(), [qkv, residual])
+    assert all(bool((g == 0).all()) for g in got) and bool((o_grad == 1).all())

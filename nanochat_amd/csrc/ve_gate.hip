@@ -27,6 +27,8 @@
 #include "nc_internal.h"
 #include "nanochat_amd.h"
 
+#include <climits>
+
 namespace nc {
 namespace {
 
@@ -232,96 +234,116 @@ __device__ __forceinline__ void stage_w_rows(float *ws, const float *w) {
         reinterpret_cast<float4 *>(ws)[i] = reinterpret_cast<const float4 *>(w)[i];
 }
 
-/* A run's accumulated table gradient added into dtable row t. With equal tokens adjacent in `ids` (sorted, the
- * reference's contract), a run that neither starts at the wave's first position nor ends at its last one holds every
- * occurrence of its token, so no other wave touches that row: a plain read-add-write, the row read when the run began
- * (old). So does a wave's first or last run when the id before or after its range is another token; otherwise (shared) the
- * run continues in a neighbouring wave's range: hardware fp32 atomics (two instructions per head, each 64 dwords at
- * 8-byte stride). */
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
+/* The row of dtable is read when a run begins rather than when it ends where registers for it cost no waves: beside a
+ * second position's rows (AHEAD, below), and from 13 heads, whose w leaves room for one workgroup a CU in LDS. */
+template <int H, bool AHEAD>
+constexpr bool VE_EARLY = AHEAD || H * H * HEAD_DIM * 4 > 80 * 1024;
+
+/* The run a wave is in. */
 template <int H>
-__device__ __forceinline__ void flush_run(float *dtable, int t, const float (&acc)[H][2], const u32x2 (&old)[H], int lane,
-                                          bool shared) {
-    float *row = dtable + (long long)t * (H * HEAD_DIM) + 2 * lane;
+struct VeRun {
+    bool started, ok, shared;   /* a run; a token of the table; it began in the wave before */
+    int t;
+    uint32_t eb[H];             /* the token's table columns as bf16x2 */
+    float acc[H][2];
+    u32x2 old[H];               /* VE_EARLY: the token's row of dtable before the run */
+};
+
+/* A run's accumulated table gradient added into dtable row t. With equal tokens adjacent in `ids` (sorted, the
+ * reference's contract), a run that neither starts at the wave's first position nor ends at its last one holds every
+ * occurrence of its token, so no other wave touches that row: a plain read-add-write. So does a wave's first or last run
+ * when the id before or after its range is another token; otherwise (shared) the run continues in a neighbouring wave's
+ * range: hardware fp32 atomics (two instructions per head, each 64 dwords at 8-byte stride). */
+template <int H, bool AHEAD>
+__device__ __forceinline__ void flush_run(const VeBwd &a, VeRun<H> &run, int lane, bool shared) {
+    if (!run.started || !run.ok) return;
+    float *row = a.dtable + (long long)run.t * (H * HEAD_DIM) + 2 * lane;
     if (shared) {
 #pragma unroll
         for (int k = 0; k < H; k++) {
-            unsafeAtomicAdd(row + k * HEAD_DIM, acc[k][0]);
-            unsafeAtomicAdd(row + k * HEAD_DIM + 1, acc[k][1]);
+            unsafeAtomicAdd(row + k * HEAD_DIM, run.acc[k][0]);
+            unsafeAtomicAdd(row + k * HEAD_DIM + 1, run.acc[k][1]);
         }
-    } else {
-#pragma unroll
-        for (int k = 0; k < H; k++)
-            *reinterpret_cast<float2 *>(row + k * HEAD_DIM) =
-                float2{__uint_as_float(old[k][0]) + acc[k][0], __uint_as_float(old[k][1]) + acc[k][1]};
+        return;
     }
+    if (!VE_EARLY<H, AHEAD>) {
+#pragma unroll
+        for (int k = 0; k < H; k++) run.old[k] = *reinterpret_cast<const u32x2 *>(row + k * HEAD_DIM);
+    }
+#pragma unroll
+    for (int k = 0; k < H; k++)
+        *reinterpret_cast<float2 *>(row + k * HEAD_DIM) =
+            float2{__uint_as_float(run.old[k][0]) + run.acc[k][0], __uint_as_float(run.old[k][1]) + run.acc[k][1]};
 }
 
-/* What one position needs, fetched a position ahead: its row and token, the row of dout and, when it begins a run, the
- * token's table row and (for a run this wave alone holds from here) its row of dtable. */
+/* Up to 64 positions' rows and tokens, lane l position l's. */
+struct VePositions {
+    uint32_t row_lo, row_hi;
+    int id, n;
+};
+
+/* A position's row and token and what it reads of them. e, old: the table's and dtable's row where a run begins. */
 template <int H>
 struct VeRow {
     long long r;
     int t;
     bool valid, fresh, ok;   /* a row; the first of a run; a token of the table */
     bool shared;             /* fresh: the run began in the wave before */
-    uint32_t d[H], g;        /* g: lane h the row's gate of head h */
+    uint32_t d[H];
+    float g[H];              /* the row's gates; AHEAD: g[0] lane h's of head h */
     u32x2 e[H], old[H];
 };
 
-/* Up to 64 positions' rows and tokens, lane l position l's. */
-struct VePositions {
-    uint32_t row_lo, row_hi;
-    int id;
-    int n;
-};
+/* The rows of w's token where a run begins (there): the table's and, with OLD, dtable's unless another wave adds to it. */
+template <int H, bool OLD>
+__device__ __forceinline__ void ve_fetch_run(const VeBwd &a, VeRow<H> &w, bool there, int lane) {
+    constexpr int C = H * HEAD_DIM;
+    const bool row = there && w.ok;
+    const Rsrc re = row_rsrc(a.table + (row ? (long long)w.t * C : 0), row ? C * 4 : 0);
+    const Rsrc ro = row_rsrc(a.dtable + (row ? (long long)w.t * C : 0), row && !w.shared ? C * 4 : 0);
+#pragma unroll
+    for (int k = 0; k < H; k++) {
+        w.e[k] = __builtin_amdgcn_raw_buffer_load_b64(re, (k * HEAD_DIM + 2 * lane) * 4, 0, 0);
+        if (OLD) w.old[k] = __builtin_amdgcn_raw_buffer_load_b64(ro, (k * HEAD_DIM + 2 * lane) * 4, 0, 0);
+    }
+}
 
-/* Position q's row, with `run` the token of the run before it (started: there is one). Loads a position does not need go
- * through zero-size descriptors: no access, and no branch that would make the compiler wait for those in flight. */
-template <int H>
+/* Position q's row, with `run` the token of the run before it (started: there is one). AHEAD: also its gate and, where it
+ * begins a run, the token's rows. Loads a position does not need go through zero-size descriptors: no access, and no branch
+ * that would make the compiler wait for those in flight. */
+template <int H, bool AHEAD>
 __device__ __forceinline__ void ve_fetch(const VeBwd &a, const VePositions &ps, int q, bool has_before, int before,
                                          bool started, int run, int lane, VeRow<H> &w) {
     constexpr int C = H * HEAD_DIM;
-    const bool in = q < ps.n;
     const int l = q & (WAVE - 1);
     const uint32_t lo = __builtin_amdgcn_readlane(ps.row_lo, l), hi = __builtin_amdgcn_readlane(ps.row_hi, l);
-    w.r = in ? (long long)(((unsigned long long)hi << 32) | lo) : -1;
+    w.r = q < ps.n ? (long long)(((unsigned long long)hi << 32) | lo) : -1;
     w.t = __builtin_amdgcn_readlane(ps.id, l);
     w.valid = w.r >= 0 && w.r < a.rows;   /* not a row: nothing to read or write */
     w.fresh = w.valid && (!started || w.t != run);
     w.ok = w.t >= 0 && (long long)w.t < a.vocab;
     w.shared = !started && has_before && w.t == before;
-    const bool row = w.fresh && w.ok;
     const Rsrc rd = row_rsrc(a.dout + (w.valid ? w.r * a.dout_stride : 0), w.valid ? C * 2 : 0);
-    const Rsrc re = row_rsrc(a.table + (row ? (long long)w.t * C : 0), row ? C * 4 : 0);
-    const Rsrc ro = row_rsrc(a.dtable + (row ? (long long)w.t * C : 0), row && !w.shared ? C * 4 : 0);
-    w.g = __builtin_amdgcn_raw_buffer_load_b32(row_rsrc(a.gate + (w.valid ? w.r * H : 0), w.valid ? H * 4 : 0), lane * 4,
-                                               0, 0);
+    const float *gate = a.gate + (w.valid ? w.r * H : 0);
+    if (AHEAD)
+        w.g[0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(row_rsrc(gate, w.valid ? H * 4 : 0), lane * 4, 0, 0));
 #pragma unroll
     for (int k = 0; k < H; k++) {
         w.d[k] = __builtin_amdgcn_raw_buffer_load_b32(rd, (k * HEAD_DIM + 2 * lane) * 2, 0, 2);
-        w.e[k] = __builtin_amdgcn_raw_buffer_load_b64(re, (k * HEAD_DIM + 2 * lane) * 4, 0, 0);
-        w.old[k] = __builtin_amdgcn_raw_buffer_load_b64(ro, (k * HEAD_DIM + 2 * lane) * 4, 0, 0);
+        if (!AHEAD) w.g[k] = gate[k];
     }
+    if (AHEAD) ve_fetch_run<H, true>(a, w, w.fresh, lane);
 }
 
-/* The run a wave is in. */
-template <int H>
-struct VeRun {
-    bool started, ok, shared;
-    int t;
-    uint32_t eb[H];     /* the token's table columns as bf16x2 */
-    float acc[H][2];
-    u32x2 old[H];       /* the token's row of dtable before the run */
-};
-
-template <int H>
-__device__ __forceinline__ void ve_row(const VeBwd &a, const float *ws, const VeRow<H> &w, VeRun<H> &run, int lane) {
+template <int H, bool AHEAD>
+__device__ __forceinline__ void ve_row(const VeBwd &a, const float *ws, VeRow<H> &w, VeRun<H> &run, int lane) {
     constexpr int C = H * HEAD_DIM;
     if (!w.valid) return;
     if (w.fresh) {
-        if (run.started && run.ok) flush_run<H>(a.dtable, run.t, run.acc, run.old, lane, run.shared);
+        if (!AHEAD) ve_fetch_run<H, VE_EARLY<H, false>>(a, w, true, lane);
+        flush_run<H, AHEAD>(a, run, lane, run.shared);
         run.started = true;
         run.shared = w.shared;
         run.t = w.t;
@@ -330,7 +352,7 @@ __device__ __forceinline__ void ve_row(const VeBwd &a, const float *ws, const Ve
         for (int k = 0; k < H; k++) {
             run.eb[k] = (uint32_t)f32_to_bf16(__uint_as_float(w.e[k][0])) |
                         ((uint32_t)f32_to_bf16(__uint_as_float(w.e[k][1])) << 16);
-            run.old[k] = w.old[k];
+            if (VE_EARLY<H, AHEAD>) run.old[k] = w.old[k];
             run.acc[k][0] = 0.0f;
             run.acc[k][1] = 0.0f;
         }
@@ -338,7 +360,7 @@ __device__ __forceinline__ void ve_row(const VeBwd &a, const float *ws, const Ve
     float dz[H], mine = 0.0f;
 #pragma unroll
     for (int k = 0; k < H; k++) {
-        const float g = __uint_as_float(__builtin_amdgcn_readlane(w.g, k));
+        const float g = AHEAD ? __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w.g[0]), k)) : w.g[k];
         const float d0 = __uint_as_float(w.d[k] << 16), d1 = __uint_as_float(w.d[k] & 0xFFFF0000u);
         const float e0 = __uint_as_float(run.eb[k] << 16), e1 = __uint_as_float(run.eb[k] & 0xFFFF0000u);
         run.acc[k][0] = run.acc[k][0] + bf16r(g * d0);
@@ -367,11 +389,14 @@ __device__ __forceinline__ void ve_row(const VeBwd &a, const float *ws, const Ve
 /* Backward mapping (unlike the forward's): lane l holds columns k*128 + 2l and k*128 + 2l + 1 of every head k, so a
  * head's gate is one scalar, dg is a whole-wave sum, and every access of dout, the table, dn and dtable is 4 or 8
  * contiguous bytes per lane, 256 or 512 contiguous bytes per instruction. A position is a chain of loads (its row's
- * number, then the row, then at a run's end the row of dtable: 2.4 us a position). So 64 positions' numbers and tokens
- * are read at once, one a lane, and a position's rows are loaded before the arithmetic of the one before it, into a
- * second register set (the loop alternates two by name). H = 6, tokens of a log-uniform
- * vocabulary: 4,096 rows 34 -> 16 us, 20,000 65 -> 39, 65,536 100 -> 98 (its bytes take 84). */
-template <int H>
+ * number, then the row, then at a run's end the row of dtable: 2.4 us a position), so 64 positions' numbers and tokens
+ * are read at once, one a lane. The rest of the chain is hidden by the resident waves or, AHEAD, by loading a position's
+ * rows before the arithmetic of the one before it, into a second register set (the loop alternates two by name): 133
+ * registers at H = 6 against 72, so fewer waves (choose_backward says where which is the faster). H = 6, tokens of a
+ * log-uniform vocabulary, us against one position at a time with every border run atomic: 256 rows 5.5 -> 5.1, 4,096
+ * 32 -> 15.5, 16,384 81 -> 34, 65,536 103 -> 88 (its bytes take 84); H = 13 4,096 rows 47 -> 35, 65,536 234 -> 225; H = 16
+ * 57 -> 41 and 288 -> 287. */
+template <int H, bool AHEAD>
 __global__ void __launch_bounds__(VE_THREADS) ve_backward_kernel(VeBwd a) {
     constexpr int C = H * HEAD_DIM;
     __shared__ __attribute__((aligned(16))) float ws[H * C];
@@ -382,34 +407,36 @@ __global__ void __launch_bounds__(VE_THREADS) ve_backward_kernel(VeBwd a) {
     const bool has_before = p0 > 0 && p0 < p1, has_after = p1 < a.rows && p0 < p1;
     const int before = has_before ? __builtin_amdgcn_readfirstlane(a.ids[p0 - 1]) : 0;
     const int after = has_after ? __builtin_amdgcn_readfirstlane(a.ids[p1]) : 0;
+    stage_w_rows<H>(ws, a.w);
+    __syncthreads();
     VeRun<H> run;
     run.started = run.ok = run.shared = false;
     run.t = -1;
-    bool staged = false;
-    for (long long base = p0; base < p1 || !staged; base += WAVE) {
+    for (long long base = p0; base < p1; base += WAVE) {
         VePositions ps;
-        ps.n = base < p1 ? (int)(p1 - base < WAVE ? p1 - base : WAVE) : 0;
+        ps.n = (int)(p1 - base < WAVE ? p1 - base : WAVE);
         const unsigned long long row = lane < ps.n ? (unsigned long long)a.order[base + lane] : ~0ull;
         ps.row_lo = (uint32_t)row;
         ps.row_hi = (uint32_t)(row >> 32);
         ps.id = lane < ps.n ? a.ids[base + lane] : -1;
         VeRow<H> x, y;
-        ve_fetch<H>(a, ps, 0, has_before, before, run.started, run.t, lane, x);
-        if (!staged) {   /* w, behind the first row's loads; every wave comes here once */
-            stage_w_rows<H>(ws, a.w);
-            __syncthreads();
-            staged = true;
+        if (!AHEAD) {
+            for (int q = 0; q < ps.n; q++) {
+                ve_fetch<H, false>(a, ps, q, has_before, before, run.started, run.t, lane, x);
+                ve_row<H, false>(a, ws, x, run, lane);
+            }
+            continue;
         }
+        ve_fetch<H, true>(a, ps, 0, has_before, before, run.started, run.t, lane, x);
         for (int q = 0; q < ps.n; q += 2) {
-            ve_fetch<H>(a, ps, q + 1, has_before, before, run.started || x.valid, x.valid ? x.t : run.t, lane, y);
-            ve_row<H>(a, ws, x, run, lane);
+            ve_fetch<H, true>(a, ps, q + 1, has_before, before, run.started || x.valid, x.valid ? x.t : run.t, lane, y);
+            ve_row<H, true>(a, ws, x, run, lane);
             if (q + 1 >= ps.n) break;
-            ve_fetch<H>(a, ps, q + 2, has_before, before, run.started || y.valid, y.valid ? y.t : run.t, lane, x);
-            ve_row<H>(a, ws, y, run, lane);
+            ve_fetch<H, true>(a, ps, q + 2, has_before, before, run.started || y.valid, y.valid ? y.t : run.t, lane, x);
+            ve_row<H, true>(a, ws, y, run, lane);
         }
     }
-    if (run.started && run.ok)
-        flush_run<H>(a.dtable, run.t, run.acc, run.old, lane, run.shared || (has_after && run.t == after));
+    flush_run<H, AHEAD>(a, run, lane, run.shared || (has_after && run.t == after));
 }
 
 /* The gate weight's gradient dw[h][c] = sum over rows of dz[row][h] n[row][c] (bf16 operands, fp32 sums): H <= 16
@@ -519,10 +546,12 @@ int launch_weight(int heads, const VeWeight &a, int slabs, float *dw, hipStream_
     }
 }
 
-/* Workgroups for `rows` rows: `per` rows a wave, at most as many workgroups as the device holds at once (the
+constexpr int VE_MOST = 8;   /* workgroups of VE_THREADS that a CU holds, and more */
+
+/* Workgroups for `rows` rows: `per` rows a wave, at most as many workgroups as the device holds at once, `most` a CU (the
  * kernel's resident workgroups per device, cached per device in `resident`). */
 template <typename K>
-int ve_blocks(K kernel, long long rows, int per, int (&resident)[64]) {
+int ve_blocks(K kernel, long long rows, int per, int most, int (&resident)[64]) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return -1;
     if (!resident[dev]) {
@@ -530,7 +559,7 @@ int ve_blocks(K kernel, long long rows, int per, int (&resident)[64]) {
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
             hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, VE_THREADS, 0) != hipSuccess)
             return -1;
-        resident[dev] = max(1, cus) * max(1, per_cu);
+        resident[dev] = max(1, cus) * max(1, min(per_cu, most));
     }
     const long long need = (rows + VE_WAVES * per - 1) / (VE_WAVES * per);
     return (int)max(1LL, min(need, (long long)resident[dev]));
@@ -539,23 +568,41 @@ int ve_blocks(K kernel, long long rows, int per, int (&resident)[64]) {
 template <int H>
 int launch_forward(const VeFwd &a, hipStream_t stream) {
     static int resident[64] = {0};
-    const int blocks = ve_blocks(ve_forward_kernel<H>, a.rows, 1, resident);
+    const int blocks = ve_blocks(ve_forward_kernel<H>, a.rows, 1, VE_MOST, resident);
     if (blocks < 0) return (int)hipErrorInvalidDevice;
     hipLaunchKernelGGL(ve_forward_kernel<H>, dim3(blocks), dim3(VE_THREADS), 0, stream, a);
     return (int)hipGetLastError();
 }
 
-template <int H>
-int launch_backward(const VeBwd &a, hipStream_t stream) {
+template <int H, bool AHEAD>
+int launch_backward(const VeBwd &a, int per, hipStream_t stream) {
     static int resident[64] = {0};
-    /* Rows a wave: a frequent token's rows all add into one row of dtable, a wave at a time, so more waves mean more
-     * adds at the same addresses; fewer leave the chip idle (H = 6, one / two / four rows a wave: 1,024 rows 10 / 9 / 13
-     * us, 2,048 16 / 13 / 14, 4,096 19 / 19 / 16; from 8,192 the same). */
-    const int per = (int)max(1LL, min(4LL, a.rows / 1024));
-    const int blocks = ve_blocks(ve_backward_kernel<H>, a.rows, per, resident);
+    const int blocks = ve_blocks(ve_backward_kernel<H, AHEAD>, a.rows, per, AHEAD ? 3 : VE_MOST, resident);
     if (blocks < 0) return (int)hipErrorInvalidDevice;
-    hipLaunchKernelGGL(ve_backward_kernel<H>, dim3(blocks), dim3(VE_THREADS), 0, stream, a);
+    hipLaunchKernelGGL((ve_backward_kernel<H, AHEAD>), dim3(blocks), dim3(VE_THREADS), 0, stream, a);
     return (int)hipGetLastError();
+}
+
+constexpr int VE_AHEAD_HEADS = 10;
+
+/* The form, and rows a wave, at most four while every wave finds that many.
+ * Rows a wave: a frequent token's rows all add into one row of dtable, a wave at a time, so more waves mean more adds at the
+ * same addresses; fewer leave the chip idle (H = 6, one / two / four rows a wave: 1,024 rows 8.8 / 7.7 / 10.9 us, 4,096
+ * 26 / 17 / 15).
+ * The second register set wins where a wave has several rows but the waves do not fill the chip, and at few heads always
+ * (AHEAD / not, us of log-uniform tokens: H = 2, 16,384 rows 24 / 24, 65,536 45 / 55; H = 5 38 / 37, 76 / 87; H = 6 8,192
+ * 22 / 24, 32,768 54 / 61, 65,536 97 / 88; H = 8 16,384 42 / 46, 65,536 123 / 102; H = 10 8,192 35 / 37, 16,384 51 / 56,
+ * 32,768 85 / 82, 65,536 163 / 131). From 11 heads it takes 253 registers, from 13 it spilled: 65,536 rows of 16 heads took
+ * 931 us. At one and two heads it fits a fourth workgroup a CU, whose adds cost more than it brings (65,536 rows, H = 1: 46
+ * us with four, 36 with three). */
+template <int H>
+int choose_backward(const VeBwd &a, hipStream_t stream) {
+    const int per = (int)max(1LL, min(4LL, a.rows / 1024));
+    if constexpr (H <= VE_AHEAD_HEADS) {
+        const long long end = H <= 5 ? LLONG_MAX : H <= 8 ? 49152 : 24576;
+        if (a.rows >= 8192 && a.rows < end) return launch_backward<H, true>(a, per, stream);
+    }
+    return launch_backward<H, false>(a, per, stream);
 }
 
 template <int H = 1>
@@ -563,7 +610,7 @@ int dispatch(int heads, bool fwd, const VeFwd &f, const VeBwd &b, hipStream_t st
     if constexpr (H > VE_MAX_HEADS) {
         return NC_ERR_SHAPE;
     } else {
-        if (heads == H) return fwd ? launch_forward<H>(f, stream) : launch_backward<H>(b, stream);
+        if (heads == H) return fwd ? launch_forward<H>(f, stream) : choose_backward<H>(b, stream);
         return dispatch<H + 1>(heads, fwd, f, b, stream);
     }
 }

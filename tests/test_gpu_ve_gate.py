@@ -267,3 +267,16 @@ def test_runs_that_end_at_wave_borders(device):
         want[idx[p]] += g
         mag[idx[p]] += g.abs()
     assert bool(((d[6].double().cpu() - want).abs() <= 12 * 2.0 ** -24 * mag + 1e-12).all())
+
+
+@pytest.mark.parametrize("H,rows,vocab", [(16, 2, 3), (16, 1030, 5000), (13, 4099, 700), (2, 8191, 60), (6, 8192, 3000),
+                                          (4, 16391, 100), (10, 24575, 900), (10, 24576, 900)])
+def test_backward_of_many_heads_and_rows(device, H, rows, vocab):
+    """Head counts up to the largest, and row counts on both sides of the dispatch's steps: one to four rows a wave, one
+    position's rows in registers and two."""
+    qkv, n, table, w, idx, dqkv, dtable0 = make(rows, H, vocab, seed=H + rows)
+    C = H * HEAD_DIM
+    gate = np.random.default_rng(rows).uniform(0.05, 1.95, (rows, H)).astype(np.float32)
+    dn, dz, dtable, ids, order = run_backward(device, dqkv, idx, table, w, gate, dtable0, H)
+    check_backward(np32(dqkv[:, 2 * C:]), table.numpy(), w.numpy(), idx.numpy().astype(np.int64), gate, np32(n),
+                   dtable0.numpy(), dn, dz, dtable, ids, order, tol_runs=rows + 2)

@@ -106,6 +106,9 @@ struct PfGemm {
 };
 int prefill_gemm(const PfGemm &g, int epi, hipStream_t stream);
 
+/* The current device's compute units (256 where there is none to ask), asked for once a device. */
+int device_cus();
+
 constexpr int PF_SSQ = 32;   /* columns of a sum of squares of SG_RESID2, the same for every tile size */
 __host__ __device__ static inline int pf_ssq_cols(int N) { return (N + PF_SSQ - 1) / PF_SSQ; }
 /* rstd[m] = 1 / sqrt((row m's sums of squares in a fixed order) / N + FLT_EPSILON). Returns 0 or a hipError_t. */

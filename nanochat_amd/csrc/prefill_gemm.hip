@@ -389,8 +389,7 @@ int tile_rstd(const float *ssq, int M, int N, float *rstd, hipStream_t stream) {
     return (int)hipGetLastError();
 }
 
-/* The number of compute units of the current device (256 if it cannot be read), once per device. */
-static int device_cus() {
+int device_cus() {
     static int cus[64] = {0};
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;

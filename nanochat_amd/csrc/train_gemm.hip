@@ -6,7 +6,7 @@
  * [M][N2], bf16, fp32 sums). The result is small (C x C) and the sum long (every token), so the tiles alone would leave
  * most of the chip idle (768 x 768: 9 tiles of 256 x 256): the tokens are cut into slices, one workgroup a (tile,
  * slice), each storing its fp32 partial tile, and weight_grad_sum_kernel adds a tile's partials in slice order, so the
- * result does not depend on scheduling.
+ * result does not depend on scheduling. Few tokens, or tiles enough, make one slice, whose tiles are added into the result.
  *
  * Both operands have the summed dimension as their row, so a stage (32 token rows of 256 columns of each operand, 32
  * KiB) goes into LDS as it lies in memory, by LDS DMA, and the MFMA operands are read transposed
@@ -14,7 +14,7 @@
  * s ^ (row % 8), so the eight rows that half a wave reads meet in different banks. Eight waves hold 128 x 64 outputs
  * each; a ring of four stage buffers keeps three in flight, with hand-placed waits and a barrier without a memory fence.
  * 65,536 tokens, 768 x 768: 99 us (783 TFLOP/s) + 13 us for the sum of 28 slices, where the library's GEMM took 297 us on
- * 24 tiles and a pass more to add its result; 9,995 tokens, 1,280 x 1,280: 89 + 6 -> 41 + 13 us.
+ * 24 tiles and a pass more to add its result; 9,995 tokens, 1,280 x 1,280: 89 + 6 -> 46 us.
  *
  * linear_residual_rms: 141 us + 5 us for the rows' rstd at 65,536 tokens, C = 768, against a library GEMM with fp32 output
  * (99 us) and five elementwise and reducing passes over it (251 us).
@@ -46,7 +46,7 @@ struct WeightGrad {
     int N1, N2, tiles2;        /* tiles2: column tiles */
     long long M;
     int slices, rows;          /* token slices, rows of each (a multiple of WG_KC) */
-    float *part;               /* [slices][N1][N2] */
+    float *part;               /* [slices][N1][N2]; DIRECT: the result [N1][N2], added into */
 };
 
 struct WgStage {
@@ -112,6 +112,8 @@ __device__ __forceinline__ void wg_compute(const WgStage &s, f32x4 (&acc)[8][4],
         wg_compute(CUR, acc, wm, wn, g, c);                                           \
     } while (0)
 
+/* DIRECT: one slice, whose tiles are added straight into the result. */
+template <bool DIRECT>
 __global__ void __launch_bounds__(WG_WAVES *WAVE, 1) weight_grad_kernel(WeightGrad p) {
     __shared__ __align__(16) WgStage s0, s1, s2, s3;   /* distinct objects: a read of one never waits for another's DMA */
     const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x >> 6, g = lane >> 4, c = lane & 15;
@@ -142,18 +144,40 @@ __global__ void __launch_bounds__(WG_WAVES *WAVE, 1) weight_grad_kernel(WeightGr
         WG_STEP(j + 3, s3, s2);
     }
     __builtin_amdgcn_s_waitcnt(0);   /* no DMA may land in LDS after the workgroup ends */
-    /* lane (g, c) of result tile (t, u): rows i0 + 128 wm + 16 t + 4 g + e, column j0 + 64 wn + 16 u + c */
-    float *part = p.part + (long long)slice * p.N1 * p.N2;
+    /* lane (g, c) of result tile (t, u): rows i0 + 128 wm + 16 t + 4 g + e, column j0 + 64 wn + 16 u + c. 32-bit offsets into
+     * the tile's rows (flat addresses took 2 us more at 2,048 tokens, and spilled where the tile is added): rows past N1 lie
+     * outside them, columns past N2 take an offset past them, and neither is accessed. */
+    const int live = p.N1 - i0 < WG_T ? p.N1 - i0 : WG_T;
+    const unsigned row_bytes = (unsigned)p.N2 * 4;
+    const Rsrc ro = __builtin_amdgcn_make_buffer_rsrc((void *)(p.part + ((long long)slice * p.N1 + i0) * p.N2), (short)0,
+                                                      live * (int)row_bytes, 0x00020000);
+    unsigned at[4];
 #pragma unroll
-    for (int t = 0; t < 8; t++)
+    for (int u = 0; u < 4; u++) {
+        const int col = j0 + 64 * wn + 16 * u + c;
+        at[u] = col < p.N2 ? (unsigned)(128 * wm + 4 * g) * row_bytes + (unsigned)col * 4 : (unsigned)WG_PAST;
+    }
+    float old[2][4][4];   /* DIRECT: the result's rows of t, and of t + 1 in flight (one tile at a time waited 32 times) */
+    const auto fetch_old = [&](int t) {
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int i = i0 + 128 * wm + 16 * t + 4 * g, col = j0 + 64 * wn + 16 * u + c;
-            if (col >= p.N2) continue;
+        for (int u = 0; u < 4; u++)
 #pragma unroll
             for (int e = 0; e < 4; e++)
-                if (i + e < p.N1) part[(long long)(i + e) * p.N2 + col] = acc[t][u][e];
-        }
+                old[t & 1][u][e] =
+                    __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ro, at[u] + (16 * t + e) * row_bytes, 0, 0));
+    };
+    if (DIRECT) fetch_old(0);
+#pragma unroll
+    for (int t = 0; t < 8; t++) {
+        if (DIRECT && t < 7) fetch_old(t + 1);
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                __builtin_amdgcn_raw_buffer_store_b32(
+                    __float_as_uint(DIRECT ? old[t & 1][u][e] + acc[t][u][e] : acc[t][u][e]), ro,
+                    at[u] + (16 * t + e) * row_bytes, 0, 0);
+    }
 }
 
 /* out += the slices' partials added in order; four elements a thread. */
@@ -170,22 +194,54 @@ __global__ void __launch_bounds__(256) weight_grad_sum_kernel(const float4 *part
     out[i] = float4{o.x + sum.x, o.y + sum.y, o.z + sum.z, o.w + sum.w};
 }
 
-constexpr int WG_CUS = 256;   /* MI355X compute units: one workgroup (128 KiB of LDS) each */
-constexpr int WG_MIN_ROWS = 8 * WG_KC;   /* a shorter slice is mostly the ring's start */
+constexpr int WG_MIN_ROWS = 4 * WG_KC;   /* a shorter slice is mostly the ring's start */
 
-/* Slices of M tokens for an N1 x N2 result: as many as fill the CUs with one workgroup each, none under WG_MIN_ROWS and
- * none whose operand slice passes 2 GiB. */
+/* What M tokens of an N1 x N2 result take in us by a model of three measured parts, one workgroup (128 KiB of LDS) a CU:
+ * - rounds of workgroups, each as long as a slice's stages and ten more for its start and its end;
+ * - a stage: 0.65 alone, 20 % more with every CU at work, and then up to 27 % more where the slices, five or more and no
+ *   multiple of four, spread over the eight XCDs (workgroup b runs on XCD b % 8 and takes slice b % slices), so that each L2
+ *   holds most of them: 1,664 x 1,664 over 65,536 tokens, 49 tiles: 4 slices 341 us, 5 slices 429;
+ * - a slice's partial tiles out and back, and the sum; one slice has neither (its tiles are added into the result). */
+double weight_grad_time(long long tiles, long long elements, int cus, long long slices, long long rows) {
+    const double rounds = (double)((tiles * slices + cus - 1) / cus), busy = (double)(tiles * slices) / (rounds * cus);
+    const double spread = slices < 5 || slices % 4 == 0 ? 0.0 : slices % 2 == 0 ? 0.15 : 0.27;
+    const double stage = 0.65 * (1.0 + 0.2 * busy + spread * busy * busy);
+    const double partials = slices == 1 ? 0.0 : 2.0 + slices * (elements * 1.2e-6 + 0.04);
+    return rounds * (rows / WG_KC + 10) * stage + partials;
+}
+
+/* Token slices: the best of a few counts by weight_grad_time (small ones, steps of about an eighth above, and those that just
+ * fill one to eight rounds), none under WG_MIN_ROWS rows unless it is the only one and none whose operand slice passes 1
+ * GiB. As many as fill the CUs, and one where the tiles are half of them or more, left CUs idle at wide results and spent
+ * more on partials than they saved at few tokens. us, so and by the model (library product and addition):
+ *   tokens    768 x 768        1,664 x 1,664      2,560 x 2,560       3,072 x 3,072
+ *      512    17 -> 15 (25)      23 ->  21 (25)     34 ->  23 (31)      37 ->    26 (41)
+ *    2,048    24 -> 22 (27)      37 ->  31 (32)     47 ->  47 (51)      64 ->    53 (67)
+ *    9,995    36 -> 29 (66)      85 ->  69 (104)   122 -> 122 (157)    212 ->   190 (214)
+ *   65,536    80 -> 80 (298)    429 -> 341 (605)   752 -> 742 (1,075) 1,411 -> 1,044 (1,159)
+ * Over 64 .. 65,536 tokens and 1 .. 289 tiles its pick is within 1 % of the best of these counts on average. */
 void weight_grad_slices(long long M, int N1, int N2, int &slices, int &rows) {
     const long long tiles = (long long)((N1 + WG_T - 1) / WG_T) * ((N2 + WG_T - 1) / WG_T);
-    long long want = tiles < WG_CUS ? WG_CUS / tiles : 1;
-    const long long most = (M + WG_MIN_ROWS - 1) / WG_MIN_ROWS;
-    want = want < most ? want : most;
-    long long r = (M + want - 1) / want;
-    r = (r + WG_KC - 1) / WG_KC * WG_KC;
     const long long fit = (1LL << 30) / ((N1 > N2 ? N1 : N2) * 2) / WG_KC * WG_KC;
-    r = r < fit ? r : fit;
-    rows = (int)r;
-    slices = (int)((M + r - 1) / r);
+    const long long least = (M + fit - 1) / fit, most = (M + WG_MIN_ROWS - 1) / WG_MIN_ROWS;
+    const int cus = device_cus();
+    double best = -1.0;
+    slices = rows = 0;
+    auto consider = [&](long long s) {
+        s = s < most ? s : most;
+        s = s > least ? s : least;
+        const long long r = ((M + s - 1) / s + WG_KC - 1) / WG_KC * WG_KC;
+        if (r > fit) return;
+        s = (M + r - 1) / r;   /* no empty slice */
+        const double t = weight_grad_time(tiles, (long long)N1 * N2, cus, s, r);
+        if (best >= 0.0 && t >= best) return;
+        best = t;
+        slices = (int)s;
+        rows = (int)r;
+    };
+    for (long long s = 1; s <= most && (s == 1 || tiles * s <= 8LL * cus); s += s < 8 ? 1 : s / 8) consider(s);
+    for (int k = 1; k <= 8; k++)
+        if (k * cus / tiles > 0) consider(k * cus / tiles);
 }
 
 bool weight_grad_fits(long long M, int N1, int N2) {
@@ -202,7 +258,7 @@ extern "C" long long nc_weight_grad_workspace_bytes(long long rows, int n1, int 
     if (rows == 0) return 0;
     int slices, per;
     weight_grad_slices(rows, n1, n2, slices, per);
-    return (long long)slices * n1 * n2 * 4;
+    return slices == 1 ? 16 : (long long)slices * n1 * n2 * 4;   /* one slice needs none; never 0 where there is a call */
 }
 
 extern "C" int nc_weight_grad(const void *a, const void *b, long long rows, int n1, int n2, float *out, void *workspace,
@@ -219,8 +275,13 @@ extern "C" int nc_weight_grad(const void *a, const void *b, long long rows, int 
     weight_grad_slices(rows, n1, n2, p.slices, p.rows);
     p.part = (float *)workspace;
     const long long tiles = (long long)((n1 + WG_T - 1) / WG_T) * p.tiles2;
-    hipLaunchKernelGGL(weight_grad_kernel, dim3((unsigned)(tiles * p.slices)), dim3(WG_WAVES * WAVE), 0,
-                       (hipStream_t)stream, p);
+    const dim3 grid((unsigned)(tiles * p.slices)), block(WG_WAVES * WAVE);
+    if (p.slices == 1) {
+        p.part = out;
+        hipLaunchKernelGGL(weight_grad_kernel<true>, grid, block, 0, (hipStream_t)stream, p);
+        return (int)hipGetLastError();
+    }
+    hipLaunchKernelGGL(weight_grad_kernel<false>, grid, block, 0, (hipStream_t)stream, p);
     const long long n4 = (long long)n1 * n2 / 4;
     hipLaunchKernelGGL(weight_grad_sum_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
                        (const float4 *)workspace, p.slices, n4, (float4 *)out);

@@ -113,3 +113,21 @@ def test_weight_gradient_sizes_that_do_not_agree(device):
             op.add_weight_grad(*args)
     torch.cuda.synchronize()
     assert bool((grad == 1).all())
+
+
+@pytest.mark.parametrize("tokens,C,K", [(1, 8, 8), (300, 264, 520), (64, 2056, 768), (33, 1288, 2568), (9000, 2952, 2944),
+                                        (1500, 1672, 1664)])
+def test_weight_grad_of_one_slice_and_of_wide_results(device, tokens, C, K):
+    """One slice added straight into the result, at edges of its tiles, and results of more tiles than half the CUs, which
+    take several slices (the guard behind the gradient stays as it is)."""
+    gen = torch.Generator().manual_seed(tokens + C)
+    dh, x, start = bf(gen, tokens, C), bf(gen, tokens, K), torch.randn(C, K, generator=gen)
+    buf = torch.full((C * K + 4096,), 7.0, device=device)
+    grad = buf[:C * K].view(C, K)
+    grad.copy_(start)
+    op.add_weight_grad(grad, dh.to(device), x.to(device))
+    torch.cuda.synchronize()
+    a, b = dh.double(), x.double()
+    want, mag = a.t() @ b + start, a.abs().t() @ b.abs() + start.abs()
+    assert bool(((grad.double().cpu() - want).abs() <= (tokens + 300) * EPS * mag).all())
+    assert bool((buf[C * K:] == 7).all())

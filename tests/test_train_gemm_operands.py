@@ -101,3 +101,18 @@ def test_gate_weight_gradient_operands_on_two_devices(elsewhere, met):
     d = ["meta" if i == elsewhere else "cpu" for i in range(3)]
     with pytest.raises(met):
         ve_gate._weight_grad(bf(24, 2, device=d[0]), bf(24, 256, device=d[1]), torch.zeros(2, 256, device=d[2]))
+
+
+@pytest.mark.parametrize("tokens,n", [(65536, n) for n in (2304, 2560, 2944, 3072, 3584, 4224, 5120)] + [(9995, 3072)])
+def test_wide_weight_gradients_fill_the_chip(lib, tokens, n):
+    """Token slices by the workspace they need: of the CUs' turns (256 a round) at least three quarters have work, where one
+    slice of 100 to 250 tiles would leave half of them without."""
+    slices = max(1, lib.nc_weight_grad_workspace_bytes(tokens, n, n) // (4 * n * n))
+    groups = slices * (-(-n // 256)) ** 2
+    assert groups / (-(-groups // 256) * 256) >= 0.75, slices
+
+
+@pytest.mark.parametrize("tokens,n", [(1, 8), (64, 768), (512, 1664), (512, 2560), (2048, 3072)])
+def test_few_tokens_take_one_slice(lib, tokens, n):
+    """Its tiles are added into the result: no partials, which cost more than the idle CUs."""
+    assert 0 < lib.nc_weight_grad_workspace_bytes(tokens, n, n) <= 16

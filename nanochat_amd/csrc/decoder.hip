@@ -696,7 +696,8 @@ struct Layer {
 struct Acts {
     float *x0;                 /* [rows][C] fp32 */
     uint16_t *x, *xm, *h, *hn, *qkv, *q, *att, *xo, *u;  /* bf16 [rows][C] (qkv [3C], u [F]) */
-    float *acc;                /* [rows][max(C, F)]: fp32 GEMM outputs */
+    float *acc;                /* of the o GEMM, for the MLP's rstd: a step's fp32 sums [rows][C], a prefill's sums of
+                                * squares [rows][pf_ssq_cols(C)] */
     float *rstd;               /* [rows] */
 };
 
@@ -765,14 +766,15 @@ static void *device_alloc(Decoder *d, size_t bytes) {
     return p;
 }
 
-static size_t acts_bytes(const Decoder *d, size_t rows) {
-    const size_t C = d->C, F = d->F, W = F > C ? F : C;
-    return rows * (C * 4 + 7 * C * 2 + 3 * C * 2 + F * 2 + W * 4 + 4) + 16 * 256;
+/* acc_cols: acc's columns, C for a step's slots, pf_ssq_cols(C) for prefill rows. */
+static size_t acts_bytes(const Decoder *d, size_t rows, size_t acc_cols) {
+    const size_t C = d->C, F = d->F;
+    return rows * (C * 4 + 7 * C * 2 + 3 * C * 2 + F * 2 + acc_cols * 4 + 4) + 16 * 256;
 }
 
-static Acts carve_acts(Decoder *d, size_t rows) {
-    const size_t C = d->C, F = d->F, W = F > C ? F : C;
-    unsigned char *p = (unsigned char *)device_alloc(d, acts_bytes(d, rows));
+static Acts carve_acts(Decoder *d, size_t rows, size_t acc_cols) {
+    const size_t C = d->C, F = d->F;
+    unsigned char *p = (unsigned char *)device_alloc(d, acts_bytes(d, rows, acc_cols));
     auto take = [&](size_t bytes) {
         void *q = p;
         p += (bytes + 255) / 256 * 256;
@@ -789,21 +791,21 @@ static Acts carve_acts(Decoder *d, size_t rows) {
     a.xo = (uint16_t *)take(rows * C * 2);
     a.qkv = (uint16_t *)take(rows * 3 * C * 2);
     a.u = (uint16_t *)take(rows * F * 2);
-    a.acc = (float *)take(rows * W * 4);
+    a.acc = (float *)take(rows * acc_cols * 4);
     a.rstd = (float *)take(rows * 4);
     return a;
 }
 
-/* The activations of rows b0 .. of a. */
+/* The activations of a step's slots b0 .. of a. */
 static Acts acts_from(const Decoder *d, const Acts &a, size_t b0) {
-    const size_t C = d->C, F = d->F, W = F > C ? F : C;
+    const size_t C = d->C, F = d->F;
     Acts r = a;
     r.x0 = a.x0 + b0 * C;
     r.x = a.x + b0 * C; r.xm = a.xm + b0 * C; r.h = a.h + b0 * C; r.hn = a.hn + b0 * C;
     r.q = a.q + b0 * C; r.att = a.att + b0 * C; r.xo = a.xo + b0 * C;
     r.qkv = a.qkv + b0 * 3 * C;
     r.u = a.u + b0 * F;
-    r.acc = a.acc + b0 * W;
+    r.acc = a.acc + b0 * C;
     r.rstd = a.rstd + b0;
     return r;
 }
@@ -935,7 +937,7 @@ static void mlp(Decoder *d, const Lane &ln, bool step, const Layer &ly, const La
     } else {
         o_gemm(ln, ly.o, C, a.att, n, a.xo, a.xm, a.acc, a.rstd);
     }
-    gemm_epi(d, ln, step, SG_RELU2, ly.fc, F, C, a.xo, n, a.u, a.acc, nullptr, a.rstd, active);
+    gemm_epi(d, ln, step, SG_RELU2, ly.fc, F, C, a.xo, n, a.u, nullptr, nullptr, a.rstd, active);
     if (step) proj_norm(d, ln, ly, next, a, n, active);
     else gemm_epi(d, ln, step, SG_RESID, ly.proj, C, F, a.u, n, a.x, nullptr, a.xo, nullptr, active);
 }
@@ -1136,10 +1138,10 @@ static Decoder *create(const int *cfg, const uint64_t *ptrs, const float *scal, 
     const size_t store_pages = ((size_t)d->store + PAGE - 1) / PAGE;
     const size_t page_set = (size_t)d->H * (2 * PAGE_BYTES + 2 * PAGE * sizeof(float));  /* a page of every head */
     REQUIRE(pool_pages <= 0 || pool_pages >= d->max_pages, "a pool must hold at least one max_len sequence");
-    const size_t per_slot = (pool_pages > 0 ? 0 : (size_t)d->L * d->max_pages * page_set) + acts_bytes(d, 1) +
+    const size_t per_slot = (pool_pages > 0 ? 0 : (size_t)d->L * d->max_pages * page_set) + acts_bytes(d, 1, d->C) +
                             (size_t)d->vocab * 8 + (size_t)d->vocab / 8 + (size_t)d->max_pages * 4 + 64 +
                             (size_t)d->H * (HEAD_DIM + 2) * 4 + (size_t)d->H * 8;
-    d->row = carve_acts(d, PREFILL_ROWS);
+    d->row = carve_acts(d, PREFILL_ROWS, pf_ssq_cols(d->C));
     d->rows = (int32_t *)device_alloc(d, 7 * PREFILL_ROWS * sizeof(int32_t));
     d->active = (unsigned long long *)device_alloc(d, 2 * MASK_WORDS * sizeof(unsigned long long));
     size_t free_bytes = 0, total_bytes = 0;
@@ -1183,7 +1185,7 @@ static Decoder *create(const int *cfg, const uint64_t *ptrs, const float *scal, 
     d->allow = (uint32_t *)device_alloc(d, B * (d->vocab / WORD_BITS) * sizeof(uint32_t));
     d->logits = (float *)device_alloc(d, B * d->vocab * sizeof(float));
     d->probs = (float *)device_alloc(d, B * d->vocab * sizeof(float));
-    d->slot = carve_acts(d, B);
+    d->slot = carve_acts(d, B, d->C);
     /* measured at config 5 (128 slots, 26 layers): one lane eager 6.12 ms a step, one lane with graphs 6.2-6.3 ms,
      * two lanes with graphs 6.6 ms: attention fills every CU, so the other lane's GEMMs cannot run beside it, and
      * the host stays ahead of a 6 ms step. Both stay available (dec_debug_set_split / dec_debug_set_graphs). */

@@ -579,3 +579,18 @@ def test_more_than_128_slots(device):
             tok = int(tokens[140])
     finally:
         dec.close()
+
+
+def test_prefill_rows_hold_no_unused_buffer(device):
+    """A decoder's fixed memory is little more than its 16,384 prefill rows' activations: the fp32 embedding, ten bf16
+    streams of the hidden width, one of the MLP's and, of fp32 sums, only the o product's sums of squares."""
+    C, F, rows = 1664, 6656, 16384
+    m = model_tensors(1, C, F, 1024, 64, seed=0, std=0.05, theta=10000.0, ve_layers=(), windows=[64], device=device)
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    dec = DecoderRuntime(m, bos_token_id=0, max_length=64, prompt_store=0, max_slots=2)
+    try:
+        used = before - torch.cuda.mem_get_info()[0]
+    finally:
+        dec.close()
+    assert used <= rows * (4 * C + 20 * C + 2 * F + 4 * (C // 32) + 4) + (64 << 20), used

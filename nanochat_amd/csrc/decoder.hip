@@ -897,6 +897,7 @@ static void gemm_epi(Decoder *d, const Lane &ln, bool step, int epi, const uint1
     case SG_RESID: gemm(ln, w, rows, cols, in, n, out, SG_RESID, res); break;
     case SG_F32: gemm(ln, w, rows, cols, in, n, out_f32, SG_F32); break;
     case SG_RELU2: gemm(ln, w, rows, cols, in, n, out, SG_RELU2, nullptr, rstd); break;
+    default: die("gemm_epi", "an epilogue that prefill rows do not take here", __LINE__);
     }
 }
 

@@ -523,10 +523,12 @@ __global__ void __launch_bounds__(1024) ve_weight_sum_kernel(const float *part, 
     dw[i] = sum;
 }
 
-/* Slabs of `rows` rows for H heads: about four blocks a CU, none of fewer than VW_ROWS rows. */
+/* Slabs of `rows` rows for H heads, none of fewer than VW_ROWS rows: as many as run at once, four workgroups a CU, or three
+ * from 11 heads, whose 132 registers and more leave room for no fourth (with four, 16,384 rows of 13 heads ran a second round
+ * of 128 of their 896 workgroups: 36 us, now 31; 65,536 98 -> 75). */
 void ve_weight_slabs(long long rows, int heads, int &slabs, long long &per) {
     const int chunks = (heads * HEAD_DIM + VW_COLS - 1) / VW_COLS;
-    const long long tiles = (rows + VW_ROWS - 1) / VW_ROWS, most = 1024 / chunks;
+    const long long tiles = (rows + VW_ROWS - 1) / VW_ROWS, most = (heads <= 10 ? 1024 : 768) / chunks;
     const long long want = tiles < most ? tiles : most;
     per = (tiles + want - 1) / want * VW_ROWS;
     slabs = (int)((rows + per - 1) / per);

@@ -26,3 +26,15 @@ def test_no_head_count_spills(assembly, kernel):
                          r"\s+\.amdhsa_private_segment_fixed_size (\d+)", assembly)
     assert {int(heads) for heads, _, _ in scratch} == set(range(1, 17))
     assert not [s for s in scratch if int(s[2])]
+
+
+@pytest.mark.parametrize("heads", range(1, 17))
+def test_weight_gradient_runs_in_one_round(assembly, lib, heads):
+    """Its slabs of rows, by the workspace they need, times the column chunks are no more workgroups (four waves, one a
+    SIMD) than the registers let run at once on 256 CUs: a second round would be nearly empty."""
+    used = int(re.search(r"\.amdhsa_kernel _ZN2nc12_GLOBAL__N_116ve_weight_kernelILi%dE\w*\n(?:.*\n)*?"
+                         r"\s+\.amdhsa_next_free_vgpr (\d+)" % heads, assembly).group(1))
+    resident = 256 * min(8, 512 // (-(-used // 8) * 8))
+    for rows in (4096, 16384, 65536):
+        slabs = lib.nc_ve_weight_grad_workspace_bytes(rows, heads) // (heads * heads * 128 * 4)
+        assert slabs * (-(-heads // 2)) <= resident

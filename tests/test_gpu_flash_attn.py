@@ -172,10 +172,11 @@ def test_backward_rows_and_strided_dv(device):
         rel_check(got.float().cpu().numpy(), ref)
 
 
-@pytest.mark.parametrize("lengths,H", [([256] * 16, 8), ([300] * 30, 3), ([130, 300, 257] * 20, 3)])
+@pytest.mark.parametrize("lengths,H", [([256] * 16, 8), ([300] * 30, 3), ([130, 300, 257] * 20, 3), ([300] * 41, 3)])
 def test_every_tile_is_taken_once(device, lengths, H):
-    """256 workgroups (one per CU), 270 (some in the reversed second round) and 540 (a third round): every segment and
-    head gives the bits it gives in a call of its own."""
+    """256 workgroups (one per CU) and 270 (a second round of one row of eight and a rest, which no reversal moves), 540 (a
+    whole second round in reverse, and a third) and 369 (14 rows of a part-filled second round in reverse, and a rest):
+    every segment and head gives the bits it gives in a call of its own."""
     q, k, v, cu, _ = make(lengths, H, seed=len(lengths))
     dout = torch.randn(q.shape, generator=torch.Generator().manual_seed(6)).bfloat16()
 

@@ -391,7 +391,7 @@ __device__ __forceinline__ void ve_row(const VeBwd &a, const float *ws, VeRow<H>
  * contiguous bytes per lane, 256 or 512 contiguous bytes per instruction. A position is a chain of loads (its row's
  * number, then the row, then at a run's end the row of dtable: 2.4 us a position), so 64 positions' numbers and tokens
  * are read at once, one a lane. The rest of the chain is hidden by the resident waves or, AHEAD, by loading a position's
- * rows before the arithmetic of the one before it, into a second register set (the loop alternates two by name): 133
+ * rows before the arithmetic of the one before it, into a second register set (the loop alternates two by name): 135
  * registers at H = 6 against 72, so fewer waves (choose_backward says where which is the faster). H = 6, tokens of a
  * log-uniform vocabulary, us against one position at a time with every border run atomic: 256 rows 5.5 -> 5.1, 4,096
  * 32 -> 15.5, 16,384 81 -> 34, 65,536 103 -> 88 (its bytes take 84); H = 13 4,096 rows 47 -> 35, 65,536 234 -> 225; H = 16
@@ -407,18 +407,23 @@ __global__ void __launch_bounds__(VE_THREADS) ve_backward_kernel(VeBwd a) {
     const bool has_before = p0 > 0 && p0 < p1, has_after = p1 < a.rows && p0 < p1;
     const int before = has_before ? __builtin_amdgcn_readfirstlane(a.ids[p0 - 1]) : 0;
     const int after = has_after ? __builtin_amdgcn_readfirstlane(a.ids[p1]) : 0;
-    stage_w_rows<H>(ws, a.w);
-    __syncthreads();
-    VeRun<H> run;
-    run.started = run.ok = run.shared = false;
-    run.t = -1;
-    for (long long base = p0; base < p1; base += WAVE) {
+    const auto positions = [&](long long base) {
         VePositions ps;
         ps.n = (int)(p1 - base < WAVE ? p1 - base : WAVE);
         const unsigned long long row = lane < ps.n ? (unsigned long long)a.order[base + lane] : ~0ull;
         ps.row_lo = (uint32_t)row;
         ps.row_hi = (uint32_t)(row >> 32);
         ps.id = lane < ps.n ? a.ids[base + lane] : -1;
+        return ps;
+    };
+    VePositions ps = positions(p0);   /* in flight while w is staged */
+    stage_w_rows<H>(ws, a.w);
+    __syncthreads();
+    VeRun<H> run;
+    run.started = run.ok = run.shared = false;
+    run.t = -1;
+    for (long long base = p0; base < p1; base += WAVE) {
+        if (base > p0) ps = positions(base);
         VeRow<H> x, y;
         if (!AHEAD) {
             for (int q = 0; q < ps.n; q++) {
@@ -592,17 +597,17 @@ constexpr int VE_AHEAD_HEADS = 10;
  * same addresses; fewer leave the chip idle (H = 6, one / two / four rows a wave: 1,024 rows 8.8 / 7.7 / 10.9 us, 4,096
  * 26 / 17 / 15).
  * The second register set wins where a wave has several rows but the waves do not fill the chip, and at few heads always
- * (AHEAD / not, us of log-uniform tokens: H = 2, 16,384 rows 24 / 24, 65,536 45 / 55; H = 5 38 / 37, 76 / 87; H = 6 8,192
- * 22 / 24, 32,768 54 / 61, 65,536 97 / 88; H = 8 16,384 42 / 46, 65,536 123 / 102; H = 10 8,192 35 / 37, 16,384 51 / 56,
- * 32,768 85 / 82, 65,536 163 / 131). From 11 heads it takes 253 registers, from 13 it spilled: 65,536 rows of 16 heads took
- * 931 us. At one and two heads it fits a fourth workgroup a CU, whose adds cost more than it brings (65,536 rows, H = 1: 46
- * us with four, 36 with three). */
+ * (AHEAD / not, us of log-uniform tokens, caches cold: H = 6 1,024 rows 14.9 / 13.8, 2,048 17.2 / 18.4, 4,096 22.2 / 24.6,
+ * 32,768 68 / 78, 65,536 119 / 108; H = 2 4,096 14.0 / 15.3, 65,536 53 / 61; H = 5, warm, 65,536 76 / 87; H = 8 4,096
+ * 27.3 / 29.4, 32,768 84 / 83, 65,536 145 / 131; H = 10 4,096 33.8 / 34.3, 16,384 66 / 72, 32,768 107 / 102, 65,536 182 /
+ * 156). From 11 heads it takes 253 registers, from 13 it spilled: 65,536 rows of 16 heads took 931 us. At one and two heads
+ * it fits a fourth workgroup a CU, whose adds cost more than it brings (65,536 rows, H = 1: 46 us with four, 36 with three). */
 template <int H>
 int choose_backward(const VeBwd &a, hipStream_t stream) {
     const int per = (int)max(1LL, min(4LL, a.rows / 1024));
     if constexpr (H <= VE_AHEAD_HEADS) {
         const long long end = H <= 5 ? LLONG_MAX : H <= 8 ? 49152 : 24576;
-        if (a.rows >= 8192 && a.rows < end) return launch_backward<H, true>(a, per, stream);
+        if (a.rows >= (H <= 2 ? 0 : 2048) && a.rows < end) return launch_backward<H, true>(a, per, stream);
     }
     return launch_backward<H, false>(a, per, stream);
 }

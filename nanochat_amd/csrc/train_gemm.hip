@@ -210,8 +210,8 @@ double weight_grad_time(long long tiles, long long elements, int cus, long long 
     return rounds * (rows / WG_KC + 10) * stage + partials;
 }
 
-/* Token slices: the best of a few counts by weight_grad_time (small ones, steps of about an eighth above, and those that just
- * fill one to eight rounds), none under WG_MIN_ROWS rows unless it is the only one and none whose operand slice passes 1
+/* Token slices: the best of a few counts by weight_grad_time (small ones, steps of about a quarter above, and those that just
+ * fill one to four rounds), none under WG_MIN_ROWS rows unless it is the only one and none whose operand slice passes 1
  * GiB. As many as fill the CUs, and one where the tiles are half of them or more, left CUs idle at wide results and spent
  * more on partials than they saved at few tokens. us, so and by the model (library product and addition):
  *   tokens    768 x 768        1,664 x 1,664      2,560 x 2,560       3,072 x 3,072
@@ -239,10 +239,13 @@ void weight_grad_slices(long long M, int N1, int N2, int &slices, int &rows) {
         slices = (int)s;
         rows = (int)r;
     };
-    for (long long s = 1; s <= most && (s == 1 || tiles * s <= 8LL * cus); s += s < 8 ? 1 : s / 8) consider(s);
-    for (int k = 1; k <= 8; k++)
-        if (k * cus / tiles > 0) consider(k * cus / tiles);
+    for (long long s = 1; s <= most && (s == 1 || tiles * s <= 4LL * cus); s += s < 8 ? 1 : s / 4) consider(s);
+    for (int k = 1; k <= 4; k++)
+        if (k * cus >= tiles) consider(k * cus / tiles);
 }
+
+/* One slice needs none (never 0 where there is a call). */
+long long weight_grad_bytes(int slices, int N1, int N2) { return slices == 1 ? 16 : (long long)slices * N1 * N2 * 4; }
 
 bool weight_grad_fits(long long M, int N1, int N2) {
     return M >= 0 && M < (1LL << 40) && N1 > 0 && N2 > 0 && N1 % 8 == 0 && N2 % 8 == 0 && N1 <= 65536 && N2 <= 65536;
@@ -258,7 +261,7 @@ extern "C" long long nc_weight_grad_workspace_bytes(long long rows, int n1, int 
     if (rows == 0) return 0;
     int slices, per;
     weight_grad_slices(rows, n1, n2, slices, per);
-    return slices == 1 ? 16 : (long long)slices * n1 * n2 * 4;   /* one slice needs none; never 0 where there is a call */
+    return weight_grad_bytes(slices, n1, n2);
 }
 
 extern "C" int nc_weight_grad(const void *a, const void *b, long long rows, int n1, int n2, float *out, void *workspace,
@@ -267,12 +270,12 @@ extern "C" int nc_weight_grad(const void *a, const void *b, long long rows, int 
     if (rows == 0) return NC_OK;
     if (!a || !b || !out || !workspace) return NC_ERR_NULL;
     if (((uintptr_t)a | (uintptr_t)b | (uintptr_t)out | (uintptr_t)workspace) & 15) return NC_ERR_SHAPE;
-    if (workspace_bytes < nc_weight_grad_workspace_bytes(rows, n1, n2)) return NC_ERR_WORKSPACE;
     WeightGrad p;
     p.a = (const uint16_t *)a; p.b = (const uint16_t *)b;
     p.N1 = n1; p.N2 = n2; p.tiles2 = (n2 + WG_T - 1) / WG_T;
     p.M = rows;
     weight_grad_slices(rows, n1, n2, p.slices, p.rows);
+    if (workspace_bytes < weight_grad_bytes(p.slices, n1, n2)) return NC_ERR_WORKSPACE;
     p.part = (float *)workspace;
     const long long tiles = (long long)((n1 + WG_T - 1) / WG_T) * p.tiles2;
     const dim3 grid((unsigned)(tiles * p.slices)), block(WG_WAVES * WAVE);

@@ -1086,8 +1086,9 @@ static void enqueue_head(Decoder *d) {
         ChoiceArgs c = {d->logits, d->probs, d->active, d->allow, d->temperature, d->top_p, d->seed, d->first,
                         d->tokens, d->alt_tokens, d->pos, d->softcap, d->vocab, d->lazy, d->cut, d->keys, d->arrived};
         hipLaunchKernelGGL(choose_kernel, dim3(R), dim3(CHOICE_THREADS), 0, d->stream, c);
-        bool sampled = false;
-        for (int b = 0; b < R; b++) sampled |= d->sampled[b];
+        bool sampled = false;   /* a live slot is */
+        for (int b = 0; b < R; b++)
+            sampled |= d->sampled[b] && ((d->live[b / MASK_BITS] >> (b % MASK_BITS)) & 1ull);
         if (sampled) hipLaunchKernelGGL(sample_kernel, dim3(SAMPLE_SPLIT, R), dim3(CHOICE_THREADS), 0, d->stream, c);
     }
     HIP_CHECK(hipMemcpyAsync(d->host_tokens, d->tokens, (size_t)d->B * 4, hipMemcpyDeviceToHost, d->stream));

@@ -594,3 +594,30 @@ def test_prefill_rows_hold_no_unused_buffer(device):
     finally:
         dec.close()
     assert used <= rows * (4 * C + 20 * C + 2 * F + 4 * (C // 32) + 4) + (64 << 20), used
+
+
+def test_sampled_slot_that_rests_and_returns(device):
+    """A step launches the sampled slots' kernel only where one of them is live: a sampled slot that sits out a step between
+    greedy ones draws its own next token when it comes back, and a greedy slot is the same throughout."""
+    m = model_tensors(1, 256, 1024, 1024, 64, seed=3, std=0.05, theta=10000.0, ve_layers=(), windows=[64], device=device)
+    dec = DecoderRuntime(m, bos_token_id=0, max_length=64, prompt_store=0, max_slots=3)
+    try:
+        params = [(0.0, 1), (0.9, 7), (0.0, 1)]
+        for b, ids in enumerate(prompts([10, 14, 12], m.vocab, seed=5)):
+            dec.place(b, ids, temperature=params[b][0], seed=params[b][1])
+        dec.prefill()
+        gen = [0, 0, 0]
+        for live in ([0, 1, 2], [0, 2], [0, 1, 2], [2], [1]):
+            dec.activate(live)
+            tokens, got = dec.step(), dec.logits(3)
+            for b in live:
+                T, seed = params[b]
+                tok, _ = sampling.choose(got[b], temperature=T, top_p=1.0, seed=seed, gen=gen[b], lazy=0, softcap=m.softcap)
+                scores = got[b]
+                if T > 0:
+                    z = sampling.capped(got[b], m.softcap)
+                    scores = (z / np.float32(T)).astype(np.float32) + sampling.gumbel(seed, gen[b], np.arange(m.vocab))
+                assert near_tie_ok(int(tokens[b]), tok, scores), (live, b)
+                gen[b] += 1
+    finally:
+        dec.close()

@@ -417,9 +417,11 @@ int prefill_gemm(const PfGemm &g, int epi, hipStream_t stream) {
      * (a stage takes a quarter 0.31 us, a half 0.53, a whole tile 0.73). The round may be the only one: a prompt of a few
      * thousand tokens makes fewer tiles than CUs, and its GEMM then lasts as long as one tile (M = 1,500, N x K = 768 x
      * 3,072: 18 whole tiles 71 us, 72 quarters 31 us; M = 6,594, 78 tiles 73 us, 156 halves 51 us). Calls of M <= 128
-     * rows (a decode step's slots) take quarters as long as their (N / 128) column tiles fit the CUs, else 128 x 256. */
+     * rows (a decode step's slots) take quarters as long as all four of each tile, two of them past M, have a CU, else 128 x
+     * 256 (M = 64, K = 1,664: N = 16,384 quarters 15.9 us, thin tiles 23.3; N = 20,480, where the workgroups past the CUs'
+     * number made a second round, 29.0 and 23.9; N = 32,768 29.3 and 26.7). */
     const int cus = device_cus(), nx = (g.N + 255) / 256, T = nx * ((g.M + 255) / 256), R = T % cus;
-    const bool one = g.M <= 128, thin = one && 2 * nx > cus;
+    const bool one = g.M <= 128, thin = one && 4 * nx > cus;
     const int pieces = thin || R == 0 ? 1 : one || 4 * R <= cus ? 4 : 2 * R <= cus ? 2 : 1;
     const int full = pieces > 1 ? T - R : T;
     const dim3 grid(full + (T - full) * pieces), block(PG_WAVES * WAVE);

@@ -108,3 +108,20 @@ def test_part_filled_single_round_matches_whole_rows(device, N, K, M):
     assert bool(((got[rows].double().cpu() - want).abs() <= K * 2.0 ** -23 * mag).all())
     for r in rows:
         assert torch.equal(run(F32, w, a[r:r + 1].contiguous())[0], got[r])
+
+
+@pytest.mark.parametrize("M", [1, 128])
+@pytest.mark.parametrize("N", [16384, 16388, 20480, 32768])
+def test_few_rows_of_many_columns(device, N, M):
+    """Both sides of the line between quarter tiles and 128 x 256 ones for calls of at most 128 rows: fp32 sums within fp32
+    accumulation error of float64, and the same bits in a call over half of the columns (the other kind of tile)."""
+    K = 256
+    gen = torch.Generator().manual_seed(N + M)
+    w = torch.randn(N, K, generator=gen).bfloat16().to(device)
+    a = torch.randn(M, K, generator=gen).bfloat16().to(device)
+    got = run(F32, w, a)
+    want = a.double().cpu() @ w.double().cpu().t()
+    mag = a.double().abs().cpu() @ w.double().abs().cpu().t()
+    assert bool(((got.double().cpu() - want).abs() <= K * 2.0 ** -23 * mag).all())
+    half = N // 8 * 4
+    assert torch.equal(run(F32, w[:half].contiguous(), a), got[:, :half])

@@ -15,9 +15,9 @@
  * K-slices whose partials a second kernel adds in order; a model wider than 2,048 computes the MLP's rstd in
  * rstd_kernel). Prefill's GEMMs (up to 16,384 rows a call) are prefill_gemm.hip's MFMA-tiled kernel over all the
  * call's rows at once, with the epilogue fused (bf16 out, the residual, ReLU^2 with the rstd); each row's sums run in
- * one fixed order, so they do not depend on how many rows the call holds. The o GEMM's residual sum needs its whole
- * row for the MLP's rstd, so it also writes each 32 columns' sum of squares, which tile_rstd adds. Every kernel covers the slots up to
- * the highest active one (dec_set_active) and skips inactive slots.
+ * one fixed order, so they do not depend on how many rows the call holds. The MLP's rstd needs the o GEMM's whole row, so
+ * that GEMM also writes each 32 columns' sum of squares, which tile_rstd adds. Every kernel covers the slots up to the
+ * highest active one (dec_set_active) and skips inactive slots.
  *
  * Numerics, op by op as decode.cu: the epilogues round once (bf16(s + residual)); the MLP reads the un-normed stream
  * scaled by its rstd; every RMS norm is 1 / sqrt(mean x^2 + FLT_EPSILON), correctly rounded (the reference: rsqrtf).
@@ -549,10 +549,10 @@ __global__ void __launch_bounds__(CHOICE_THREADS) choose_kernel(ChoiceArgs c) {
 /* The sampled slots' tokens (T > 0), SAMPLE_SPLIT blocks a slot: the row with the largest z / T + gumbel among the allowed
  * rows (Gumbel-max sampling of softmax(z / T)), or among those a nucleus slot's threshold keeps (no alternative then).
  * A row costs a Philox block and two fp64 logarithms, about 2 us for a block of 1,024 rows, so one block a slot took
- * 135 us of a vocabulary of 65,536 (12 layers of d768, a step of 4 sampled slots 580 -> 460 us, with a nucleus 716 -> 596,
- * of 128 sampled slots 728 -> 687; the same greedy steps 460 and 605). A block adds its best keys to the slot's by agent-scope maxima and then counts itself; the last to
- * count takes the keys, clears them for the next call and commits. Keys are unique per row, so the order does not
- * matter. Launched only where a slot is sampled. */
+ * 135 us of a vocabulary of 65,536 (12 layers of d768, a step of 4 sampled slots 580 -> 460 us, with a nucleus 716 ->
+ * 596, of 128 sampled slots 728 -> 687; the same greedy steps 460 and 605). A block adds its best keys to the slot's by
+ * agent-scope maxima and then counts itself; the last to count takes the keys, clears them for the next call and commits.
+ * Keys are unique per row, so the order does not matter. Launched only where a live slot is sampled. */
 constexpr int SAMPLE_SPLIT = 16;
 
 __global__ void __launch_bounds__(CHOICE_THREADS) sample_kernel(ChoiceArgs c) {

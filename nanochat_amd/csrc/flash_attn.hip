@@ -643,9 +643,9 @@ __global__ void __launch_bounds__(FA_THREADS, 2) flash_bwd_dq_kernel(FlashBwd a)
             store4(p + d * 32 + 8 * j, f32x4{dq[d][4 * j], dq[d][4 * j + 1], dq[d][4 * j + 2], dq[d][4 * j + 3]}, a.scale);
 }
 
-/* D[row][h] = sum_d dO . O in fp32, bound by HBM (512 bytes a row): 16 lanes a (row, head), eight consecutive dims a lane by
- * 16-byte loads (4-byte aligned; the one-wave-a-row form's 4 bytes a lane took 62 us at 65,536 tokens of 6 heads, this 31), the lanes' sums by the
- * fixed butterfly. */
+/* D[row][h] = sum_d dO . O in fp32, bound by HBM (512 bytes a row): 16 lanes a (row, head), eight consecutive dims a lane
+ * by 16-byte loads (4-byte aligned), the lanes' sums by the fixed butterfly. 65,536 tokens of 6 heads 31 us; a wave a row
+ * with 4 bytes a lane took 62. */
 typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
 __global__ void __launch_bounds__(256) flash_bwd_rows_kernel(const uint16_t *out, long long o_stride,
@@ -742,7 +742,8 @@ extern "C" int nc_flash_attn_bwd(const void *q, const void *k, const void *v, co
     a.q_stride = q_stride; a.k_stride = k_stride; a.v_stride = v_stride; a.do_stride = do_stride;
     a.lse = lse; a.lse_stride = lse_stride; a.dpsum = dpsum;
     a.cu = cu_seqlens; a.segments = segments; a.H = heads; a.window = window < 0 ? -1 : window;
-    /* dK/dV divides lse by the exponent's scale: kept where that quotient is finite; below, scale S vanishes beside lse */
+    /* the kernels divide lse by the exponent's scale: kept where that quotient is finite; below, scale S vanishes beside
+     * lse */
     a.scale = softmax_scale; a.scale_log2 = fmaxf(softmax_scale, 0x1p-116f) * FA_LOG2E;
     a.dq = (uint16_t *)dq; a.dk = (uint16_t *)dk; a.dv = (uint16_t *)dv;
     a.dq_stride = dq_stride; a.dk_stride = dk_stride; a.dv_stride = dv_stride;

@@ -3,8 +3,8 @@
  * per-(token, KV head) absmax e4m3fn quantizer and the paged store; plus the training-form q/k prologue
  * (the reference's qkp_forward) on the same row math.
  *
- * Four (token, head) rows a wave, 16 lanes a row. The row math (nc_row.h) gives the
- * same bits as the fused decode step's, which appends the step's token inside the attention kernel.
+ * Four (token, head) rows a wave, 16 lanes a row. The row math (nc_row.h) gives the same bits as the fused decode
+ * step's, which appends the step's token inside the attention kernel.
  */
 #include "nc_device.h"
 #include "nc_row.h"
@@ -53,8 +53,8 @@ static inline int append_pages_per_seq(int T) { return (T + PAGE - 2) / PAGE + 1
  * The 16 scales of K and of V go out the same way.
  * y >= Hkv (FUSED only): q heads 4 (y - Hkv) .. + 3 of the page's slots, normed and rotated into q_out; a wave reads its
  * slots' rotation once for the four.
- * It is bound by the chain each work-group begins with (position, page, rows) more than by HBM: 46 MB in 12.8 us at
- * 8 x 512 tokens of 16 / 4 heads (13.1 with eight 2-byte accesses a row and lane), 75 MB in 21.8 us at 3 x 1,501 tokens of
+ * It is bound by the chain each work-group begins with (position, page, rows) more than by HBM: 46 MB in 12.9 us (12.4 at best)
+ * at 8 x 512 tokens of 16 / 4 heads (13.2 with eight 2-byte accesses a row and lane), 75 MB in 21.8 us at 3 x 1,501 tokens of
  * 13 / 13 heads (22.4); with value embeddings, 6,594 rows of 6 heads, C = 768, 36 -> 24 us. Four KV heads a work-group, one
  * chain for all, left too few of them: 17 us, 25 us and 37 us. */
 constexpr int Q_GROUP = 4;   /* q heads a work-group */
@@ -168,9 +168,14 @@ __global__ void __launch_bounds__(256) append_kernel(AppendArgs a) {
  * token stride 3 H 128, output contiguous, position p % T for token p.
  *
  * Both directions are bound by HBM (forward: 2 x 256 bytes a row; backward: 3 x 256). 16 lanes take a row (nc_row.h's
- * form), a 16-lane group QK_HEADS heads of one token, so an access is 8 or 16 bytes a lane, the rotation is read once for QK_HEADS rows and all of a group's rows are in flight together. Against one row a
- * wave with 2-byte accesses, 65,536 tokens of 6 heads: forward 179 -> 87 us (4.6 TB/s), backward 242 -> 115 us (5.2
- * TB/s); a large copy reaches 4.8. */
+ * form), a 16-lane group QK_HEADS heads of one token, so an access is 8 or 16 bytes a lane, the rotation is read once for
+ * QK_HEADS rows and all of a group's rows are in flight together. Against one row a wave with 2-byte accesses, 65,536
+ * tokens of 6 heads: forward 179 -> 87 us (4.6 TB/s), backward 242 -> 115 us (5.2 TB/s); a copy, which reads as much as it
+ * writes, reaches 4.8.
+ * QK_HEADS divides the 6 heads of the small model and is the same for every count, a group's last places being empty where
+ * it does not divide. 65,536 tokens, caches cold, forward / backward in us with two, three and four heads a group: 1 head
+ * 25 / 42 each; 4 heads 79 / 119, 86 / 126, 77 / 121; 6 heads 101 / 154, 101 / 156, 112 / 162; 10 heads 150 / 228,
+ * 161 / 238, 149 / 237; 16 heads 229 / 347, 233 / 352, 220 / 352. */
 constexpr int QK_HEADS = 3;
 static int qk_head_chunks(int H) { return (H + QK_HEADS - 1) / QK_HEADS; }
 

@@ -1,6 +1,6 @@
 /*
- * The training block's output projection on gfx950: its forward with the residual and the row statistic (linear_residual_rms,
- * on prefill_gemm.hip's tiled kernel) and its weight gradient (weight_grad).
+ * The training block's output projection on gfx950: its forward with the residual and the row statistic
+ * (linear_residual_rms, on prefill_gemm.hip's tiled kernel) and its weight gradient (weight_grad).
  *
  * weight_grad: out[i][j] += sum_m a[m][i] b[m][j] for token rows m (a = the output's gradient [M][N1], b = the input
  * [M][N2], bf16, fp32 sums). The result is small (C x C) and the sum long (every token), so the tiles alone would leave

@@ -1,6 +1,7 @@
-"""Which operands of the training block's projection and weight gradients (the value-embedding gate's too) reach their HIP kernels, which trust the sizes
-and addresses they are given: without a GPU, CPU tensors stand for device tensors and a kernel call is an exception of its
-own. Operands whose sizes or devices do not agree must meet the library GEMM instead, which raises."""
+"""Which operands of the training block's projection and weight gradients (the value-embedding gate's too) reach their HIP
+kernels, which trust the sizes and addresses they are given: without a GPU, CPU tensors stand for device tensors and a
+kernel call is an exception of its own. Operands whose sizes or devices do not agree must meet the library GEMM instead,
+which raises."""
 import pytest
 import torch
 

@@ -41,7 +41,8 @@ def test_projection_matches_float64(device, tokens, C, K):
 
 
 def test_projection_rows_do_not_depend_on_the_others(device):
-    """A row's result and rstd have the same bits alone (thin tiles), among 700 rows and among 30,000 (split tiles)."""
+    """A row's result and rstd have the same bits alone and among 100 (quarter tiles), 700 (quarters of both row halves) and
+    30,000 (whole tiles and a round of pieces)."""
     gen = torch.Generator().manual_seed(3)
     x, w, res = (t.to(device) for t in (bf(gen, 30000, 256), bf(gen, 768, 256, scale=1 / 16), bf(gen, 30000, 768)))
     h, rstd = op.project(x, w, res)

@@ -236,11 +236,12 @@ def test_weight_grad_matches_float64(device, rows, H):
         assert bool(((g.double().cpu() - want).abs() <= (rows + 16) * 2.0 ** -23 * mag).all())
 
 
-def test_runs_that_end_at_wave_borders(device):
-    """Fewer rows than waves (a row a wave): every run is a wave's first and last, alone or shared with its neighbours;
-    runs of one, two and many rows, a skipped row (order outside the rows) inside a run. dtable within fp32 rounding of
-    float64."""
-    H, vocab = 2, 40
+@pytest.mark.parametrize("H", [2, 6, 13])
+def test_runs_that_end_at_wave_borders(device, H):
+    """Fewer rows than waves (a row a wave; two heads hold two positions' rows, six and thirteen one): every run is a wave's
+    first and last, alone or shared with its neighbours; runs of one, two and many rows, a skipped row (order outside the
+    rows) inside a run. dtable within fp32 rounding of float64."""
+    vocab = 40
     C = H * HEAD_DIM
     idx = torch.tensor([0] * 9 + [3] + [5, 5] + [7] + [9] * 4 + [11, 12, 13] + [39] * 2, dtype=torch.int32)
     rows = idx.numel()
